@@ -1183,6 +1183,68 @@ __global__ __launch_bounds__(kPersistMaxWaves * 64) void attn_decode_persistent_
   if (cur >= 0) finish(cur);
 }
 
+// Running merge of softmax partials (m, l in log2 units, O / l) for four
+// dims of one query head.  add() folds U partials at a time, so their loads
+// can all be in flight together.
+struct MergeState {
+  float m = kNegBig, l = 0.0f, o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+
+  template <int U>
+  __device__ __forceinline__ void add(const float2 (&ml)[U], const float4 (&v)[U]) {
+    float mx = m;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      mx = fmaxf(mx, ml[u].x);
+    const float fs = fast_exp2(m - mx);
+    l *= fs;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] *= fs;
+    m = mx;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float f = ml[u].y * fast_exp2(ml[u].x - mx);
+      l += f;
+      o[0] = fmaf(v[u].x, f, o[0]); o[1] = fmaf(v[u].y, f, o[1]);
+      o[2] = fmaf(v[u].z, f, o[2]); o[3] = fmaf(v[u].w, f, o[3]);
+    }
+  }
+};
+
+// Where a row's partials lie: entry i < np is the row's i-th walked piece,
+// entry np + k its k-th prefix split.
+struct MergeSource {
+  const float* ws_ml; const float* ws_acc; const float* pfx_ml; const float* pfx_acc;
+  int64_t pb;                         // the row and head's first prefix split
+  int sq, np, nsplit, g0, num_seqs, num_heads, hq;
+
+  // Entries i, i + step, ... (U of them); those past the last count nothing
+  // (m = kNegBig, l = 0; the loads re-read the last).
+  template <int D, int U>
+  __device__ __forceinline__ void load(int i, int step, int d, float2 (&ml)[U],
+                                       float4 (&v)[U]) const {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int e = min(i + u * step, np + nsplit - 1);
+      const float* m;
+      const float* a;
+      if (e < np) {
+        const int64_t base =
+            (int64_t)piece_slot(sq, min(e, 2), g0 + e, num_seqs) * num_heads + hq;
+        m = ws_ml + base * 2;
+        a = ws_acc + base * D + d;
+      } else {
+        m = pfx_ml + (pb + e - np) * 2;
+        a = pfx_acc + (pb + e - np) * D + d;
+      }
+      ml[u] = *reinterpret_cast<const float2*>(m);
+      v[u] = *reinterpret_cast<const float4*>(a);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i + u * step >= np + nsplit) ml[u] = make_float2(kNegBig, 0.0f);
+  }
+};
+
 // Merge the pieces of every sequence that spans several workgroup ranges
 // (same flattened split as the persistent kernel), together with its
 // shared-prefix partials if it has any; write zeros for a sequence with no
@@ -1269,7 +1331,8 @@ __global__ __launch_bounds__(512) void attn_persist_reduce_kernel(
     put(L, O);
     return;
   }
-  // three or more pieces, or more than four splits: pieces from their slots
+  // three or more pieces, or more than four splits: pieces from their slots,
+  // eight loads in flight at a time
   int g0 = 0;
   if (np == 3) {
     const int a = ws_off[sq], b = ws_off[sq + 1];
@@ -1277,35 +1340,73 @@ __global__ __launch_bounds__(512) void attn_persist_reduce_kernel(
     g0 = rs.owner(a);
     np = rs.owner(b - 1) - g0 + 1;
   }
-  auto piece = [&](int i, float2& ml, float4& v) __attribute__((always_inline)) {
-    const int64_t base = (int64_t)piece_slot(sq, min(i, 2), g0 + i, num_seqs) * num_heads + hq;
-    ml = *reinterpret_cast<const float2*>(ws_ml + base * 2);
-    v = *reinterpret_cast<const float4*>(ws_acc + base * D + d);
-  };
+  const MergeSource src{ws_ml, ws_acc, pfx.ml, pfx.acc, pb, sq, np, nsplit, g0, num_seqs,
+                        num_heads, hq};
+  MergeState st;
+  for (int i = 0; i < np + nsplit; i += 8) {
+    float2 ml[8]; float4 v[8];
+    src.load<D, 8>(i, 1, d, ml, v);
+    st.add(ml, v);
+  }
+  put(st.l, st.o);
+}
+
+// The same merge for batches of few rows, whose rows span many ranges each
+// (one row: every range): one workgroup per (row, query head), NG groups of
+// D / 4 lanes (thread = 4 dims) that take the row's pieces and prefix splits
+// i = group, group + NG, ... four loads at a time, then one pass over the
+// groups' states in LDS.  A row's pieces are latency, not bandwidth: the
+// narrow kernel read a 94-piece row (1500 tokens) in a chain of load round
+// trips, 51.8 us by trace; here they are in flight at once (the call 62.5 ->
+// 17.2 us).
+template <typename T, int D>
+__global__ __launch_bounds__(256) void attn_persist_reduce_wide_kernel(
+    const int32_t* __restrict__ ws_off, int num_seqs, int num_wgs, int num_heads,
+    const float* __restrict__ ws_acc, const float* __restrict__ ws_ml,
+    T* __restrict__ out, int64_t out_stride, PrefixArgs pfx) {
+  constexpr int LPH = D / 4;          // lanes per group
+  constexpr int NG = 256 / LPH;       // groups
+  __shared__ float s_ml[NG][2];
+  __shared__ float s_o[NG][D];
+  const int sq = blockIdx.x, hq = blockIdx.y;
+  const int grp = (int)threadIdx.x / LPH;
+  const int d = ((int)threadIdx.x % LPH) * 4;
+  const int hdr = ws_off[2 * num_seqs + 1 + sq];
+  const int a = ws_off[sq], b = ws_off[sq + 1], total = ws_off[num_seqs];
+  int np = header_pieces(hdr);
+  if (np == 1) return;                // finished (with its prefix) by the decode kernel
+  const int nsplit = pfx.blocks != nullptr ? header_splits(hdr) : 0;
+  int g0 = 0;
+  if (np > 0) {
+    const RangeSplit rs = make_range_split(total, num_wgs);
+    g0 = rs.owner(a);
+    np = rs.owner(b - 1) - g0 + 1;
+  }
+  const int64_t pb = ((int64_t)sq * num_heads + hq) * kPrefixMaxSplits;
+  const MergeSource src{ws_ml, ws_acc, pfx.ml, pfx.acc, pb, sq, np, nsplit, g0, num_seqs,
+                        num_heads, hq};
+  MergeState st;
+  for (int i = grp; i < np + nsplit; i += 4 * NG) {
+    float2 ml[4]; float4 v[4];
+    src.load<D, 4>(i, NG, d, ml, v);
+    st.add(ml, v);
+  }
+  if (d == 0) { s_ml[grp][0] = st.m; s_ml[grp][1] = st.l; }
+  *reinterpret_cast<float4*>(&s_o[grp][d]) = make_float4(st.o[0], st.o[1], st.o[2], st.o[3]);
+  __syncthreads();
+  if (threadIdx.x >= D) return;
+  const int dim = threadIdx.x;
   float M = kNegBig;
-  for (int i = 0; i < np; ++i) {
-    float2 ml; float4 v;
-    piece(i, ml, v);
-    M = fmaxf(M, ml.x);
+#pragma unroll
+  for (int g = 0; g < NG; ++g) M = fmaxf(M, s_ml[g][0]);
+  float L = 0.0f, O = 0.0f;
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {      // s_o holds sums of l-weighted values
+    const float f = fast_exp2(s_ml[g][0] - M);
+    L = fmaf(s_ml[g][1], f, L);
+    O = fmaf(s_o[g][dim], f, O);
   }
-  for (int sp = 0; sp < nsplit; ++sp) M = fmaxf(M, pfx.ml[(pb + sp) * 2]);
-  float L = 0.0f, O[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int i = 0; i < np; ++i) {
-    float2 ml; float4 v;
-    piece(i, ml, v);
-    const float f = ml.y * fast_exp2(ml.x - M);
-    L += f;
-    O[0] = fmaf(v.x, f, O[0]); O[1] = fmaf(v.y, f, O[1]);
-    O[2] = fmaf(v.z, f, O[2]); O[3] = fmaf(v.w, f, O[3]);
-  }
-  for (int sp = 0; sp < nsplit; ++sp) {
-    const float f = pfx.ml[(pb + sp) * 2 + 1] * fast_exp2(pfx.ml[(pb + sp) * 2] - M);
-    L += f;
-    const float4 v = *reinterpret_cast<const float4*>(pfx.acc + (pb + sp) * D + d);
-    O[0] = fmaf(v.x, f, O[0]); O[1] = fmaf(v.y, f, O[1]);
-    O[2] = fmaf(v.z, f, O[2]); O[3] = fmaf(v.w, f, O[3]);
-  }
-  put(L, O);
+  elem<T>::store(out + (int64_t)sq * out_stride + (int64_t)hq * D + dim, L > 0.0f ? O / L : 0.0f);
 }
 
 // Merge the partitions of one (row, query head); rows with a single
@@ -1467,8 +1568,19 @@ static void launch_persistent(const void* q, int64_t q_stride, const void* kc, c
                      dim3(64 * num_kv_heads), lds, st, (const T*)q, q_stride, (const T*)kc,
                      (const T*)vc, num_kv_heads, num_cache_blocks, bt, max_blocks, ctx, num_seqs,
                      scale_log2, (T*)out, out_stride, ws_off, ws_acc, ws_ml, pfx, p.sync_mask);
-  constexpr int kHeadsPerReduceWg = 512 / (D / 4);
   const int H = num_kv_heads * G;
+  // A workgroup per (row, query head) while a row spans three ranges or more
+  // on average; past that most rows have one or two pieces and the extra
+  // workgroups cost more than they hide.  Whole calls as graph replays,
+  // narrow / wide: 2 rows 27.1 / 15.4 us, 8 rows 30.1 / 23.6, 48 rows (32
+  // heads) 90.7 / 83.1, 128 rows 185.5 / 179.8, 256 rows 194.7 / 196.0.
+  if (2 * num_seqs <= p.num_wgs) {
+    hipLaunchKernelGGL((attn_persist_reduce_wide_kernel<T, D>), dim3(num_seqs, H), dim3(256), 0,
+                       st, (const int32_t*)ws_off, num_seqs, p.num_wgs, H, (const float*)ws_acc,
+                       (const float*)ws_ml, (T*)out, out_stride, pfx);
+    return;
+  }
+  constexpr int kHeadsPerReduceWg = 512 / (D / 4);
   hipLaunchKernelGGL((attn_persist_reduce_kernel<T, D>),
                      dim3(num_seqs, (H + kHeadsPerReduceWg - 1) / kHeadsPerReduceWg), dim3(512),
                      0, st, (const int32_t*)ws_off, num_seqs, p.num_wgs, H,

@@ -165,6 +165,30 @@ def test_decode_long_contexts(device):
     _check_attention(got, _oracle(batch), "long contexts")
 
 
+@pytest.mark.parametrize("rows,heads", [(1, (16, 8, 128)), (3, (16, 2, 128)), (7, (8, 8, 64)),
+                                        (128, (16, 8, 128)), (129, (16, 8, 128))])
+def test_decode_few_rows_of_many_pieces(device, rows, heads):
+    """Rows cut into up to one piece per workgroup: the reduce kernel that
+    takes a workgroup per (row, head) up to half as many rows as workgroups,
+    and the other one just past that; empty, one-block and two-block rows
+    among the long ones.  fp16 outputs round at 2^-11, so 3e-3 of the largest
+    value and 1e-3 relative L2 bound one rounding plus fp32 merges."""
+    H, Hkv, D = heads
+    _say(f"decode few rows rows={rows} {heads}")
+    batch = workloads.paged_decode(seed=rows, num_seqs=rows, num_heads=H, num_kv_heads=Hkv,
+                                   head_dim=D, ctx_lo=1, ctx_hi=2000, dtype=torch.float16,
+                                   scale_inputs=False, tail_fill=float("nan"),
+                                   ctx_head=[5000, 17, 2050][:rows])
+    got = _run_attention(batch, device, use_cu=False).float().cpu()
+    ref = _oracle(batch)
+    assert (got - ref).abs().max() <= 3e-3 * ref.abs().max()
+    assert (got - ref).norm() <= 1e-3 * ref.norm()
+    if rows > 3:     # a row without tokens is zero
+        batch.context_lens[2] = 0
+        got = _run_attention(batch, device, use_cu=False).float().cpu()
+        assert (got[2] == 0).all() and torch.isfinite(got).all()
+
+
 @pytest.mark.parametrize("heads", [(16, 8, 128), (8, 1, 64), (32, 4, 128)])
 def test_decode_lockstep_interval_bit_identical(device, heads, monkeypatch):
     """The persistent kernel's wavefront lockstep barrier (LV_ATTN_SYNC,
