@@ -43,6 +43,62 @@ template <> struct Mfma32<f16> {
   }
 };
 
+// 16 x 16 instructions (the matrix-core decode kernel).  Layouts:
+//   A[i][k]: lane i + 16 * (k / E), element k % E    (E = 8: K = 32; E = 4: K = 16)
+//   B[k][j]: lane j + 16 * (k / E), element k % E
+//   D[i][j]: lane j + 16 * (i / 4), element i % 4
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
+
+template <typename T> struct Mfma16;
+template <> struct Mfma16<bf16> {
+  __device__ __forceinline__ static f32x4_t run32(uint4 a, uint4 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  }
+  __device__ __forceinline__ static f32x4_t run16(i16x4_t a, i16x4_t b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
+  }
+  // The leading bits of x that T holds (truncated; x - head(x) is exact).
+  __device__ __forceinline__ static float head(float x) {
+    return __uint_as_float(__float_as_uint(x) & 0xffff0000u);
+  }
+  __device__ __forceinline__ static uint16_t head_bits(float x) {
+    return (uint16_t)(__float_as_uint(x) >> 16);
+  }
+};
+template <> struct Mfma16<f16> {
+  __device__ __forceinline__ static f32x4_t run32(uint4 a, uint4 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
+                                                  __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  }
+  __device__ __forceinline__ static f32x4_t run16(i16x4_t a, i16x4_t b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4_t, a),
+                                                 __builtin_bit_cast(f16x4_t, b), c, 0, 0, 0);
+  }
+  __device__ __forceinline__ static float head(float x) { return (float)(_Float16)x; }
+  __device__ __forceinline__ static uint16_t head_bits(float x) { return float_to_f16_bits(x); }
+};
+
+// 16 bytes per lane from global memory (base + the lane's byte offset) into
+// LDS at byte address lds + 16 lane, issued from inline assembly: the
+// compiler does not track it, so nothing waits for it but wait_vmcnt.
+// lds and base are the same in every lane.  Kernels that use this read M0
+// nowhere else.
+__device__ __forceinline__ void load_lds16_stream(uint64_t base, uint32_t offset, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, %2 nt" ::"v"(offset), "s"(lds),
+               "s"(base)
+               : "memory", "m0");
+}
+
+// Waits until at most N of the wavefront's vector-memory operations are
+// outstanding (they complete in order) (wait_lds: until
+// its LDS operations are done).
+template <int N>
+__device__ __forceinline__ void wait_vmem() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // 16 bytes per lane from global memory straight into LDS at wave base + 16 lane.
 __device__ __forceinline__ void load_lds16(const void* g, uint16_t* lds_wave_base) {

@@ -303,7 +303,8 @@ __global__ __launch_bounds__(kAttnThreads) void attn_rows_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Persistent decode kernel.
+// Persistent decode kernel, vector form: fp32, and bf16 / fp16 batches whose
+// row offsets the matrix-core form below has no LDS for.
 //
 // The blocks of all decode sequences form one flattened list (sequence-major:
 // sequence s owns entries off[s] .. off[s+1]-1, off = exclusive scan of
@@ -389,6 +390,49 @@ __device__ void scan_block_counts(const int32_t* __restrict__ ctx,
   }
   if (t == nt - 1) s_off[n] = s_part[nt - 1];
   __syncthreads();
+}
+
+// A flattened list entry: its sequence, its block in the sequence's table and
+// that block's physical id (clamped and reported if out of range).
+struct Entry { int seq, blk, phys; };
+
+__device__ __forceinline__ Entry resolve_entry(int j, bool live, const int32_t* s_off,
+                                               const int32_t* s_skip, int num_seqs,
+                                               const int32_t* __restrict__ block_tables,
+                                               int max_blocks, int64_t num_cache_blocks) {
+  Entry e{0, 0, 0};
+  if (live) {
+    int lo = 0, hi = num_seqs - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (s_off[mid] <= j) lo = mid; else hi = mid - 1;
+    }
+    e.seq = lo;
+    e.blk = j - s_off[lo] + (s_skip ? s_skip[lo] : 0);
+    e.phys = block_tables[(int64_t)lo * max_blocks + e.blk];
+    if (e.phys < 0 || e.phys >= num_cache_blocks) {   // clamped and reported
+      report_device_error(LV_DEVERR_BLOCK_ID);
+      e.phys = 0;
+    }
+  }
+  return e;
+}
+
+// ws_off: offsets [num_seqs + 1], each sequence's skipped blocks [num_seqs],
+// then its header word [num_seqs] (written by one workgroup).
+template <int BS>
+__device__ __forceinline__ void write_row_headers(int32_t* __restrict__ ws_off,
+                                                  const int32_t* s_off, const int32_t* s_skip,
+                                                  int num_seqs, const RangeSplit& rs) {
+  for (int i = threadIdx.x; i <= num_seqs; i += blockDim.x) {
+    ws_off[i] = s_off[i];
+    if (i < num_seqs) {
+      const int skip = s_skip ? s_skip[i] : 0;
+      if (s_skip) ws_off[num_seqs + 1 + i] = skip;
+      const int nsplit = (skip * BS + kPrefixKeysPerSplit - 1) / kPrefixKeysPerSplit;
+      ws_off[2 * num_seqs + 1 + i] = row_header(s_off[i], s_off[i + 1], rs, nsplit);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -950,21 +994,8 @@ __global__ __launch_bounds__(kPersistMaxWaves * 64) void attn_decode_persistent_
   scan_block_counts<BS>(ctx, pfx.blocks, num_seqs, max_tokens, s_off, s_part, s_skip);
   const int total = s_off[num_seqs];
   const int H = num_kv_heads * G;
-  const int grid = (int)gridDim.x;
-
-  const RangeSplit rs = make_range_split(total, grid);
-  // ws_off: offsets [num_seqs + 1], each sequence's skipped blocks
-  // [num_seqs], then its header word [num_seqs]
-  if (blockIdx.x == 0)
-    for (int i = threadIdx.x; i <= num_seqs; i += blockDim.x) {
-      ws_off[i] = s_off[i];
-      if (i < num_seqs) {
-        const int skip = has_pfx ? s_skip[i] : 0;
-        if (has_pfx) ws_off[num_seqs + 1 + i] = skip;
-        const int nsplit = (skip * BS + kPrefixKeysPerSplit - 1) / kPrefixKeysPerSplit;
-        ws_off[2 * num_seqs + 1 + i] = row_header(s_off[i], s_off[i + 1], rs, nsplit);
-      }
-    }
+  const RangeSplit rs = make_range_split(total, (int)gridDim.x);
+  if (blockIdx.x == 0) write_row_headers<BS>(ws_off, s_off, has_pfx ? s_skip : nullptr, num_seqs, rs);
   if (total == 0) return;
   const int r0 = rs.start((int)blockIdx.x);
   const int r1 = rs.start((int)blockIdx.x + 1);
@@ -1000,57 +1031,6 @@ __global__ __launch_bounds__(kPersistMaxWaves * 64) void attn_decode_persistent_
       if (whole && cur_skip > 0) {
         // fold in the prefix partials (splits of 128 keys), then normalise
         const int nsplit = (cur_skip * BS + kPrefixKeysPerSplit - 1) / kPrefixKeysPerSplit;
-        if constexpr (G <= 2) {
-          if (nsplit <= 4) {
-            // up to four splits: every partial is loaded in one round trip,
-            // then merged in the order of the general loop below
-            float qm[G][4], ql[G][4], qa[G][4][S::VEC];
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-              const int64_t pb = ((int64_t)sq * H + kvh * G + g) * kPrefixMaxSplits;
-#pragma unroll
-              for (int sp = 0; sp < 4; ++sp) {
-                qm[g][sp] = kNegBig;
-                ql[g][sp] = 0.0f;
-#pragma unroll
-                for (int j = 0; j < S::VEC; ++j) qa[g][sp][j] = 0.0f;
-                if (sp < nsplit) {
-                  qm[g][sp] = pfx.ml[(pb + sp) * 2];
-                  ql[g][sp] = pfx.ml[(pb + sp) * 2 + 1];
-                  const float* ap = pfx.acc + (pb + sp) * D + st.dc * VEC;
-#pragma unroll
-                  for (int j = 0; j < S::VEC; ++j) qa[g][sp][j] = ap[j];
-                }
-              }
-            }
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-              const int hq = kvh * G + g;
-              float mx = st.m[g];
-#pragma unroll
-              for (int sp = 0; sp < 4; ++sp)
-                if (sp < nsplit) mx = fmaxf(mx, qm[g][sp]);
-              const float fs = fast_exp2(st.m[g] - mx);
-              float L = st.l[g] * fs;
-              float o[S::VEC];
-#pragma unroll
-              for (int j = 0; j < S::VEC; ++j) o[j] = st.acc[g][j] * fs;
-#pragma unroll
-              for (int sp = 0; sp < 4; ++sp)
-                if (sp < nsplit) {
-                  const float f = ql[g][sp] * fast_exp2(qm[g][sp] - mx);
-                  L += f;
-#pragma unroll
-                  for (int j = 0; j < S::VEC; ++j) o[j] = fmaf(qa[g][sp][j], f, o[j]);
-                }
-              const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-              T* op = out + (int64_t)sq * out_stride + (int64_t)hq * D + st.dc * VEC;
-#pragma unroll
-              for (int j = 0; j < VEC; ++j) elem<T>::store(op + j, o[j] * inv);
-            }
-            return;
-          }
-        }
 #pragma unroll
         for (int g = 0; g < G; ++g) {
           const int hq = kvh * G + g;
@@ -1103,31 +1083,16 @@ __global__ __launch_bounds__(kPersistMaxWaves * 64) void attn_decode_persistent_
   uint4 k3[NBUF == 4 ? S::LOADS : 1], v3[NBUF == 4 ? S::LOADS : 1];
   for (int base = r0; base < r1; base += 64) {
     const int cnt = min(64, r1 - base);
-    // Lane i resolves flattened entry base + i: its sequence, logical block
-    // and physical block id.
-    int lseq = 0, lblk = 0, id = 0;
-    if (lane < cnt) {
-      const int j = base + lane;
-      int lo = 0, hi = num_seqs - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (s_off[mid] <= j) lo = mid; else hi = mid - 1;
-      }
-      lseq = lo;
-      lblk = j - s_off[lo] + (has_pfx ? s_skip[lo] : 0);   // block index in the table
-      id = block_tables[(int64_t)lo * max_blocks + lblk];
-      if (id < 0 || id >= num_cache_blocks) {   // clamped and reported
-        report_device_error(LV_DEVERR_BLOCK_ID);
-        id = 0;
-      }
-    }
-    auto phys = [&](int i) { return __builtin_amdgcn_readlane(id, min(i, cnt - 1)); };
+    // Lane i resolves flattened entry base + i.
+    const Entry en = resolve_entry(base + lane, lane < cnt, s_off, has_pfx ? s_skip : nullptr,
+                                   num_seqs, block_tables, max_blocks, num_cache_blocks);
+    auto phys = [&](int i) { return __builtin_amdgcn_readlane(en.phys, min(i, cnt - 1)); };
     // Start (or continue) the sequence of entry i, then fold its block in;
     // i >= cnt is a fully masked no-op so process() always runs.
     auto visit = [&](const uint4* kk, const uint4* vv, int i) {
       const bool real = i < cnt;
-      const int sq = __builtin_amdgcn_readlane(lseq, min(i, cnt - 1));
-      const int lb = __builtin_amdgcn_readlane(lblk, min(i, cnt - 1));
+      const int sq = __builtin_amdgcn_readlane(en.seq, min(i, cnt - 1));
+      const int lb = __builtin_amdgcn_readlane(en.blk, min(i, cnt - 1));
       if (real && sq != cur) {
         if (cur >= 0) finish(cur);
         cur = sq;
@@ -1209,6 +1174,316 @@ struct MergeState {
     }
   }
 };
+
+// ---------------------------------------------------------------------------
+// Persistent decode kernel on the matrix cores (bf16 / fp16).
+//
+// The same flattened block list, ranges, pieces and lockstep as
+// attn_decode_persistent_kernel above; only a wavefront's work on a block
+// differs.  There every lane multiplies its 8 dims of a K row with all G
+// query heads: 2 G multiply-adds per loaded element, about 400 + 50 G vector
+// instructions per block, which at G = 8 is the bound and not HBM.  Here a
+// 16-token block of one kv head is one 16 x 16 tile:
+//   * K and V go from HBM to LDS directly (two stages of one block, private
+//     to the wavefront, so no barrier guards them; block i + 1 is in flight
+//     while block i is computed);
+//   * S^T = K Q^T: rows = tokens, columns = query heads, D / 32 products of
+//     16x16x32.  The 16 columns repeat the G heads, so every lane has the
+//     scores of its column's head;
+//   * softmax in fp32, one reference maximum per column, raised only when a
+//     score exceeds it by 2^4;
+//   * O^T += V^T P^T, D / 16 products of 16x16x16 with V^T by the LDS
+//     transpose read.  P stays fp32-exact: its leading, middle and trailing
+//     bits (8 each in bf16, 11 each in fp16) are three values of the
+//     element type in three columns of the same product (G = 8: the third
+//     in a second product), so O sums the fp32 weights' products in fp32.
+// Column c of a tile is head c % G, part c / G of P (parts past the third
+// are zero).
+//
+// LDS row r of a block holds its 16-byte chunk j at j ^ swz(r); the token of
+// tile row 4 g + e is 4 perm(g) + e, perm = 0 2 1 3.  With D = 128 swz is
+// ChunkLds's; with D = 64 two rows share the 64 banks, and swz takes pairs of
+// rows through 0 2 1 3 4 6 5 7.  Both keep the K reads (16 rows, one chunk)
+// and the transpose reads (rows 0-3 and 8-11, or 4-7 and 12-15, two chunks)
+// free of bank conflicts.
+// ---------------------------------------------------------------------------
+template <typename T, int D>
+struct MfmaBlock {
+  static constexpr int BS = 16;
+  static constexpr int CPR = D / 8;            // 16-byte chunks per row
+  static constexpr int RPL = 64 / CPR;         // rows one 64-lane load fills
+  static constexpr int LOADS = BS / RPL;       // loads per K or V block
+  static constexpr int KBYTES = BS * D * 2;    // one K or V block
+  static constexpr int STAGE = 2 * KBYTES;
+  __device__ __forceinline__ static int swz(int row) {
+    if constexpr (D == 128) return ChunkLds<128, 4>::swz(row);
+    return (int)((0x75643120u >> (4 * (row >> 1))) & 7);
+  }
+  __device__ __forceinline__ static int at(int row, int chunk) {   // bytes
+    return row * (2 * D) + 16 * (chunk ^ swz(row));
+  }
+};
+
+// Sum over the columns that hold parts of the same head (c, c + G, ...).
+template <int G>
+__device__ __forceinline__ float part_sum(float x) {
+  x += dpp<0x128>(x);                          // row_ror:8
+  if constexpr (G <= 4) x += dpp<0x124>(x);    // row_ror:4
+  if constexpr (G <= 2) x += dpp<0x122>(x);    // row_ror:2
+  if constexpr (G <= 1) x += dpp<0x121>(x);    // row_ror:1
+  return x;
+}
+
+// Dynamic LDS the kernel may ask for: a CU's 160 KB less s_part and slack.
+constexpr size_t kMfmaMaxDynLds = (160 - 4) * 1024;
+
+template <int G>
+__device__ __forceinline__ float part_max(float x) {
+  x = fmaxf(x, dpp<0x128>(x));
+  if constexpr (G <= 4) x = fmaxf(x, dpp<0x124>(x));
+  if constexpr (G <= 2) x = fmaxf(x, dpp<0x122>(x));
+  if constexpr (G <= 1) x = fmaxf(x, dpp<0x121>(x));
+  return x;
+}
+
+template <typename T, int D, int G, int BS>
+__global__ __launch_bounds__(kPersistMaxWaves * 64) void attn_decode_mfma_kernel(
+    const T* __restrict__ q, int64_t q_stride,
+    const T* __restrict__ kc, const T* __restrict__ vc, int num_kv_heads, int64_t num_cache_blocks,
+    const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ ctx,
+    int num_seqs, float scale_log2, T* __restrict__ out, int64_t out_stride,
+    int32_t* __restrict__ ws_off, float* __restrict__ ws_acc, float* __restrict__ ws_ml,
+    PrefixArgs pfx, int sync_mask) {
+  using M = Mfma16<T>;
+  using B = MfmaBlock<T, D>;
+  static_assert(BS == B::BS, "16-token blocks");
+  constexpr int QS = D / 32;                   // k-steps of K Q^T
+  constexpr int NB = D / 16;                   // 16-dim blocks of O^T
+  // fp16 weights are kept between 2^-14 and 2^15: the reference maximum sits
+  // 2^10 under the score that set it
+  constexpr float kLift = std::is_same<T, f16>::value ? 10.0f : 0.0f;
+  // LDS: the wavefronts' stages, s_off [num_seqs + 1], then (shared prefixes
+  // only) s_skip [num_seqs]
+  extern __shared__ __align__(16) unsigned char s_dyn[];
+  __shared__ int32_t s_part[kPersistMaxWaves * 64];
+  int32_t* s_off = reinterpret_cast<int32_t*>(s_dyn + num_kv_heads * 2 * B::STAGE);
+  int32_t* s_skip = s_off + num_seqs + 1;
+  const int max_tokens = max_blocks * BS;
+  const bool has_pfx = pfx.blocks != nullptr;
+  scan_block_counts<BS>(ctx, pfx.blocks, num_seqs, max_tokens, s_off, s_part, s_skip);
+  const int total = s_off[num_seqs];
+  const int H = num_kv_heads * G;
+  const RangeSplit rs = make_range_split(total, (int)gridDim.x);
+  if (blockIdx.x == 0) write_row_headers<BS>(ws_off, s_off, has_pfx ? s_skip : nullptr, num_seqs, rs);
+  if (total == 0) return;
+  const int r0 = rs.start((int)blockIdx.x);
+  const int r1 = rs.start((int)blockIdx.x + 1);
+  if (r0 >= r1) return;
+
+  const int lane = threadIdx.x & 63;
+  const int kvh = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const int head = col % G, part = col / G;
+  const int64_t tok_stride = (int64_t)num_kv_heads * D;
+  const uint64_t blk_bytes = (uint64_t)BS * tok_stride * sizeof(T);
+  const unsigned char* stage0 = s_dyn + kvh * 2 * B::STAGE;
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
+      (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)stage0);
+  const uint64_t kbase = (uint64_t)(kc + (int64_t)kvh * D);
+  const uint64_t vbase = (uint64_t)(vc + (int64_t)kvh * D);
+
+  // Load u of a block fills rows RPL u ..: lane l's 16 bytes land in slot
+  // l % CPR of row RPL u + l / CPR, which holds chunk slot ^ swz(row).
+  uint32_t goff[B::LOADS];
+#pragma unroll
+  for (int u = 0; u < B::LOADS; ++u) {
+    const int r = B::RPL * u + lane / B::CPR;
+    goff[u] = (uint32_t)(r * tok_stride * (int)sizeof(T)) + 16u * ((lane % B::CPR) ^ B::swz(r));
+  }
+  auto stage = [&](int s, int phys) __attribute__((always_inline)) {
+    const uint64_t at = (uint64_t)(uint32_t)phys * blk_bytes;
+    const uint32_t dst = lds0 + s * B::STAGE;
+    wait_lds();      // the stage's last reads have returned
+#pragma unroll
+    for (int u = 0; u < B::LOADS; ++u) load_lds16_stream(kbase + at, goff[u], dst + 1024 * u);
+#pragma unroll
+    for (int u = 0; u < B::LOADS; ++u)
+      load_lds16_stream(vbase + at, goff[u], dst + B::KBYTES + 1024 * u);
+  };
+
+  // LDS byte offsets of the tile operands, and the tokens of this lane's
+  // four scores.
+  auto perm = [](int x) { return ((x & 1) << 1) | (x >> 1); };
+  const int krow = 4 * perm(col >> 2) + (col & 3);
+  int koff[QS], voff[NB];
+#pragma unroll
+  for (int s = 0; s < QS; ++s) koff[s] = B::at(krow, 4 * s + g);
+  const int vrow = 4 * perm(g) + (col >> 2);
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+    voff[b] = B::at(vrow, 2 * b + ((col & 3) >> 1)) + 8 * (col & 1);
+  const int tok0 = 4 * perm(g);
+
+  uint4 qf[QS];
+  f32x4_t o[NB];
+  float m = kNegBig, l = 0.0f;
+  int cur = -1, cur_end = 0, cur_skip = 0;   // as in the kernel above
+
+  auto start = [&](int sq) __attribute__((always_inline)) {
+    cur = sq;
+    cur_end = min(max(ctx[sq], 0), max_tokens);
+    cur_skip = has_pfx ? s_skip[sq] : 0;
+    const T* qp = q + (int64_t)sq * q_stride + (int64_t)(kvh * G + head) * D + 8 * g;
+#pragma unroll
+    for (int s = 0; s < QS; ++s) qf[s] = load16(qp + 32 * s);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) o[b] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    m = kNegBig;
+    l = 0.0f;
+  };
+
+  auto process = [&](int s, int blk) __attribute__((always_inline)) {
+    unsigned char* kt = s_dyn + kvh * 2 * B::STAGE + s * B::STAGE;
+    unsigned char* vt = kt + B::KBYTES;
+    const int left = cur_end - blk * BS;       // tokens of the block in the context
+    if (left < BS) {
+      // rows past the context may hold anything: zero their V (0 * NaN)
+      for (int c = lane; c < BS * B::CPR; c += 64)
+        if (c / B::CPR >= left)
+          *reinterpret_cast<uint4*>(vt + 16 * c) = make_uint4(0, 0, 0, 0);
+    }
+    uint4 kf[QS];
+#pragma unroll
+    for (int i = 0; i < QS; ++i) kf[i] = *reinterpret_cast<const uint4*>(kt + koff[i]);
+    i16x4_t vf[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) vf[b] = lds_read_tr16(reinterpret_cast<uint16_t*>(vt + voff[b]));
+    f32x4_t sc = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < QS; ++i) sc = M::run32(kf[i], qf[i], sc);
+    float x[4], mx = kNegBig;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      x[e] = sc[e] * scale_log2;
+      if (left < BS && tok0 + e >= left) x[e] = kNegBig;
+      mx = fmaxf(mx, x[e]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = xor32_max(mx);
+    if (__ballot(mx - kLift > m + 4.0f)) {     // uniform; rare after a row's first block
+      if (mx - kLift > m + 4.0f) {
+        const float alpha = fast_exp2(m - (mx - kLift));
+        m = mx - kLift;
+        l *= alpha;
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[b][e] *= alpha;
+      }
+    }
+    uint16_t w0[4], w1[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool in = !(left < BS && tok0 + e >= left);
+      const float p = in ? fast_exp2(x[e] - m) : 0.0f;
+      l += p;
+      const float r1 = p - M::head(p), r2 = r1 - M::head(r1);
+      const uint16_t b0 = M::head_bits(p), b1 = M::head_bits(r1), b2 = M::head_bits(r2);
+      w0[e] = part == 0 ? b0 : part == 1 ? b1 : part == 2 ? b2 : (uint16_t)0;
+      w1[e] = part == 0 ? b2 : (uint16_t)0;
+    }
+    const i16x4_t p0 = {(short)w0[0], (short)w0[1], (short)w0[2], (short)w0[3]};
+#pragma unroll
+    for (int b = 0; b < NB; ++b) o[b] = M::run16(vf[b], p0, o[b]);
+    if constexpr (G == 8) {
+      const i16x4_t p1 = {(short)w1[0], (short)w1[1], (short)w1[2], (short)w1[3]};
+#pragma unroll
+      for (int b = 0; b < NB; ++b) o[b] = M::run16(vf[b], p1, o[b]);
+    }
+  };
+
+  // As in the kernel above: whole rows to `out` (with their prefix partials,
+  // the columns of a head taking splits part, part + 16 / G, ... each), other
+  // pieces to their slots.  Lane (col < G, g) writes head col, dims 16 b + 4 g ..
+  auto finish = [&](int sq) __attribute__((always_inline)) {
+    const int a = s_off[sq];
+    const bool whole = a >= r0 && s_off[sq + 1] <= r1;
+    const int hq = kvh * G + head;
+    float L = l + __shfl_xor(l, 16);
+    L = xor32_sum(L);
+    if (whole && cur_skip > 0) {
+      const int nsplit = (cur_skip * BS + kPrefixKeysPerSplit - 1) / kPrefixKeysPerSplit;
+      const int64_t pb = ((int64_t)sq * H + hq) * kPrefixMaxSplits;
+      float mm = m;
+      if (part != 0) L = 0.0f;
+      for (int sp = part; sp < nsplit; sp += 16 / G) {
+        const float2 ml = *reinterpret_cast<const float2*>(pfx.ml + (pb + sp) * 2);
+        const float* ap = pfx.acc + (pb + sp) * D + 4 * g;
+        float4 v[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) v[b] = *reinterpret_cast<const float4*>(ap + 16 * b);
+        const float mx = fmaxf(mm, ml.x);
+        const float fs = fast_exp2(mm - mx), f = ml.y * fast_exp2(ml.x - mx);
+        mm = mx;
+        L = L * fs + f;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          o[b][0] = fmaf(o[b][0], fs, v[b].x * f); o[b][1] = fmaf(o[b][1], fs, v[b].y * f);
+          o[b][2] = fmaf(o[b][2], fs, v[b].z * f); o[b][3] = fmaf(o[b][3], fs, v[b].w * f);
+        }
+      }
+      const float mx = part_max<G>(mm);
+      const float fs = fast_exp2(mm - mx);
+      L = part_sum<G>(L * fs);
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[b][e] *= fs;
+    }
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[b][e] = part_sum<G>(o[b][e]);
+    if (col >= G) return;
+    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    if (whole) {
+      T* op = out + (int64_t)sq * out_stride + (int64_t)hq * D + 4 * g;
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) elem<T>::store(op + 16 * b + e, o[b][e] * inv);
+      return;
+    }
+    const int slot = piece_slot(sq, rs.piece_rank(a, (int)blockIdx.x), (int)blockIdx.x, num_seqs);
+    const int64_t base = (int64_t)slot * H + hq;
+    float* wp = ws_acc + base * D + 4 * g;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      *reinterpret_cast<float4*>(wp + 16 * b) =
+          make_float4(o[b][0] * inv, o[b][1] * inv, o[b][2] * inv, o[b][3] * inv);
+    if (g == 0) { ws_ml[base * 2] = m; ws_ml[base * 2 + 1] = L; }
+  };
+
+  for (int base = r0; base < r1; base += 64) {
+    const int cnt = min(64, r1 - base);
+    const Entry en = resolve_entry(base + lane, lane < cnt, s_off, has_pfx ? s_skip : nullptr,
+                                   num_seqs, block_tables, max_blocks, num_cache_blocks);
+    stage(0, __builtin_amdgcn_readlane(en.phys, 0));
+    for (int i = 0; i < cnt; ++i) {
+      if (sync_mask >= 0 && (i & sync_mask) == 0) __builtin_amdgcn_s_barrier();
+      const int sq = __builtin_amdgcn_readlane(en.seq, i);
+      if (i + 1 < cnt) stage((i + 1) & 1, __builtin_amdgcn_readlane(en.phys, i + 1));
+      if (sq != cur) {
+        if (cur >= 0) finish(cur);
+        start(sq);
+      }
+      if (i + 1 < cnt) wait_vmem<2 * B::LOADS>();   // block i has landed, i + 1 may not have
+      else wait_vmem<0>();
+      process(i & 1, __builtin_amdgcn_readlane(en.blk, i));
+    }
+  }
+  if (cur >= 0) finish(cur);
+}
 
 // Where a row's partials lie: entry i < np is the row's i-th walked piece,
 // entry np + k its k-th prefix split.
@@ -1485,16 +1760,22 @@ struct AttnPlan {
 };
 
 static AttnPlan plan_decode(int num_decodes, int num_heads, int num_kv_heads, int head_dim,
-                            int block_size, int max_blocks) {
+                            int block_size, int max_blocks, lv_dtype dtype) {
   AttnPlan p{};
   p.nt = !env_is("LV_ATTN_NT", '0');
   p.persistent = !env_is("LV_ATTN_DECODE_KERNEL", 'r') && num_kv_heads <= kPersistMaxWaves &&
                  num_decodes <= kPersistMaxSeqs;
   if (p.persistent) {
-    // One workgroup of num_kv_heads wavefronts per CU; each wavefront keeps
-    // NBUF - 1 blocks (8 KiB each at the Qwen3 shape) in flight.
+    // Workgroups of num_kv_heads wavefronts.  fp32 (vector kernel): one per
+    // CU, each wavefront keeping NBUF - 1 blocks in flight.  bf16 / fp16
+    // (matrix cores): enough that a CU has some eight wavefronts, two 8 KB
+    // stages each at head_dim 128.  Measured (1 / 2 / 3 / 4 per CU, us): 4 kv
+    // heads 59.4 / 55.4 / 65.8 / 63.9; 2 kv heads, 256 rows 85.2 / 63.2 /
+    // 59.8 / 62.2; 1 kv head 41.3 / 27.5 / 22.7 / 21.8; 8 kv heads 179.7 / 193.
     p.nbuf = env_int("LV_ATTN_NBUF", 2) == 4 ? 4 : 2;
-    p.num_wgs = env_int("LV_ATTN_PERSIST_WGS", device_cu_count() * (num_kv_heads == 1 ? 4 : 1));
+    const int per_cu = dtype == LV_F32 ? (num_kv_heads == 1 ? 4 : 1)
+                       : num_kv_heads >= 5 ? 1 : num_kv_heads >= 3 ? 2 : num_kv_heads == 2 ? 3 : 4;
+    p.num_wgs = env_int("LV_ATTN_PERSIST_WGS", device_cu_count() * per_cu);
     // wavefront lockstep interval in blocks (LV_ATTN_SYNC=0: none)
     int sync = env_is("LV_ATTN_SYNC", '0') ? 0 : env_int("LV_ATTN_SYNC", 4);
     int pow2 = 2;
@@ -1563,11 +1844,31 @@ static void launch_persistent(const void* q, int64_t q_stride, const void* kc, c
                          dim3((unsigned)(pfx.max_items * num_kv_heads)), dim3(256), 0, st, ca);
     }
   }
-  const size_t lds = sizeof(int32_t) * (size_t)(num_seqs + 1 + (pfx.blocks ? num_seqs : 0));
-  hipLaunchKernelGGL((attn_decode_persistent_kernel<T, D, G, BS, NT, NBUF>), dim3(p.num_wgs),
-                     dim3(64 * num_kv_heads), lds, st, (const T*)q, q_stride, (const T*)kc,
-                     (const T*)vc, num_kv_heads, num_cache_blocks, bt, max_blocks, ctx, num_seqs,
-                     scale_log2, (T*)out, out_stride, ws_off, ws_acc, ws_ml, pfx, p.sync_mask);
+  // Matrix cores for bf16 / fp16 at every group size (calls as graph replays,
+  // vector kernel -> this one, same box: 256 rows of G = 2 188.2 -> 179.9 us,
+  // 48 rows of G = 4 91 -> 75, of G = 8 143 -> 79.5, 5 long rows of 2 kv heads
+  // and G = 8 118 -> 34, one row 14.1 -> 12.3); the vector kernel for fp32,
+  // and where the row offsets no longer fit in LDS beside the stages (about
+  // 7100 rows at 8 kv heads of 128 dims, half that with shared prefixes).
+  size_t lds = sizeof(int32_t) * (size_t)(num_seqs + 1 + (pfx.blocks ? num_seqs : 0));
+  bool vector = true;
+  if constexpr (!std::is_same<T, float>::value) {
+    const size_t stages = (size_t)num_kv_heads * 2 * MfmaBlock<T, D>::STAGE;
+    if (stages + lds <= kMfmaMaxDynLds) {
+      vector = false;
+      hipLaunchKernelGGL((attn_decode_mfma_kernel<T, D, G, BS>), dim3(p.num_wgs),
+                         dim3(64 * num_kv_heads), stages + lds, st, (const T*)q, q_stride,
+                         (const T*)kc, (const T*)vc, num_kv_heads, num_cache_blocks, bt,
+                         max_blocks, ctx, num_seqs, scale_log2, (T*)out, out_stride, ws_off,
+                         ws_acc, ws_ml, pfx, p.sync_mask);
+    }
+  }
+  if (vector)
+    hipLaunchKernelGGL((attn_decode_persistent_kernel<T, D, G, BS, NT, NBUF>), dim3(p.num_wgs),
+                       dim3(64 * num_kv_heads), lds, st, (const T*)q, q_stride, (const T*)kc,
+                       (const T*)vc, num_kv_heads, num_cache_blocks, bt, max_blocks, ctx,
+                       num_seqs, scale_log2, (T*)out, out_stride, ws_off, ws_acc, ws_ml, pfx,
+                       p.sync_mask);
   const int H = num_kv_heads * G;
   // A workgroup per (row, query head) while a row spans three ranges or more
   // on average; past that most rows have one or two pieces and the extra
@@ -1606,10 +1907,14 @@ static void launch(const LaunchArgs& a, const AttnPlan& p, char* ws) {
                                            a.num_cache_blocks, a.bt, a.max_blocks, a.ctx,       \
                                            a.n_rows, a.scale_log2, a.out, a.out_stride, p, ws,  \
                                            a.pfx, a.st)
-    if (p.nt && p.nbuf == 4) LV_PERSIST(true, 4);
-    else if (p.nt) LV_PERSIST(true, 2);
-    else if (p.nbuf == 4) LV_PERSIST(false, 4);
-    else LV_PERSIST(false, 2);
+    if constexpr (std::is_same<T, float>::value) {   // the knobs are the vector kernel's
+      if (p.nt && p.nbuf == 4) LV_PERSIST(true, 4);
+      else if (p.nt) LV_PERSIST(true, 2);
+      else if (p.nbuf == 4) LV_PERSIST(false, 4);
+      else LV_PERSIST(false, 2);
+    } else {
+      LV_PERSIST(true, 2);
+    }
 #undef LV_PERSIST
   } else if (p.nt) {
     launch_rows<T, D, G, BS, true>(a.q, a.q_stride, a.kc, a.vc, a.num_kv_heads,
@@ -1711,14 +2016,15 @@ extern "C" size_t lv_paged_attention_workspace_size(int32_t num_seqs, int32_t nu
                                                     int32_t head_dim, int32_t block_size,
                                                     int32_t max_blocks, int32_t max_query_len,
                                                     lv_dtype dtype) {
-  (void)num_seqs; (void)num_tokens; (void)max_query_len; (void)dtype;
+  (void)num_seqs; (void)num_tokens; (void)max_query_len;
   if (num_decodes <= 0 || block_size <= 0 || max_blocks <= 0 || num_heads <= 0) return 0;
   // num_kv_heads is not an argument: take the larger of the persistent plan
   // at its biggest grid (one kv head) and the workgroup-per-row plan (used
   // above kPersistMaxWaves kv heads).
-  const lv::AttnPlan a = lv::plan_decode(num_decodes, num_heads, 1, head_dim, block_size, max_blocks);
+  const lv::AttnPlan a = lv::plan_decode(num_decodes, num_heads, 1, head_dim, block_size,
+                                         max_blocks, dtype);
   const lv::AttnPlan b = lv::plan_decode(num_decodes, num_heads, lv::kPersistMaxWaves + 1, head_dim,
-                                         block_size, max_blocks);
+                                         block_size, max_blocks, dtype);
   return a.bytes() > b.bytes() ? a.bytes() : b.bytes();
 }
 
@@ -1769,7 +2075,8 @@ static int paged_attention_impl(const void* query_dev, int64_t q_stride_t,
   // fails before anything is launched.
   AttnPlan pd{};
   if (num_decodes > 0) {
-    pd = plan_decode(num_decodes, num_heads, num_kv_heads, head_dim, block_size, max_blocks);
+    pd = plan_decode(num_decodes, num_heads, num_kv_heads, head_dim, block_size, max_blocks,
+                     dtype);
     // the persistent kernel's flattened block list is indexed in 32 bits
     LV_REQUIRE(!pd.persistent || (int64_t)num_decodes * max_blocks <= (1ll << 31) - (1ll << 16),
                "lv_paged_attention: num_decodes * max_blocks above 2^31 - 2^16 (persistent "

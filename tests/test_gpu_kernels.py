@@ -165,6 +165,50 @@ def test_decode_long_contexts(device):
     _check_attention(got, _oracle(batch), "long contexts")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads", [(16, 8, 128), (6, 3, 128), (20, 5, 64), (64, 8, 128),
+                                   (8, 1, 64), (2, 2, 64)])
+@pytest.mark.parametrize("kind", ["plain", "peaky", "small", "many"])
+def test_decode_matrix_cores_one_rounding(device, dtype, heads, kind):
+    """The matrix-core decode kernel rounds nothing to 16 bits but the output
+    (K Q^T products are exact in fp32, the softmax weights enter V^T P^T as
+    three exact parts): each output is within half a unit in the last place
+    of the fp64 result plus 2e-6 of the largest |value| for fp32 sums.  Block
+    and 64-block edges, NaN past the context, softmaxes dominated by a few
+    keys, values below the smallest normal fp16, and (rows past what its LDS
+    holds) the vector kernel that takes over."""
+    H, Hkv, D = heads
+    _say(f"decode matrix cores {dtype} {heads} {kind}")
+    if kind == "many":
+        batch = workloads.paged_decode(seed=2, num_seqs=7300, num_heads=H, num_kv_heads=Hkv,
+                                       head_dim=D, ctx_lo=1, ctx_hi=20, dtype=dtype,
+                                       scale_inputs=False, tail_fill=float("nan"))
+    else:
+        batch = workloads.paged_decode(seed=3, num_seqs=19, num_heads=H, num_kv_heads=Hkv,
+                                       head_dim=D, ctx_lo=1, ctx_hi=900, dtype=dtype,
+                                       scale_inputs=False, tail_fill=float("nan"),
+                                       ctx_head=[1, 15, 16, 17, 31, 33, 1023, 1024, 1025, 2500])
+        if kind == "peaky":
+            batch.query *= 8
+        if kind == "small":
+            batch.value_cache *= 2.0 ** -18
+    got = _run_attention(batch, device, use_cu=False).double().cpu()
+    G, ulp = H // Hkv, 2.0 ** (-9 if dtype == torch.bfloat16 else -12)
+    tiny = 2.0 ** (-134 if dtype == torch.bfloat16 else -25)   # half the smallest step
+    for r in range(0, batch.query.shape[0], 37 if kind == "many" else 1):
+        n = int(batch.context_lens[r])
+        blk = batch.block_tables[r, :-(-n // 16)].long()
+        k = batch.key_cache[blk].reshape(-1, Hkv, D)[:n].double()
+        v = batch.value_cache[blk].reshape(-1, Hkv, D)[:n].double()
+        for h in range(H):
+            p = torch.softmax(k[:, h // G] @ batch.query[r, h].double() * batch.scale, 0)
+            ref = p @ v[:, h // G]
+            bound = ulp * 2 * ref.abs().clamp_min(2.0 ** -14 if dtype == torch.float16 else 0)
+            bound = torch.maximum(bound, torch.full_like(ref, tiny)) + 2e-6 * v.abs().max()
+            err = (got[r, h] - ref).abs()
+            assert (err <= bound).all(), (r, h, n, float((err / bound).max()))
+
+
 @pytest.mark.parametrize("rows,heads", [(1, (16, 8, 128)), (3, (16, 2, 128)), (7, (8, 8, 64)),
                                         (128, (16, 8, 128)), (129, (16, 8, 128))])
 def test_decode_few_rows_of_many_pieces(device, rows, heads):
