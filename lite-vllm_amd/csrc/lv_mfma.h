@@ -18,9 +18,6 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 typedef short i16x8_t __attribute__((ext_vector_type(8)));
 
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
 
 template <typename T> struct Mfma32;
 template <> struct Mfma32<bf16> {
@@ -30,7 +27,7 @@ template <> struct Mfma32<bf16> {
   }
   // Two fp32 values -> packed pair, round to nearest even (v_cvt_pk_bf16_f32).
   __device__ __forceinline__ static uint32_t pack2(float a, float b) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, bf16x2_t));
+    return float_to_bf16_pair(a, b);
   }
 };
 template <> struct Mfma32<f16> {

@@ -136,3 +136,54 @@ def test_silu_mul_matches_oracle(device, dtype, T, inter):
     want = L.silu_mul(gu)
     got = ops.silu_mul(gu.to(device))
     _close(got, want, dtype, exact_frac=0.98)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,Hkv,D", [(16, 8, 128), (4, 2, 64), (8, 1, 256), (6, 3, 128)])
+@pytest.mark.parametrize("form", ["vector", "few tokens", "odd rows"])
+def test_qk_norm_rope_cache_forms(device, dtype, H, Hkv, D, form):
+    """The 16-byte form (from 4096 head slots on, aligned rows) and the scalar
+    one on either side of that line and for rows off 16-byte boundaries:
+    oracle bar, padding and out-of-range slots unwritten, rows at positions
+    without a cos / sin entry NaN."""
+    _say(f"qk_norm_rope_cache {form} {dtype} {H} {Hkv} {D}")
+    per = H + 2 * Hkv
+    T = -(-4096 // per) + (3 if form == "odd rows" else -1 if form == "few tokens" else 0)
+    g = torch.Generator().manual_seed(T)
+    nb, P = T // 16 + 3, 999
+    pad = 1 if form == "odd rows" else 0
+    qkv = torch.randn(T, per * D + pad, generator=g).to(dtype)
+    cos, sin = _rope_tables(D, P, dtype)
+    pos = torch.randint(0, P, (T,), generator=g)
+    slots = torch.randperm(nb * 16, generator=g)[:T]
+    slots[1] = -1
+    qw, kw = ((torch.rand(D, generator=g) + 0.5).to(dtype) for _ in range(2))
+    kc = torch.full((nb, 16, Hkv, D), 3.0, dtype=dtype)
+    vc = torch.full((nb, 16, Hkv, D), 3.0, dtype=dtype)
+    kc_d, vc_d = kc.to(device), vc.to(device)
+    want = L.qk_norm_rope_cache(qkv[:, :per * D], H, Hkv, D, cos, sin, pos, slots, kc, vc, qw, kw,
+                                1e-6)
+    bad_pos, bad_slot = pos.clone(), slots.clone()
+    bad_pos[2], bad_slot[3] = P, nb * 16
+    last = slots[3]
+    kc.view(-1, Hkv, D)[last] = 3.0
+    vc.view(-1, Hkv, D)[last] = 3.0
+    dv = lambda t: t.to(device)
+    ops.device_errors(clear=True)
+    got = ops.qk_norm_rope_cache(dv(qkv)[:, :per * D], H, Hkv, D, dv(cos), dv(sin), dv(bad_pos),
+                                 dv(bad_slot), kc_d, vc_d, q_norm_weight=dv(qw),
+                                 k_norm_weight=dv(kw), eps=1e-6).cpu()
+    assert ops.device_errors(clear=True) == 2      # LV_DEVERR_SLOT
+    assert got[2].isnan().all() and kc_d.cpu().view(-1, Hkv, D)[slots[2]].isnan().all()
+    keep = torch.arange(T) != 2
+
+    def pair_mag(x):
+        a, b = x.float().chunk(2, dim=-1)
+        m = (a * a + b * b).sqrt()
+        return torch.cat([m, m], dim=-1)
+    _close(got[keep], want[keep], dtype, scale=pair_mag(want[keep]))
+    rest = torch.ones(nb * 16, dtype=torch.bool)
+    rest[slots[2]] = False
+    gk, wk = kc_d.cpu().view(-1, Hkv, D)[rest], kc.view(-1, Hkv, D)[rest]
+    _close(gk, wk, dtype, scale=pair_mag(wk))
+    assert torch.equal(vc_d.cpu(), vc)
