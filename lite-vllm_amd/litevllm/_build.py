@@ -69,6 +69,29 @@ def _compile(src: Path, hipcc: str) -> Path:
     return obj
 
 
+def _build_native() -> Path:
+    """Compile litevllm/_native.so (host code only): the direct calls of the C
+    ABI on torch tensors that litevllm/ops.py makes."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+    src = CSRC / "native" / "torch_calls.cpp"
+    out = PKG_DIR / "_native.so"
+    tmp = out.with_suffix(".so.tmp")
+    rocm = Path(_hipcc()).resolve().parent.parent
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-I{INCLUDE}",
+           *(f"-isystem{p}" for p in cpp_extension.include_paths()), f"-isystem{rocm}/include",
+           f"-I{sysconfig.get_paths()['include']}", str(src),
+           *(f"-L{p}" for p in cpp_extension.library_paths()),
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-o", str(tmp)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for {src.name}:\n{' '.join(cmd)}\n{proc.stderr}")
+    os.replace(tmp, out)
+    return out
+
+
 def sources() -> list[Path]:
     return sorted(CSRC.glob("*.hip"))
 
@@ -81,8 +104,10 @@ def build(verbose: bool = True) -> Path:
     if not srcs:
         raise RuntimeError(f"no HIP sources under {CSRC}")
     workers = max(1, min(len(srcs), os.cpu_count() or 1, 8))
-    with concurrent.futures.ThreadPoolExecutor(max_workers=workers) as ex:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=workers + 1) as ex:
+        native = ex.submit(_build_native)
         objs = list(ex.map(lambda s: _compile(s, hipcc), srcs))
+        native.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-fno-gpu-rdc",
            *map(str, objs), "-o", str(tmp)]

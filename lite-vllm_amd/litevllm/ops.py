@@ -4,6 +4,12 @@ Each wrapper checks shapes, dtypes and devices on the host, passes raw
 pointers plus the current HIP stream to liblitevllm_hip.so, and raises
 ``RuntimeError`` with the library's message on failure.  Inputs must be
 tensors on a ROCm ("cuda") device: there is no CPU path behind these calls.
+
+The per-layer wrappers first offer the call to ``litevllm._native`` (csrc/
+native/torch_calls.cpp), which makes the same checks and the same call in
+native code and returns None, having done nothing, where a check fails or the
+scratch buffer is still to be made; the code here then names the fault or
+makes the buffer.
 """
 
 from __future__ import annotations
@@ -59,6 +65,25 @@ def _check_int(name: str, t: torch.Tensor, dtype: torch.dtype, dim: int) -> None
                            f"got {t.dtype} {tuple(t.shape)} contiguous={t.is_contiguous()}")
 
 
+_native_module = None
+
+
+def _native():
+    """The native call module, bound to the loaded library on first use."""
+    global _native_module
+    if _native_module is None:
+        lib = _hip.load()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise RuntimeError("litevllm/_native.so is not built or does not load; build it with "
+                               "`python -m litevllm._build`") from e
+        module.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+                     for name in _hip.SIGNATURES}, _workspaces)
+        _native_module = module
+    return _native_module
+
+
 # ---------------------------------------------------------------------------
 # Device-side index errors
 # ---------------------------------------------------------------------------
@@ -106,6 +131,8 @@ def kv_scatter(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tensor,
     key/value: [T, Hkv, D] (token stride free, heads contiguous);
     caches: contiguous [N, bs, Hkv, D]; slot_mapping: int64 [T].
     """
+    if (_native_module or _native()).kv_scatter(key, value, key_cache, value_cache, slot_mapping):
+        return
     dev = key_cache.device
     for n, t in (("key", key), ("value", value), ("key_cache", key_cache),
                  ("value_cache", value_cache), ("slot_mapping", slot_mapping)):
@@ -314,6 +341,11 @@ def paged_attention(query: torch.Tensor, key_cache: torch.Tensor, value_cache: t
     selects lv_paged_attention_prefix: the decode rows' shared prefixes are
     read once per group; ``prefix_workspace`` is its scratch as above.
     """
+    done = (_native_module or _native()).paged_attention(
+        query, key_cache, value_cache, block_tables, context_lens, num_kv_heads, scale, cu_seqlens,
+        num_decodes, max_query_len, out, workspace, prefix, prefix_workspace)
+    if done is not None:
+        return done
     dev = key_cache.device
     for n, t in (("query", query), ("key_cache", key_cache), ("value_cache", value_cache),
                  ("block_tables", block_tables), ("context_lens", context_lens),
@@ -485,6 +517,9 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor,
     (uint8, >= lv_sample_workspace_size bytes) replaces the per-stream
     scratch buffer when given.
     """
+    done = (_native_module or _native()).sample(logits, temperature, uniform, out, workspace)
+    if done is not None:
+        return done
     dev = logits.device
     for n, t in (("logits", logits), ("temperature", temperature), ("uniform", uniform),
                  ("out", out)):
@@ -544,6 +579,9 @@ def add_rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float,
     Reference: litevllm/models/llama.py:24-27 (RMSNorm) and the residual adds
     of the decoder layer (models/qwen3.py:131-140).  x/residual/out: [T, hidden].
     """
+    done = (_native_module or _native()).add_rms_norm(x, weight, eps, residual, out)
+    if done is not None:
+        return done
     dev = x.device
     for n, t in (("x", x), ("weight", weight), ("residual", residual), ("out", out)):
         _require_device(n, t, dev)
@@ -583,6 +621,11 @@ def qk_norm_rope_cache(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, hea
     Reference: models/qwen3.py:75-84, layers/rotary_emb.py:92-117,
     layers/attention.py:79-84.
     """
+    done = (_native_module or _native()).qk_norm_rope_cache(
+        qkv, num_heads, num_kv_heads, head_dim, cos_cache, sin_cache, positions, slot_mapping,
+        key_cache, value_cache, q_norm_weight, k_norm_weight, eps, q_out)
+    if done is not None:
+        return done
     dev = qkv.device
     for n, t in (("qkv", qkv), ("cos_cache", cos_cache), ("sin_cache", sin_cache),
                  ("positions", positions), ("slot_mapping", slot_mapping),
@@ -628,6 +671,9 @@ def silu_mul(gate_up: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch
 
     Reference: models/llama.py:37-38.
     """
+    done = (_native_module or _native()).silu_mul(gate_up, out)
+    if done is not None:
+        return done
     dev = gate_up.device
     _require_device("gate_up", gate_up, dev)
     _require_device("out", out, dev)
@@ -677,6 +723,9 @@ def linear(x: torch.Tensor, weight: torch.Tensor, activation: Optional[str] = No
     Reference: layers/linear.py:15-65 (ColumnParallelLinear /
     RowParallelLinear = nn.Linear), models/llama.py:38.
     """
+    done = (_native_module or _native()).linear(x, weight, _ACTIVATIONS.get(activation), out)
+    if done is not None:
+        return done
     dev = x.device
     for name, t in (("x", x), ("weight", weight), ("out", out)):
         _require_device(name, t, dev)
