@@ -532,15 +532,25 @@ struct ChunkArgs {
 // barrier depends only on (unit, its item), never on the team or the lane,
 // and teams that share a workgroup run the same item, so all wavefronts of
 // the workgroup meet the same barriers.
-template <typename T, int D, int G, int BS, int W, int BPW, bool PFX>
+//
+// HK = 2 (chunks that leave the chip idle): the workgroup has half as many
+// rows, and wavefronts w and w + W / 2 share 32 of them, taking the first and
+// the second 32 keys of every 64-key tile; the second hands its O, maximum
+// and sum over through LDS at the end (in the tiles, and xml).  Twice the
+// workgroups, each with half the work per tile.
+template <typename T, int D, int G, int BS, int W, int BPW, bool PFX, int HK>
 __device__ __forceinline__ void chunk_mfma_body(const ChunkArgs<T>& A, int unit, int kvh_sel,
                                                 int tid, uint16_t* Ks0, uint16_t* Ks1,
-                                                uint16_t* Vs0, uint16_t* Vs1) {
+                                                uint16_t* Vs0, uint16_t* Vs1,
+                                                float2* xml = nullptr) {
+  static_assert(HK == 1 || (HK == 2 && !PFX && W == 4 && BPW == 1), "split tiles");
   using M = Mfma32<T>;
   using v8 = typename M::v8;
   using L = ChunkLds<D, W * BPW>;
   constexpr int kThreads = 64 * W;
-  constexpr int QT = 32 * W / G;       // query tokens per workgroup
+  constexpr int RW = W / HK;           // wavefronts with rows of their own
+  constexpr int QT = 32 * RW / G;      // query tokens per workgroup
+  constexpr int KB = 2 / HK;           // 32-key halves of a sub-tile per wavefront
   constexpr int KT = 16 * W * BPW;     // keys per LDS tile
   constexpr int NSUB = KT / 64;        // 64-key sub-tiles per LDS tile
   static_assert(NSUB == 1 || NSUB == 2, "one or two 64-key sub-tiles");
@@ -617,7 +627,8 @@ __device__ __forceinline__ void chunk_mfma_body(const ChunkArgs<T>& A, int unit,
   const int32_t* __restrict__ bt = A.block_tables + (int64_t)seq * max_blocks;
 
   // This lane's query row (the B-operand column of K Q^T).
-  const int row = 32 * wave + lr;
+  const int row = 32 * (HK == 1 ? wave : wave % RW) + lr;
+  const int kh = HK == 1 ? 0 : wave / RW;   // HK = 2: this wavefront's half of each tile
   const int qtok = qt0 + row % QT;
   const int qg = row / QT;
   const int qpos = PFX ? pos0 : pos0 + qtok;
@@ -736,8 +747,9 @@ __device__ __forceinline__ void chunk_mfma_body(const ChunkArgs<T>& A, int unit,
     auto kread = [&](int j) __attribute__((always_inline)) {
       return *reinterpret_cast<const uint4*>(kb_lds + 32 * (j >> 3) * D + kx[j & 7]);
     };
+    kb_lds += 32 * kh * D;
     static_assert(QSTEPS == 8 || QSTEPS == 4, "head_dim 128 or 64");
-    constexpr int NJ = 2 * QSTEPS;
+    constexpr int NJ = KB * QSTEPS;
     uint4 ka[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) ka[j] = kread((j / QSTEPS) * 8 + j % QSTEPS);
@@ -756,9 +768,9 @@ __device__ __forceinline__ void chunk_mfma_body(const ChunkArgs<T>& A, int unit,
   const int lim = min(qpos, kend - 1);   // last key each row may see
   auto mask = [&](auto MaskT, f32x16_t* sv, int k0) {
     if constexpr (decltype(MaskT)::value) {
-      const int d = lim - k0 - 4 * h;
+      const int d = lim - k0 - 32 * kh - 4 * h;
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
         for (int i = 0; i < 16; ++i)
           if (32 * kb + 8 * (i >> 2) + (i & 3) > d) sv[kb][i] = kNegBig;
@@ -771,22 +783,25 @@ __device__ __forceinline__ void chunk_mfma_body(const ChunkArgs<T>& A, int unit,
   auto soft = [&](const f32x16_t* sv, uint32_t (*pw)[8]) {
     float mx = kNegBig;
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sv[kb][i]);
     mx = xor32_max(mx) * scale_log2;
     float alpha = 1.0f;
-    if (mx > m_run + 8.0f) {
+    // HK = 2: while every key of a row has been masked in this wavefront's
+    // halves, m_run stays kNegBig and the weights are 0
+    if (mx > m_run + 8.0f && (HK == 1 || mx > kNegBig * 0.01f)) {
       alpha = fast_exp2(m_run - mx);
       m_run = mx;
     }
+    const float m_ref = HK == 2 && m_run == kNegBig ? 0.0f : m_run;
     float psum = 0.0f;
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
       for (int i = 0; i < 16; i += 2) {
-        const float p0 = fast_exp2(fmaf(sv[kb][i], scale_log2, -m_run));
-        const float p1 = fast_exp2(fmaf(sv[kb][i + 1], scale_log2, -m_run));
+        const float p0 = fast_exp2(fmaf(sv[kb][i], scale_log2, -m_ref));
+        const float p1 = fast_exp2(fmaf(sv[kb][i + 1], scale_log2, -m_ref));
         psum += p0 + p1;
         pw[kb][i >> 1] = M::pack2(p0, p1);
       }
@@ -804,8 +819,9 @@ __device__ __forceinline__ void chunk_mfma_body(const ChunkArgs<T>& A, int unit,
   // O^T += V^T P^T over one 64-key sub-tile, four 16-key steps; each step's
   // transpose reads are issued together ahead of its MFMAs.
   auto pv = [&](const uint16_t* vb_lds, const uint32_t (*pw)[8]) {
+    vb_lds += 32 * kh * D;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int t = 0; t < 2 * KB; ++t) {
       const uint32_t* pp = &pw[t >> 1][4 * (t & 1)];
       const v8 pb = __builtin_bit_cast(v8, make_uint4(pp[0], pp[1], pp[2], pp[3]));
       i16x4_t lo[DBLK], hi[DBLK];
@@ -892,6 +908,32 @@ __device__ __forceinline__ void chunk_mfma_body(const ChunkArgs<T>& A, int unit,
   // Row sum over both halves of the wavefront, then write this lane's
   // query row: O^T slot i of block b is dim 32 b + 8 (i / 4) + 4 h + i % 4.
   l_run = xor32_sum(l_run);
+  if constexpr (HK == 2) {
+    // (past the last step's barrier nobody reads the tiles)
+    uint16_t* const tiles[4] = {Ks0, Ks1, Vs0, Vs1};
+    constexpr int RT = 64 * RW;          // threads with rows of their own
+    static_assert(2 * L::TILE >= 4 * RT * 16 && DBLK <= 4, "O exchange fits the tiles");
+    const int rt = tid % RT;
+    if (kh == 1) {
+#pragma unroll
+      for (int b = 0; b < DBLK; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          reinterpret_cast<float*>(tiles[b])[i * RT + rt] = o[b][i];
+      xml[rt] = make_float2(m_run, l_run);
+    }
+    __syncthreads();
+    if (kh == 1) return;
+    const float2 other = xml[rt];
+    const float mx = fmaxf(m_run, other.x);
+    const float f0 = fast_exp2(m_run - mx), f1 = fast_exp2(other.x - mx);
+    l_run = l_run * f0 + other.y * f1;
+#pragma unroll
+    for (int b = 0; b < DBLK; ++b)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        o[b][i] = o[b][i] * f0 + reinterpret_cast<const float*>(tiles[b])[i * RT + rt] * f1;
+  }
   if (qtok >= qlen || !qrow_ok) return;
   const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
   if constexpr (PFX) {
@@ -953,7 +995,7 @@ __device__ __forceinline__ int chunk_rank_pick(const ChunkArgs<T>& a, int grp, i
 
 // Prefill chunks (PFX = false) or the shared-prefix pass as a launch of its
 // own (PFX = true: workgroup = (item, kv head)).
-template <typename T, int D, int G, int BS, int W, int BPW, bool PFX>
+template <typename T, int D, int G, int BS, int W, int BPW, bool PFX, int HK>
 __global__ __launch_bounds__(64 * W, PFX ? 1 : 8 / (W * BPW)) void attn_chunk_mfma_kernel(
     ChunkArgs<T> a) {
   using L = ChunkLds<D, W * BPW>;
@@ -963,15 +1005,16 @@ __global__ __launch_bounds__(64 * W, PFX ? 1 : 8 / (W * BPW)) void attn_chunk_mf
   __shared__ __align__(16) uint16_t Ks0[L::TILE], Ks1[L::TILE], Vs0[L::TILE], Vs1[L::TILE];
   const int wg = (int)blockIdx.x;
   if constexpr (PFX) {
-    chunk_mfma_body<T, D, G, BS, W, BPW, true>(a, wg / a.num_kv_heads, wg % a.num_kv_heads,
-                                               (int)threadIdx.x, Ks0, Ks1, Vs0, Vs1);
+    chunk_mfma_body<T, D, G, BS, W, BPW, true, 1>(a, wg / a.num_kv_heads, wg % a.num_kv_heads,
+                                                  (int)threadIdx.x, Ks0, Ks1, Vs0, Vs1);
   } else {
     __shared__ int s_ctx[kChunkRankMax];
     __shared__ int s_pick;
     const int grp = (wg / kXcds / a.nq_tiles) * kXcds + wg % kXcds;
     const int pick = chunk_rank_pick(a, grp, s_ctx, &s_pick);
-    chunk_mfma_body<T, D, G, BS, W, BPW, false>(a, wg, pick, (int)threadIdx.x, Ks0, Ks1, Vs0,
-                                                Vs1);
+    __shared__ float2 s_ml[HK == 2 ? 32 * W : 1];
+    chunk_mfma_body<T, D, G, BS, W, BPW, false, HK>(a, wg, pick, (int)threadIdx.x, Ks0, Ks1, Vs0,
+                                                    Vs1, s_ml);
   }
 }
 
@@ -1840,7 +1883,7 @@ static void launch_persistent(const void* q, int64_t q_stride, const void* kc, c
       const ChunkArgs<T> ca{(const T*)q, q_stride, (const T*)kc, (const T*)vc, num_kv_heads,
                             num_cache_blocks, bt, max_blocks, nullptr, ctx, 0, 1, num_seqs,
                             scale_log2, (T*)out, out_stride, pfx};
-      hipLaunchKernelGGL((attn_chunk_mfma_kernel<T, D, G, 16, 4, 1, true>),
+      hipLaunchKernelGGL((attn_chunk_mfma_kernel<T, D, G, 16, 4, 1, true, 1>),
                          dim3((unsigned)(pfx.max_items * num_kv_heads)), dim3(256), 0, st, ca);
     }
   }
@@ -1962,26 +2005,38 @@ static int dispatch(lv_dtype dt, int D, int G, int BS, const LaunchArgs& a, cons
   }
 }
 
-template <typename T, int D, int G, int W, int BPW>
-static void launch_chunk_kernel_w(const LaunchArgs& a, const int32_t* cu, int seq_begin,
-                                  int n_seqs, int max_query_len) {
-  constexpr int QT = 32 * W / G;
-  const int nq = (max_query_len + QT - 1) / QT;
-  const int groups = a.num_kv_heads * n_seqs;
+template <typename T, int D, int G, int HK>
+static void launch_chunk_kernel_h(const LaunchArgs& a, const int32_t* cu, int seq_begin,
+                                  int groups, int nq) {
   const int64_t wgs = (int64_t)((groups + kXcds - 1) / kXcds) * kXcds * nq;
   const ChunkArgs<T> ca{(const T*)a.q, a.q_stride, (const T*)a.kc, (const T*)a.vc,
                         a.num_kv_heads, a.num_cache_blocks, a.bt, a.max_blocks, cu, a.ctx,
                         seq_begin, nq, groups, a.scale_log2, (T*)a.out, a.out_stride,
                         PrefixArgs{}};
-  hipLaunchKernelGGL((attn_chunk_mfma_kernel<T, D, G, 16, W, BPW, false>), dim3((unsigned)wgs),
-                     dim3(64 * W), 0, a.st, ca);
+  hipLaunchKernelGGL((attn_chunk_mfma_kernel<T, D, G, 16, 4, 1, false, HK>), dim3((unsigned)wgs),
+                     dim3(256), 0, a.st, ca);
 }
 
-// Chunk workgroups: 4 wavefronts, 64-key tiles, two workgroups per CU.
+// Chunk workgroups: 4 wavefronts, 64-key tiles, two workgroups per CU, 128
+// (query token, head) rows or, split tiles, 64.
 template <typename T, int D, int G>
 static void launch_chunk_kernel(const LaunchArgs& a, const int32_t* cu, int seq_begin, int n_seqs,
                                 int max_query_len) {
-  launch_chunk_kernel_w<T, D, G, 4, 1>(a, cu, seq_begin, n_seqs, max_query_len);
+  const int groups = a.num_kv_heads * n_seqs;
+  const int nq = (max_query_len + 128 / G - 1) / (128 / G);
+  // Split tiles while 128-row workgroups would leave half the slots (two per
+  // CU) empty: 64 rows each, every wavefront with half the dependent chain
+  // (K Q^T, softmax, P V) per tile.  Calls as graph replays, 128-row / split
+  // (16 / 8 heads, D = 128): one prompt of 777 tokens (104 workgroups) 21.6 /
+  // 16.8 us, of 2000 (256) 43.3 / 35.5, 6 chunks of 512 at up to 3000 (384)
+  // 76.6 / 68.9; 8 chunks (512) 87.3 / 87.4, 15 chunks (960) 146 / 157.
+  // Four tiles in flight, or 128-key tiles over eight wavefronts, were slower
+  // but for a few workgroups on long contexts.
+  if ((int64_t)groups * nq * 2 <= 3 * (int64_t)device_cu_count())
+    launch_chunk_kernel_h<T, D, G, 2>(a, cu, seq_begin, groups,
+                                      (max_query_len + 64 / G - 1) / (64 / G));
+  else
+    launch_chunk_kernel_h<T, D, G, 1>(a, cu, seq_begin, groups, nq);
 }
 
 template <typename T, int D>

@@ -209,6 +209,49 @@ def test_decode_matrix_cores_one_rounding(device, dtype, heads, kind):
             assert (err <= bound).all(), (r, h, n, float((err / bound).max()))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads", [(16, 8, 128), (4, 2, 64), (16, 2, 128), (8, 8, 64)])
+@pytest.mark.parametrize("lens", [[(1, 0), (2, 700)], [(31, 33), (32, 0), (33, 31)],
+                                  [(63, 1), (64, 64), (65, 0), (129, 900)], [(5, 4200)],
+                                  "full"])
+def test_chunks_of_few_workgroups(device, dtype, heads, lens):
+    """Chunks whose grid leaves the chip idle run on split key tiles (two
+    wavefronts share 32 rows, 32 keys of each tile apiece), fuller grids on
+    whole ones: lengths around a tile, rows with all keys in the first half of
+    a tile, more than 64 tiles, NaN past the context.  Weights and outputs
+    are rounded to 16 bits once each: 1.5 units in the last place of the
+    largest |value| a row can see, and 2^-8 (2^-11) relative L2."""
+    H, Hkv, D = heads
+    if lens == "full":       # as many 128-row workgroups as take the whole tiles
+        n = 400 // Hkv
+        lens = [(17 + i % 40, (i * 37) % 90) for i in range(n)]
+    _say(f"chunks {dtype} {heads} {lens[:4]}")
+    g = torch.Generator().manual_seed(len(lens))
+    nblk = [-(-(q + o) // 16) for q, o in lens]
+    pool = sum(nblk) + 1
+    perm = (torch.randperm(pool - 1, generator=g) + 1).to(torch.int32)
+    bt, at = torch.zeros(len(lens), max(nblk), dtype=torch.int32), 0
+    kc, vc = (torch.randn(pool, 16, Hkv, D, generator=g).to(dtype) for _ in range(2))
+    for i, (n, (q, o)) in enumerate(zip(nblk, lens)):
+        bt[i, :n] = perm[at:at + n]
+        at += n
+        if (q + o) % 16:
+            kc[bt[i, n - 1], (q + o) % 16:] = float("nan")
+            vc[bt[i, n - 1], (q + o) % 16:] = float("nan")
+    cu = torch.tensor([0] + [q for q, _ in lens]).cumsum(0).to(torch.int32)
+    ctx = torch.tensor([q + o for q, o in lens], dtype=torch.int32)
+    query = torch.randn(int(cu[-1]), H, D, generator=g).to(dtype)
+    scale = D ** -0.5
+    got = ops.paged_attention(*(t.to(device) for t in (query, kc, vc, bt, ctx)), scale=scale,
+                              cu_seqlens=cu.to(device), num_decodes=0,
+                              max_query_len=max(q for q, _ in lens)).float().cpu()
+    ref = oatt.mixed_attention(query, kc, vc, bt, cu, ctx, scale)
+    ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert torch.isfinite(got).all()
+    assert (got - ref).norm() <= ulp * ref.norm()
+    assert (got - ref).abs().max() <= 1.5 * ulp * float(vc.nan_to_num(0).abs().max())
+
+
 @pytest.mark.parametrize("rows,heads", [(1, (16, 8, 128)), (3, (16, 2, 128)), (7, (8, 8, 64)),
                                         (128, (16, 8, 128)), (129, (16, 8, 128))])
 def test_decode_few_rows_of_many_pieces(device, rows, heads):
