@@ -362,33 +362,52 @@ __device__ __forceinline__ int walked_blocks(const int32_t* __restrict__ ctx,
   return skip ? nb - min(max(skip[i], 0), min(nb, kPrefixMaxBlocks)) : nb;
 }
 
+// Inclusive sum over the lanes up to this one.
+__device__ __forceinline__ int32_t wave_scan(int32_t v, int lane) {
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int32_t u = __shfl_up(v, d);
+    if (lane >= d) v += u;
+  }
+  return v;
+}
+
+// Every thread takes a run of rows, wavefronts scan their threads' sums by
+// lane shuffles, and one exchange of the wavefronts' totals through LDS
+// (s_part) makes the offsets: two barriers.  (A Hillis-Steele scan over all
+// threads in LDS took 2 log2(threads) of them, on the critical path of every
+// decode call before its first K / V load.)  Runs longer than kRun rows read
+// the context lengths a second time.
 template <int BS>
 __device__ void scan_block_counts(const int32_t* __restrict__ ctx,
                                   const int32_t* __restrict__ skip, int n, int max_tokens,
                                   int32_t* s_off, int32_t* s_part, int32_t* s_skip) {
+  constexpr int kRun = 2;
   const int t = threadIdx.x, nt = blockDim.x;
+  const int lane = t & 63, wave = t >> 6, waves = nt >> 6;
   const int per = (n + nt - 1) / nt;
   const int lo = min(n, t * per), hi = min(n, lo + per);
-  int32_t sum = 0;
+  int32_t w[kRun] = {0, 0}, sum = 0;
   for (int i = lo; i < hi; ++i) {
-    const int w = walked_blocks<BS>(ctx, skip, i, max_tokens);
-    if (skip) s_skip[i] = (min(max(ctx[i], 0), max_tokens) + BS - 1) / BS - w;
-    sum += w;
+    const int v = walked_blocks<BS>(ctx, skip, i, max_tokens);
+    if (skip) s_skip[i] = (min(max(ctx[i], 0), max_tokens) + BS - 1) / BS - v;
+    if (i == lo) w[0] = v;
+    if (i == lo + 1) w[1] = v;
+    sum += v;
   }
-  s_part[t] = sum;
+  const int32_t incl = wave_scan(sum, lane);
+  if (lane == 63) s_part[wave] = incl;
   __syncthreads();
-  for (int d = 1; d < nt; d <<= 1) {
-    const int32_t v = (t >= d) ? s_part[t - d] : 0;
-    __syncthreads();
-    s_part[t] += v;
-    __syncthreads();
+  int32_t run = incl - sum;
+  for (int v = 0; v < waves; ++v) {
+    const int32_t p = s_part[v];
+    if (v < wave) run += p;
   }
-  int32_t run = (t == 0) ? 0 : s_part[t - 1];
+  if (t == nt - 1) s_off[n] = run + sum;
   for (int i = lo; i < hi; ++i) {
     s_off[i] = run;
-    run += walked_blocks<BS>(ctx, skip, i, max_tokens);
+    run += i == lo ? w[0] : i == lo + 1 ? w[1] : walked_blocks<BS>(ctx, skip, i, max_tokens);
   }
-  if (t == nt - 1) s_off[n] = s_part[nt - 1];
   __syncthreads();
 }
 
@@ -1031,7 +1050,7 @@ __global__ __launch_bounds__(kPersistMaxWaves * 64) void attn_decode_persistent_
   // LDS: s_off [num_seqs + 1], then (shared prefixes only) s_skip [num_seqs]
   extern __shared__ int32_t s_off[];
   int32_t* s_skip = s_off + num_seqs + 1;
-  __shared__ int32_t s_part[kPersistMaxWaves * 64];
+  __shared__ int32_t s_part[kPersistMaxWaves];
   const int max_tokens = max_blocks * BS;
   const bool has_pfx = pfx.blocks != nullptr;
   scan_block_counts<BS>(ctx, pfx.blocks, num_seqs, max_tokens, s_off, s_part, s_skip);
@@ -1308,7 +1327,7 @@ __global__ __launch_bounds__(kPersistMaxWaves * 64) void attn_decode_mfma_kernel
   // LDS: the wavefronts' stages, s_off [num_seqs + 1], then (shared prefixes
   // only) s_skip [num_seqs]
   extern __shared__ __align__(16) unsigned char s_dyn[];
-  __shared__ int32_t s_part[kPersistMaxWaves * 64];
+  __shared__ int32_t s_part[kPersistMaxWaves];
   int32_t* s_off = reinterpret_cast<int32_t*>(s_dyn + num_kv_heads * 2 * B::STAGE);
   int32_t* s_skip = s_off + num_seqs + 1;
   const int max_tokens = max_blocks * BS;
