@@ -401,6 +401,14 @@ int lv_linear(const void* x_dev, int64_t x_stride_t, const void* weight_dev,
               int64_t weight_stride_n, void* y_dev, int64_t y_stride_t, int64_t m, int64_t n,
               int64_t k, int32_t activation, lv_dtype dtype, void* stream);
 
+/* The plain form in fp32 (products and sums in fp32), for small models and
+ * batches; the same reference code.  k must be a multiple of 4 and x / weight
+ * rows 16-byte aligned (else LV_ERR_INVALID); any m and n.  Large products
+ * belong to the library GEMM. */
+int lv_linear_f32(const float* x_dev, int64_t x_stride_t, const float* weight_dev,
+                  int64_t weight_stride_n, float* y_dev, int64_t y_stride_t, int64_t m, int64_t n,
+                  int64_t k, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -39,6 +39,7 @@ struct Api {
   decltype(&lv_qk_norm_rope_cache) qk_norm_rope_cache;
   decltype(&lv_silu_mul) silu_mul;
   decltype(&lv_linear) linear;
+  decltype(&lv_linear_f32) linear_f32;
 };
 Api api{};
 
@@ -46,7 +47,7 @@ constexpr const char* kNames[] = {
     "lv_last_error", "lv_kv_scatter", "lv_paged_attention_workspace_size", "lv_paged_attention",
     "lv_paged_attention_prefix_workspace_size", "lv_paged_attention_prefix",
     "lv_sample_workspace_size", "lv_sample", "lv_add_rms_norm", "lv_qk_norm_rope_cache",
-    "lv_silu_mul", "lv_linear"};
+    "lv_silu_mul", "lv_linear", "lv_linear_f32"};
 constexpr size_t kNumNames = sizeof(kNames) / sizeof(kNames[0]);
 static_assert(sizeof(Api) == kNumNames * sizeof(void*), "one pointer per name");
 
@@ -418,6 +419,29 @@ FAST(linear, 4) {
   return done(rc, "lv_linear", &out);
 }
 
+// (x, weight, out) -> out.  Rows off 16-byte boundaries are not plain either:
+// the layer that asks has a library product to fall back on.
+FAST(linear_f32, 3) {
+  const at::Tensor *x = A.tensor(0), *w = A.tensor(1), *given = A.maybe(2);
+  if (!A.ok || !x->is_cuda() || x->scalar_type() != at::kFloat || x->dim() != 2 || w->dim() != 2)
+    NOT_PLAIN();
+  const at::Device dev = x->device();
+  const int64_t M = x->size(0), K = x->size(1), N = w->size(0);
+  if (M == 0 || !on(x, dev) || !on(w, dev) || !on(given, dev) || !is_rows(*x, K, at::kFloat) ||
+      !is_rows(*w, K, at::kFloat) || w->size(1) != K || K == 0 || K % 4 || N == 0 ||
+      x->stride(0) % 4 || w->stride(0) % 4 || ((uintptr_t)ptr(x) | (uintptr_t)ptr(w)) % 16 ||
+      (given && (!is_rows(*given, N, at::kFloat) || given->size(0) != M)))
+    NOT_PLAIN();
+  const at::Tensor out = given ? *given : empty({M, N}, *x);
+  void* st = stream_of(dev);
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = api.linear_f32((const float*)ptr(x), x->stride(0), (const float*)ptr(w), w->stride(0),
+                      (float*)out.data_ptr(), out.stride(0), M, N, K, st);
+  Py_END_ALLOW_THREADS
+  return done(rc, "lv_linear_f32", &out);
+}
+
 #define METHOD(NAME) {#NAME, (PyCFunction)(void (*)(void))NAME, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {{"bind", bind, METH_VARARGS, nullptr},
                          METHOD(kv_scatter),
@@ -427,6 +451,7 @@ PyMethodDef methods[] = {{"bind", bind, METH_VARARGS, nullptr},
                          METHOD(qk_norm_rope_cache),
                          METHOD(silu_mul),
                          METHOD(linear),
+                         METHOD(linear_f32),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods};
 

@@ -119,6 +119,11 @@ SIGNATURES: dict[str, tuple] = {
         _c_i64, _c_i64, _c_i64,        # m, n, k
         _c_i32, ctypes.c_int, _c_p,    # activation, dtype, stream
     ]),
+    "lv_linear_f32": (ctypes.c_int, [
+        _c_p, _c_i64, _c_p, _c_i64,    # x, x_stride, weight, weight_stride
+        _c_p, _c_i64,                  # y, y_stride
+        _c_i64, _c_i64, _c_i64, _c_p,  # m, n, k, stream
+    ]),
 }
 
 _lock = threading.Lock()

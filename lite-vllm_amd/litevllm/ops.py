@@ -747,3 +747,41 @@ def linear(x: torch.Tensor, weight: torch.Tensor, activation: Optional[str] = No
                        _stream(dev))
     _hip.check(rc, "lv_linear")
     return out
+
+
+def linear_f32(x: torch.Tensor, weight: torch.Tensor,
+               out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """y = x @ weight.T in fp32 on the MFMA kernel for small products (K a
+    multiple of 4, rows 16-byte aligned).
+
+    Reference: layers/linear.py:15-65.
+    """
+    done = (_native_module or _native()).linear_f32(x, weight, out)
+    if done is not None:
+        return done
+    dev = x.device
+    for name, t in (("x", x), ("weight", weight), ("out", out)):
+        _require_device(name, t, dev)
+    M, K = x.shape
+    N = weight.shape[0]
+    _check_rows("x", x, K, torch.float32)
+    _check_rows("weight", weight, K, torch.float32)
+    if weight.shape[1] != K:
+        raise RuntimeError(f"weight {tuple(weight.shape)} does not match x {tuple(x.shape)}")
+    if out is None:
+        out = torch.empty((M, N), dtype=x.dtype, device=dev)
+    _check_rows("out", out, N, x.dtype)
+    if out.shape[0] != M:
+        raise RuntimeError("`out` rows != x rows")
+    if M == 0:
+        return out
+    rc = _hip.load().lv_linear_f32(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0),
+                                   _ptr(out), out.stride(0), M, N, K, _stream(dev))
+    _hip.check(rc, "lv_linear_f32")
+    return out
+
+
+def linear_f32_if_plain(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
+    """linear_f32, or None for operands it has no kernel for (for callers with
+    another product to fall back on)."""
+    return (_native_module or _native()).linear_f32(x, weight, None)

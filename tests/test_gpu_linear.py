@@ -117,3 +117,40 @@ def test_silu_mul_epilogue_equals_plain_then_silu_mul(dtype, m, cfg, monkeypatch
     tol = (4 * _ulp(want, dtype) + 4 * _ulp(up, dtype) * (gate.abs() + 1)
            + 2 * _ulp(gate, dtype) * up.abs() + 1e-5)
     assert (err <= tol).all(), err.max()
+
+
+@pytest.mark.parametrize("m", [1, 31, 32, 33, 320])
+@pytest.mark.parametrize("nk", [(512, 256), (33, 4), (31, 36), (256, 688), (1, 60), (100, 2052)])
+def test_linear_f32_matches_fp64(m, nk):
+    """fp32 products and sums: k 2^-24 of sum |x w| bounds any order of the
+    sum.  Edges of the 32 x 32 tiles, a last half chunk (k % 8 == 4), strided
+    rows; nothing is written past the output's columns."""
+    n, k = nk
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k + 4, device="cuda", generator=g)[:, 4:]
+    w = torch.randn(n, k + 8, device="cuda", generator=g)[:, :k]
+    buf = torch.full((m, n + 3), 7.0, device="cuda")
+    y = ops.linear_f32(x, w, out=buf[:, :n])
+    ref = x.double() @ w.double().T
+    bound = (k + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert ((y.double() - ref).abs() <= bound).all()
+    assert (buf[:, n:] == 7.0).all()
+
+
+def test_linear_f32_forms_left_to_the_library():
+    """The layer runs what lv_linear_f32 has no kernel for on the library, and
+    keeps autograd; the op itself refuses such operands."""
+    from litevllm.models.llama import Linear
+    lin = Linear(256, 64, bias=False).cuda()
+    x = torch.randn(9, 257, device="cuda")
+    assert ops.linear_f32_if_plain(x[:, 1:], lin.weight) is None     # rows off 16 bytes
+    with pytest.raises(RuntimeError, match="16-byte aligned"):
+        ops.linear_f32(x[:, 1:], lin.weight.detach())
+    with torch.inference_mode():
+        y = lin(x[:, 1:])
+        z = lin(x[:, :256].contiguous())
+    for got, a in ((y, x[:, 1:]), (z, x[:, :256])):
+        ref = a.double() @ lin.weight.detach().double().T
+        assert (got.double() - ref).norm() <= 1e-6 * ref.norm()
+    lin(x[:, :256].contiguous()).sum().backward()
+    assert lin.weight.grad is not None
