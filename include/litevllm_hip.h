@@ -198,6 +198,16 @@ size_t lv_paged_attention_workspace_size(int32_t num_seqs, int32_t num_decodes,
                                          int32_t max_blocks, int32_t max_query_len,
                                          lv_dtype dtype);
 
+/* lv_paged_attention_workspace_size plus what lets the prefill-chunk rows of
+ * such a call split their keys over more workgroups (few chunks at long
+ * offsets leave most of the GPU idle otherwise).  Optional: with less
+ * workspace the chunk rows run unsplit, with results equal to fp32 rounding. */
+size_t lv_paged_attention_split_workspace_size(int32_t num_seqs, int32_t num_decodes,
+                                               int64_t num_tokens, int32_t num_heads,
+                                               int32_t num_kv_heads, int32_t head_dim,
+                                               int32_t block_size, int32_t max_blocks,
+                                               int32_t max_query_len, lv_dtype dtype);
+
 int lv_paged_attention(const void* query_dev, int64_t q_stride_t,
                        const void* key_cache_dev, const void* value_cache_dev,
                        int64_t num_cache_blocks,

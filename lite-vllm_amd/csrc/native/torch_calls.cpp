@@ -15,6 +15,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -30,6 +31,7 @@ struct Api {
   decltype(&lv_last_error) last_error;
   decltype(&lv_kv_scatter) kv_scatter;
   decltype(&lv_paged_attention_workspace_size) attention_ws;
+  decltype(&lv_paged_attention_split_workspace_size) split_ws;
   decltype(&lv_paged_attention) attention;
   decltype(&lv_paged_attention_prefix_workspace_size) prefix_ws;
   decltype(&lv_paged_attention_prefix) attention_prefix;
@@ -44,7 +46,8 @@ struct Api {
 Api api{};
 
 constexpr const char* kNames[] = {
-    "lv_last_error", "lv_kv_scatter", "lv_paged_attention_workspace_size", "lv_paged_attention",
+    "lv_last_error", "lv_kv_scatter", "lv_paged_attention_workspace_size",
+    "lv_paged_attention_split_workspace_size", "lv_paged_attention",
     "lv_paged_attention_prefix_workspace_size", "lv_paged_attention_prefix",
     "lv_sample_workspace_size", "lv_sample", "lv_add_rms_norm", "lv_qk_norm_rope_cache",
     "lv_silu_mul", "lv_linear", "lv_linear_f32"};
@@ -235,7 +238,7 @@ FAST(paged_attention, 14) {
   if (given && (!is_heads(*given, H, D) || given->size(0) != T ||
                 given->scalar_type() != q->scalar_type()))
     NOT_PLAIN();
-  const size_t ws_bytes = api.attention_ws(B, nd, T, H, D, bs, max_blocks, max_q, dt);
+  size_t ws_bytes = api.attention_ws(B, nd, T, H, D, bs, max_blocks, max_q, dt);
   if (ws && !is_scratch(*ws, ws_bytes)) NOT_PLAIN();
   // shared prefixes: PrefixPlan(blocks, items, members)
   const at::Tensor *pb = nullptr, *pi = nullptr, *pm = nullptr, *pws = nullptr;
@@ -253,8 +256,10 @@ FAST(paged_attention, 14) {
       NOT_PLAIN();
   }
   void* st = stream_of(dev);
-  if (ws_bytes == 0) ws = nullptr;
-  else if (!ws && !(ws = scratch(dev, st, ws_bytes, kind_attn))) NOT_PLAIN();
+  if (!ws && nd < B &&
+      c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None)
+    ws_bytes = api.split_ws(B, nd, T, H, hkv, D, bs, max_blocks, max_q, dt);
+  if (ws_bytes > 0 && !ws && !(ws = scratch(dev, st, ws_bytes, kind_attn))) NOT_PLAIN();
   if (pb && !pws && pws_bytes > 0 && !(pws = scratch(dev, st, pws_bytes, kind_prefix)))
     NOT_PLAIN();
   // held past the GIL's release: another thread may grow the pool's entry

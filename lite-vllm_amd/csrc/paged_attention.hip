@@ -20,6 +20,7 @@
 // workspace and are merged by attn_reduce_kernel.
 #include <stdlib.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include <type_traits>
@@ -528,688 +529,6 @@ __device__ __forceinline__ i16x4_t lds_read_tr16(const uint16_t* p) {
 // Chunk sequences a chunk workgroup ranks by length (more: index order).
 constexpr int kChunkRankMax = 256;
 
-// Arguments of the MFMA attention body (prefill chunks or shared-prefix
-// units).
-template <typename T>
-struct ChunkArgs {
-  const T* __restrict__ q; int64_t q_stride;
-  const T* __restrict__ kc; const T* __restrict__ vc; int num_kv_heads; int64_t num_cache_blocks;
-  const int32_t* __restrict__ block_tables; int max_blocks;
-  const int32_t* __restrict__ cu; const int32_t* __restrict__ ctx; int seq_begin;
-  int nq_tiles, num_groups; float scale_log2; T* __restrict__ out; int64_t out_stride;
-  PrefixArgs pfx;
-};
-
-// PFX = false: prefill chunks (causal, normalised output rows); `unit` is
-// the workgroup id and `kvh_sel` the chunk sequence (index from seq_begin)
-// the caller's longest-first order gives it.  PFX = true: one shared-prefix
-// unit -- `unit` is the work item, `kvh_sel` the kv head: up to QT group
-// members against one 128-key split of the group's prefix (no causal mask;
-// every prefix key precedes every member's query), writing prefix partials.
-// The body runs on one team of W wavefronts (`tid` = thread index in the
-// team) with its own four LDS tiles.  Every early exit before the last
-// barrier depends only on (unit, its item), never on the team or the lane,
-// and teams that share a workgroup run the same item, so all wavefronts of
-// the workgroup meet the same barriers.
-//
-// HK = 2 (chunks that leave the chip idle): the workgroup has half as many
-// rows, and wavefronts w and w + W / 2 share 32 of them, taking the first and
-// the second 32 keys of every 64-key tile; the second hands its O, maximum
-// and sum over through LDS at the end (in the tiles, and xml).  Twice the
-// workgroups, each with half the work per tile.
-template <typename T, int D, int G, int BS, int W, int BPW, bool PFX, int HK>
-__device__ __forceinline__ void chunk_mfma_body(const ChunkArgs<T>& A, int unit, int kvh_sel,
-                                                int tid, uint16_t* Ks0, uint16_t* Ks1,
-                                                uint16_t* Vs0, uint16_t* Vs1,
-                                                float2* xml = nullptr) {
-  static_assert(HK == 1 || (HK == 2 && !PFX && W == 4 && BPW == 1), "split tiles");
-  using M = Mfma32<T>;
-  using v8 = typename M::v8;
-  using L = ChunkLds<D, W * BPW>;
-  constexpr int kThreads = 64 * W;
-  constexpr int RW = W / HK;           // wavefronts with rows of their own
-  constexpr int QT = 32 * RW / G;      // query tokens per workgroup
-  constexpr int KB = 2 / HK;           // 32-key halves of a sub-tile per wavefront
-  constexpr int KT = 16 * W * BPW;     // keys per LDS tile
-  constexpr int NSUB = KT / 64;        // 64-key sub-tiles per LDS tile
-  static_assert(NSUB == 1 || NSUB == 2, "one or two 64-key sub-tiles");
-  constexpr int QSTEPS = D / 16;       // k-steps of K Q^T
-  constexpr int DBLK = D / 32;         // 32-dim blocks of O^T
-  constexpr int CPR = L::CPR;
-  constexpr int RPI = 64 / CPR;        // key rows per wave-wide 1 KiB load
-  constexpr int LPW = BS / RPI;        // loads per wavefront per tile (one block each)
-  static_assert(BS == 16 && (W == 4 || W == 8), "each wavefront stages one 16-token block");
-  const T* __restrict__ q = A.q;
-  const int64_t q_stride = A.q_stride;
-  const T* __restrict__ kc = A.kc;
-  const T* __restrict__ vc = A.vc;
-  const int num_kv_heads = A.num_kv_heads;
-  const int64_t num_cache_blocks = A.num_cache_blocks;
-  const int max_blocks = A.max_blocks;
-  const float scale_log2 = A.scale_log2;
-  const PrefixArgs& pfx = A.pfx;
-
-  // XCD-aware, longest-first order (chunks): workgroups are dispatched
-  // round-robin over the XCDs (id % kXcds) and, on each XCD, in id order as
-  // slots free up.  Workgroup id w serves group g = (w / kXcds / nq) *
-  // kXcds + w % kXcds -- kv head g % Hkv of the (g / Hkv)-th longest chunk
-  // sequence (the caller ranks them) -- and query tile nq - 1 - (w / kXcds)
-  // % nq: all query tiles of one group run on one XCD and share its L2 copy
-  // of the group's K/V, and each XCD starts with the longest tiles, which
-  // shortens the tail of the last wave of workgroups.
-  int kvh, seq, q0, qlen, qt0, pos0, kb0, kend, mbeg = 0, split = 0;
-  if constexpr (PFX) {
-    const int item = unit;
-    kvh = kvh_sel;
-    if (item >= pfx.max_items) return;
-    const int4 it = *reinterpret_cast<const int4*>(pfx.items + 4 * item);
-    // unused item (leader < 0), leaders beyond the decode rows (num_groups),
-    // member slices outside `members` or wider than QT, splits beyond the
-    // partial buffers: skipped
-    if (it.x < 0 || it.x >= A.num_groups || it.w < 0 || it.w >= kPrefixMaxSplits || it.y < 0 ||
-        it.z < 1 || it.z > QT || it.y > pfx.num_members - it.z)
-      return;
-    seq = it.x;                                 // the group leader's block table
-    mbeg = it.y;
-    qlen = it.z;                                // members in this item (<= QT)
-    split = it.w;
-    q0 = 0;
-    qt0 = 0;
-    const int pkeys = min(min(pfx.blocks[seq], max_blocks), kPrefixMaxBlocks) * BS;
-    kb0 = split * kPrefixKeysPerSplit;
-    kend = min(pkeys, kb0 + kPrefixKeysPerSplit);
-    pos0 = 0x3fffffff;                          // queries follow every prefix key
-    if (kb0 >= kend) return;
-  } else {
-    const int wg = unit;
-    const int slot = wg / kXcds;
-    const int grp = (slot / A.nq_tiles) * kXcds + wg % kXcds;
-    if (grp >= A.num_groups) return;
-    kvh = grp % num_kv_heads;
-    seq = A.seq_begin + kvh_sel;
-    q0 = A.cu[seq];
-    qlen = A.cu[seq + 1] - q0;
-    qt0 = (A.nq_tiles - 1 - slot % A.nq_tiles) * QT;
-    if (qt0 >= qlen) return;
-    const int ctxlen = min(A.ctx[seq], max_blocks * BS);
-    pos0 = ctxlen - qlen;                                      // position of chunk row 0
-    kb0 = 0;
-    kend = max(0, min(ctxlen, pos0 + min(qt0 + QT, qlen)));    // keys [0, kend)
-    if (kend <= 0) return;
-  }
-  const int ntiles = (kend - kb0 + KT - 1) / KT;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63;
-  const int lr = lane & 31;        // this lane's query column / key row
-  const int h = lane >> 5;         // half of the wavefront
-  const int64_t tok_stride = (int64_t)num_kv_heads * D;
-  const int32_t* __restrict__ bt = A.block_tables + (int64_t)seq * max_blocks;
-
-  // This lane's query row (the B-operand column of K Q^T).
-  const int row = 32 * (HK == 1 ? wave : wave % RW) + lr;
-  const int kh = HK == 1 ? 0 : wave / RW;   // HK = 2: this wavefront's half of each tile
-  const int qtok = qt0 + row % QT;
-  const int qg = row / QT;
-  const int qpos = PFX ? pos0 : pos0 + qtok;
-  int qrow = PFX ? pfx.members[mbeg + min(qtok, qlen - 1)] : q0 + min(qtok, qlen - 1);
-  bool qrow_ok = true;
-  if constexpr (PFX) {
-    qrow_ok = qrow >= 0 && qrow < A.num_groups;
-    qrow = qrow_ok ? qrow : seq;
-  }
-  v8 qf[QSTEPS];
-  {
-    const T* qp = q + (int64_t)qrow * q_stride + (int64_t)(kvh * G + qg) * D + 8 * h;
-#pragma unroll
-    for (int st = 0; st < QSTEPS; ++st) qf[st] = __builtin_bit_cast(v8, load16(qp + 16 * st));
-  }
-
-  // Staging: wavefront w loads block w of the tile (rows 16w..16w+15) with
-  // LPW wave-wide loads; lane l of load u fills LDS slot l % CPR of row
-  // 16w + RPI u + l / CPR, i.e. the row's chunk (l % CPR) ^ swz(row).
-  int64_t goff[LPW];
-#pragma unroll
-  for (int u = 0; u < LPW; ++u) {
-    const int r = RPI * u + lane / CPR;            // row inside the block
-    const int chunk = (lane % CPR) ^ L::swz(r);        // 16-row blocks keep row & 15
-    goff[u] = (int64_t)r * tok_stride + (int64_t)kvh * D + 8 * chunk;
-  }
-  const int last_blk = (kend - 1) / BS;
-  const int64_t blk_elems = (int64_t)BS * tok_stride;
-  // Chunks: physical ids of this wavefront's blocks (blocks wave + W j of
-  // each tile), 64 tiles at a time: lane l of bids[j] holds tile bid_tb + l,
-  // loaded ahead so staging a tile never waits for a block-table read.  (A
-  // shared-prefix unit has at most two tiles and reads its ids directly.)
-  int bids[BPW];
-  int bid_tb = 0;
-  auto load_bids = [&](int tb) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < BPW; ++j) {
-      const int b = bt[min((kb0 + (tb + lane) * KT) / BS + wave + W * j, last_blk)];
-      const bool bad = b < 0 || b >= num_cache_blocks;   // clamped and reported
-      if (bad) report_device_error(LV_DEVERR_BLOCK_ID);
-      bids[j] = bad ? 0 : b;
-    }
-    bid_tb = tb;
-  };
-  if constexpr (!PFX) load_bids(0);
-  // Wavefront w stages blocks w, w + W, ... (BPW of them) of the tile.
-  auto stage = [&](uint16_t* Kst, uint16_t* Vst, int k0) {
-    const int tile = (k0 - kb0) / KT;
-    if constexpr (!PFX) {
-      if (tile - bid_tb >= 64) load_bids(tile);   // contexts beyond 64 tiles
-    }
-#pragma unroll
-    for (int j = 0; j < BPW; ++j) {
-      const int blk = wave + W * j;
-      int b;
-      if constexpr (PFX) {
-        b = bt[min(k0 / BS + blk, last_blk)];
-        if (b < 0 || b >= num_cache_blocks) {   // clamped and reported
-          report_device_error(LV_DEVERR_BLOCK_ID);
-          b = 0;
-        }
-      } else {
-        b = __builtin_amdgcn_readlane(bids[j], tile - bid_tb);
-      }
-      const T* kp = kc + (int64_t)b * blk_elems;
-      const T* vp = vc + (int64_t)b * blk_elems;
-      uint16_t* kd = Kst + 16 * blk * D;
-      uint16_t* vd = Vst + 16 * blk * D;
-#pragma unroll
-      for (int u = 0; u < LPW; ++u) {
-        load_lds16(kp + goff[u], kd + RPI * u * D);
-        load_lds16(vp + goff[u], vd + RPI * u * D);
-      }
-    }
-  };
-  // Rows at or past kend hold data of the clamped block: zero their V so a
-  // zero probability never meets a NaN (their scores are masked).
-  auto zero_tail = [&](uint16_t* Vst, int k0) {
-    for (int c = tid; c < KT * CPR; c += kThreads)
-      if (k0 + c / CPR >= kend) store16(Vst + (c / CPR) * D + 8 * (c % CPR), make_uint4(0, 0, 0, 0));
-  };
-
-  f32x16_t o[DBLK];
-#pragma unroll
-  for (int b = 0; b < DBLK; ++b)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) o[b][i] = 0.0f;
-  float m_run = kNegBig, l_run = 0.0f;
-
-
-  // Per-lane LDS offsets of the MFMA operands.  Rows 32 kb + lr share
-  // lr's swizzle (it depends on row % 16 only), so the K offset of step st
-  // is kx[st] plus the constant 32 kb D; the V rows 16 t + vrow (+ 8)
-  // likewise share a swizzle across t.
-  int kx[QSTEPS];
-  {
-    const int y = h ^ L::swz(lr);         // (2 st + h) ^ sw == 2 st ^ y
-#pragma unroll
-    for (int st = 0; st < QSTEPS; ++st) kx[st] = lr * D + 8 * ((2 * st) ^ y);
-  }
-  const int vrow = 4 * h + ((lane & 15) >> 2);
-  int voff[DBLK][2];
-#pragma unroll
-  for (int b = 0; b < DBLK; ++b) {
-    const int dim = 32 * b + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-    voff[b][0] = L::at(vrow, dim >> 3) + (dim & 7);
-    voff[b][1] = L::at(vrow + 8, dim >> 3) + (dim & 7);
-  }
-
-  // S^T of one 64-key sub-tile (raw scores, two 32-key halves): 16 MFMAs,
-  // step j = (half j / 8, k-step j % 8), with four K operand reads in
-  // flight.  The order is pinned (read j + 4 goes out right after MFMA j
-  // frees its buffer): left to itself the scheduler, at this register
-  // budget, gives all reads one buffer and waits out each read in turn.
-  auto qk = [&](const uint16_t* kb_lds, f32x16_t* sv) {
-    auto kread = [&](int j) __attribute__((always_inline)) {
-      return *reinterpret_cast<const uint4*>(kb_lds + 32 * (j >> 3) * D + kx[j & 7]);
-    };
-    kb_lds += 32 * kh * D;
-    static_assert(QSTEPS == 8 || QSTEPS == 4, "head_dim 128 or 64");
-    constexpr int NJ = KB * QSTEPS;
-    uint4 ka[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) ka[j] = kread((j / QSTEPS) * 8 + j % QSTEPS);
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      __builtin_amdgcn_sched_barrier(0);
-      const int kb = j / QSTEPS, st = j % QSTEPS;
-      sv[kb] = M::run(__builtin_bit_cast(v8, ka[j & 3]), qf[st], st ? sv[kb] : f32x16_t{});
-      if (j + 4 < NJ) ka[j & 3] = kread(((j + 4) / QSTEPS) * 8 + (j + 4) % QSTEPS);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  // Causal / range mask (MaskT = std::true_type on tiles that may need it;
-  // those run in a loop of their own so the mask is never straight-line code
-  // on the others): slot i of half kb holds key k0 + 32 kb + 8 (i/4) + 4 h + i%4.
-  const int lim = min(qpos, kend - 1);   // last key each row may see
-  auto mask = [&](auto MaskT, f32x16_t* sv, int k0) {
-    if constexpr (decltype(MaskT)::value) {
-      const int d = lim - k0 - 32 * kh - 4 * h;
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (32 * kb + 8 * (i >> 2) + (i & 3) > d) sv[kb][i] = kNegBig;
-    }
-  };
-  // Online softmax in log2 units with a lazily raised maximum: the running
-  // maximum m_run moves only when a row's maximum exceeds it by more than
-  // 2^8 (or on the first tile), so probabilities stay below 256 and the O
-  // rescale is rare.  Returns the factor O must be scaled by (1 = none).
-  auto soft = [&](const f32x16_t* sv, uint32_t (*pw)[8]) {
-    float mx = kNegBig;
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sv[kb][i]);
-    mx = xor32_max(mx) * scale_log2;
-    float alpha = 1.0f;
-    // HK = 2: while every key of a row has been masked in this wavefront's
-    // halves, m_run stays kNegBig and the weights are 0
-    if (mx > m_run + 8.0f && (HK == 1 || mx > kNegBig * 0.01f)) {
-      alpha = fast_exp2(m_run - mx);
-      m_run = mx;
-    }
-    const float m_ref = HK == 2 && m_run == kNegBig ? 0.0f : m_run;
-    float psum = 0.0f;
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int i = 0; i < 16; i += 2) {
-        const float p0 = fast_exp2(fmaf(sv[kb][i], scale_log2, -m_ref));
-        const float p1 = fast_exp2(fmaf(sv[kb][i + 1], scale_log2, -m_ref));
-        psum += p0 + p1;
-        pw[kb][i >> 1] = M::pack2(p0, p1);
-      }
-    l_run = l_run * alpha + psum;
-    return alpha;
-  };
-  auto rescale = [&](float alpha) {
-    if (__ballot(alpha != 1.0f)) {   // uniform branch, rare after the first tile
-#pragma unroll
-      for (int b = 0; b < DBLK; ++b)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o[b][i] *= alpha;
-    }
-  };
-  // O^T += V^T P^T over one 64-key sub-tile, four 16-key steps; each step's
-  // transpose reads are issued together ahead of its MFMAs.
-  auto pv = [&](const uint16_t* vb_lds, const uint32_t (*pw)[8]) {
-    vb_lds += 32 * kh * D;
-#pragma unroll
-    for (int t = 0; t < 2 * KB; ++t) {
-      const uint32_t* pp = &pw[t >> 1][4 * (t & 1)];
-      const v8 pb = __builtin_bit_cast(v8, make_uint4(pp[0], pp[1], pp[2], pp[3]));
-      i16x4_t lo[DBLK], hi[DBLK];
-#pragma unroll
-      for (int b = 0; b < DBLK; ++b) {
-        lo[b] = lds_read_tr16(vb_lds + 16 * t * D + voff[b][0]);
-        hi[b] = lds_read_tr16(vb_lds + 16 * t * D + voff[b][1]);
-      }
-#pragma unroll
-      for (int b = 0; b < DBLK; ++b) {
-        const i16x8_t a = __builtin_shufflevector(lo[b], hi[b], 0, 1, 2, 3, 4, 5, 6, 7);
-        o[b] = M::run(__builtin_bit_cast(v8, a), pb, o[b]);
-      }
-    }
-  };
-  // One LDS tile.  With two sub-tiles the code order lets the second
-  // half's K Q^T overlap the first half's softmax and the first half's
-  // P V overlap the second half's softmax (no branch between them).
-  auto compute = [&](auto MaskT, const uint16_t* kb_lds, const uint16_t* vb_lds, int k0) {
-    if constexpr (NSUB == 1) {
-      f32x16_t sv[2];
-      uint32_t pw[2][8];
-      qk(kb_lds, sv);
-      mask(MaskT, sv, k0);
-      rescale(soft(sv, pw));
-      pv(vb_lds, pw);
-    } else {
-      f32x16_t s0[2], s1[2];
-      uint32_t p0[2][8], p1[2][8];
-      qk(kb_lds, s0);
-      mask(MaskT, s0, k0);
-      qk(kb_lds + 64 * D, s1);
-      mask(MaskT, s1, k0 + 64);
-      rescale(soft(s0, p0));
-      pv(vb_lds, p0);
-      rescale(soft(s1, p1));
-      pv(vb_lds + 64 * D, p1);
-    }
-  };
-
-  // One step: start loading the next tile into the other stage, compute
-  // this one, then wait for the loads and make them visible to all.
-  auto step = [&](auto MaskT, uint16_t* Kc, uint16_t* Vc, uint16_t* Kn, uint16_t* Vn, int it) {
-    const int k0 = kb0 + it * KT;
-    const bool more = it + 1 < ntiles;
-    if (more) stage(Kn, Vn, k0 + KT);
-    compute(MaskT, Kc, Vc, k0);
-    __builtin_amdgcn_s_waitcnt(0);   // this thread's LDS loads have landed
-    __syncthreads();                 // ... and everyone's; the current stage is free
-    if (more && k0 + 2 * KT > kend) {
-      zero_tail(Vn, k0 + KT);
-      __syncthreads();
-    }
-  };
-  stage(Ks0, Vs0, kb0);
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  if (kb0 + KT > kend) {
-    zero_tail(Vs0, kb0);
-    __syncthreads();
-  }
-  // Tiles [0, nfull) need no mask for any row of the workgroup (its
-  // earliest row sits at position pos0 + qt0); the rest may.
-  const int nfull = PFX ? (kend - kb0) / KT
-                        : min(ntiles, min(kend, pos0 + qt0 + 1) / KT);
-  const std::false_type plain{};
-  const std::true_type masked{};
-  int it = 0;
-  for (; it + 1 < nfull; it += 2) {
-    step(plain, Ks0, Vs0, Ks1, Vs1, it);
-    step(plain, Ks1, Vs1, Ks0, Vs0, it + 1);
-  }
-  if (it < nfull) {
-    step(plain, Ks0, Vs0, Ks1, Vs1, it);
-    ++it;
-  }
-  for (; it < ntiles; ++it) {
-    if (it & 1)
-      step(masked, Ks1, Vs1, Ks0, Vs0, it);
-    else
-      step(masked, Ks0, Vs0, Ks1, Vs1, it);
-  }
-
-  // Row sum over both halves of the wavefront, then write this lane's
-  // query row: O^T slot i of block b is dim 32 b + 8 (i / 4) + 4 h + i % 4.
-  l_run = xor32_sum(l_run);
-  if constexpr (HK == 2) {
-    // (past the last step's barrier nobody reads the tiles)
-    uint16_t* const tiles[4] = {Ks0, Ks1, Vs0, Vs1};
-    constexpr int RT = 64 * RW;          // threads with rows of their own
-    static_assert(2 * L::TILE >= 4 * RT * 16 && DBLK <= 4, "O exchange fits the tiles");
-    const int rt = tid % RT;
-    if (kh == 1) {
-#pragma unroll
-      for (int b = 0; b < DBLK; ++b)
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          reinterpret_cast<float*>(tiles[b])[i * RT + rt] = o[b][i];
-      xml[rt] = make_float2(m_run, l_run);
-    }
-    __syncthreads();
-    if (kh == 1) return;
-    const float2 other = xml[rt];
-    const float mx = fmaxf(m_run, other.x);
-    const float f0 = fast_exp2(m_run - mx), f1 = fast_exp2(other.x - mx);
-    l_run = l_run * f0 + other.y * f1;
-#pragma unroll
-    for (int b = 0; b < DBLK; ++b)
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        o[b][i] = o[b][i] * f0 + reinterpret_cast<const float*>(tiles[b])[i * RT + rt] * f1;
-  }
-  if (qtok >= qlen || !qrow_ok) return;
-  const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
-  if constexpr (PFX) {
-    const int H = num_kv_heads * G;
-    const int64_t base = ((int64_t)qrow * H + kvh * G + qg) * kPrefixMaxSplits + split;
-    if (h == 0) {
-      pfx.ml[base * 2] = m_run;
-      pfx.ml[base * 2 + 1] = l_run;
-    }
-    float* ap = pfx.acc + base * D + 4 * h;
-#pragma unroll
-    for (int b = 0; b < DBLK; ++b)
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4)
-        *reinterpret_cast<float4*>(ap + 32 * b + 8 * g4) =
-            make_float4(o[b][4 * g4] * inv, o[b][4 * g4 + 1] * inv, o[b][4 * g4 + 2] * inv,
-                        o[b][4 * g4 + 3] * inv);
-    return;
-  }
-  T* op = A.out + (int64_t)(q0 + qtok) * A.out_stride + (int64_t)(kvh * G + qg) * D + 4 * h;
-#pragma unroll
-  for (int b = 0; b < DBLK; ++b)
-#pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4)
-      *reinterpret_cast<uint2*>(op + 32 * b + 8 * g4) =
-          make_uint2(M::pack2(o[b][4 * g4] * inv, o[b][4 * g4 + 1] * inv),
-                     M::pack2(o[b][4 * g4 + 2] * inv, o[b][4 * g4 + 3] * inv));
-}
-
-
-// The chunk sequence a chunk workgroup of group g serves: group rank
-// r = g / Hkv names the r-th chunk sequence by descending context length
-// (ties by index), so the longest sequences' tiles are dispatched first.
-// Every workgroup ranks the sequences itself (kChunkRankMax of them at
-// most; beyond that the order is the index order).  All threads of the
-// workgroup call it (it may hold two barriers).
-template <typename T>
-__device__ __forceinline__ int chunk_rank_pick(const ChunkArgs<T>& a, int grp, int* s_ctx,
-                                               int* s_pick) {
-  const int nseq = a.num_groups / a.num_kv_heads;
-  int pick = grp / a.num_kv_heads;
-  if (grp < a.num_groups && nseq > 1 && nseq <= kChunkRankMax) {
-    for (int t = threadIdx.x; t < nseq; t += blockDim.x) s_ctx[t] = a.ctx[a.seq_begin + t];
-    __syncthreads();
-    for (int t = threadIdx.x; t < nseq; t += blockDim.x) {
-      const int c = s_ctx[t];
-      int rank = 0;
-      for (int u = 0; u < nseq; ++u) {
-        const int cu = s_ctx[u];
-        rank += (cu > c || (cu == c && u < t)) ? 1 : 0;
-      }
-      if (rank == pick) *s_pick = t;
-    }
-    __syncthreads();
-    pick = *s_pick;
-  }
-  return pick;
-}
-
-// Prefill chunks (PFX = false) or the shared-prefix pass as a launch of its
-// own (PFX = true: workgroup = (item, kv head)).
-template <typename T, int D, int G, int BS, int W, int BPW, bool PFX, int HK>
-__global__ __launch_bounds__(64 * W, PFX ? 1 : 8 / (W * BPW)) void attn_chunk_mfma_kernel(
-    ChunkArgs<T> a) {
-  using L = ChunkLds<D, W * BPW>;
-  // One LDS object per stage and operand: a load in flight into one stage
-  // provably does not alias the reads of the other, so the compiler does not
-  // make those reads wait for it.
-  __shared__ __align__(16) uint16_t Ks0[L::TILE], Ks1[L::TILE], Vs0[L::TILE], Vs1[L::TILE];
-  const int wg = (int)blockIdx.x;
-  if constexpr (PFX) {
-    chunk_mfma_body<T, D, G, BS, W, BPW, true, 1>(a, wg / a.num_kv_heads, wg % a.num_kv_heads,
-                                                  (int)threadIdx.x, Ks0, Ks1, Vs0, Vs1);
-  } else {
-    __shared__ int s_ctx[kChunkRankMax];
-    __shared__ int s_pick;
-    const int grp = (wg / kXcds / a.nq_tiles) * kXcds + wg % kXcds;
-    const int pick = chunk_rank_pick(a, grp, s_ctx, &s_pick);
-    __shared__ float2 s_ml[HK == 2 ? 32 * W : 1];
-    chunk_mfma_body<T, D, G, BS, W, BPW, false, HK>(a, wg, pick, (int)threadIdx.x, Ks0, Ks1, Vs0,
-                                                    Vs1, s_ml);
-  }
-}
-
-template <typename T, int D, int G, int BS, bool NT, int NBUF>
-__global__ __launch_bounds__(kPersistMaxWaves * 64) void attn_decode_persistent_kernel(
-    const T* __restrict__ q, int64_t q_stride,
-    const T* __restrict__ kc, const T* __restrict__ vc, int num_kv_heads, int64_t num_cache_blocks,
-    const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ ctx,
-    int num_seqs, float scale_log2, T* __restrict__ out, int64_t out_stride,
-    int32_t* __restrict__ ws_off, float* __restrict__ ws_acc, float* __restrict__ ws_ml,
-    PrefixArgs pfx, int sync_mask) {
-  using S = HeadState<T, D, G, BS, NT>;
-  constexpr int VEC = S::VEC;
-  // LDS: s_off [num_seqs + 1], then (shared prefixes only) s_skip [num_seqs]
-  extern __shared__ int32_t s_off[];
-  int32_t* s_skip = s_off + num_seqs + 1;
-  __shared__ int32_t s_part[kPersistMaxWaves];
-  const int max_tokens = max_blocks * BS;
-  const bool has_pfx = pfx.blocks != nullptr;
-  scan_block_counts<BS>(ctx, pfx.blocks, num_seqs, max_tokens, s_off, s_part, s_skip);
-  const int total = s_off[num_seqs];
-  const int H = num_kv_heads * G;
-  const RangeSplit rs = make_range_split(total, (int)gridDim.x);
-  if (blockIdx.x == 0) write_row_headers<BS>(ws_off, s_off, has_pfx ? s_skip : nullptr, num_seqs, rs);
-  if (total == 0) return;
-  const int r0 = rs.start((int)blockIdx.x);
-  const int r1 = rs.start((int)blockIdx.x + 1);
-  if (r0 >= r1) return;
-
-  const int lane = threadIdx.x & 63;
-  const int kvh = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (kvh >= num_kv_heads) return;
-  const int64_t tok_stride = (int64_t)num_kv_heads * D;
-  const int64_t blk_stride = (int64_t)BS * tok_stride;
-
-  S st;
-  st.tg = lane / S::RL;
-  st.dc = lane % S::RL;
-  const int64_t lane_off = (int64_t)kvh * D + st.dc * VEC + st.tg * tok_stride;
-  const T* kbase = kc + lane_off;
-  const T* vbase = vc + lane_off;
-
-  int cur = -1;     // sequence whose state st holds (uniform)
-  int cur_end = 0;  // its context length
-  int cur_skip = 0; // its leading blocks attended by the shared-prefix units
-
-  // Finish sequence sq: a piece covering the whole sequence goes straight
-  // to `out` (merged with the row's shared-prefix partials, which the
-  // prefix launch before this one wrote), any other piece to its workspace
-  // slot (piece_slot), for the reduce kernel.
-  auto finish = [&](int sq) __attribute__((always_inline)) {
-    st.merge_token_groups();
-    const int a = s_off[sq], b = s_off[sq + 1];
-    const bool whole = a >= r0 && b <= r1;
-    if (st.tg != 0) return;
-    {
-      if (whole && cur_skip > 0) {
-        // fold in the prefix partials (splits of 128 keys), then normalise
-        const int nsplit = (cur_skip * BS + kPrefixKeysPerSplit - 1) / kPrefixKeysPerSplit;
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          const int hq = kvh * G + g;
-          const int64_t pb = ((int64_t)sq * H + hq) * kPrefixMaxSplits;
-          float mx = st.m[g];
-          for (int sp = 0; sp < nsplit; ++sp) mx = fmaxf(mx, pfx.ml[(pb + sp) * 2]);
-          const float fs = fast_exp2(st.m[g] - mx);
-          float L = st.l[g] * fs;
-          float o[S::VEC];
-#pragma unroll
-          for (int j = 0; j < S::VEC; ++j) o[j] = st.acc[g][j] * fs;
-          for (int sp = 0; sp < nsplit; ++sp) {
-            const float f = pfx.ml[(pb + sp) * 2 + 1] * fast_exp2(pfx.ml[(pb + sp) * 2] - mx);
-            L += f;
-            const float* ap = pfx.acc + (pb + sp) * D + st.dc * VEC;
-#pragma unroll
-            for (int j = 0; j < S::VEC; ++j) o[j] = fmaf(ap[j], f, o[j]);
-          }
-          const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-          T* op = out + (int64_t)sq * out_stride + (int64_t)hq * D + st.dc * VEC;
-#pragma unroll
-          for (int j = 0; j < VEC; ++j) elem<T>::store(op + j, o[j] * inv);
-        }
-        return;
-      }
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const int hq = kvh * G + g;
-      const float inv = st.l[g] > 0.0f ? 1.0f / st.l[g] : 0.0f;
-      if (whole) {
-        T* op = out + (int64_t)sq * out_stride + (int64_t)hq * D + st.dc * VEC;
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) elem<T>::store(op + j, st.acc[g][j] * inv);
-      } else {
-        const int slot = piece_slot(sq, rs.piece_rank(a, (int)blockIdx.x), (int)blockIdx.x,
-                                    num_seqs);
-        const int64_t base = (int64_t)slot * H + hq;
-        float* wp = ws_acc + base * D + st.dc * VEC;
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) wp[j] = st.acc[g][j] * inv;
-        if (st.dc == 0) { ws_ml[base * 2] = st.m[g]; ws_ml[base * 2 + 1] = st.l[g]; }
-      }
-    }
-  };
-
-  static_assert(NBUF == 2 || NBUF == 4, "NBUF");
-  uint4 k0[S::LOADS], v0[S::LOADS], k1[S::LOADS], v1[S::LOADS];
-  uint4 k2[NBUF == 4 ? S::LOADS : 1], v2[NBUF == 4 ? S::LOADS : 1];
-  uint4 k3[NBUF == 4 ? S::LOADS : 1], v3[NBUF == 4 ? S::LOADS : 1];
-  for (int base = r0; base < r1; base += 64) {
-    const int cnt = min(64, r1 - base);
-    // Lane i resolves flattened entry base + i.
-    const Entry en = resolve_entry(base + lane, lane < cnt, s_off, has_pfx ? s_skip : nullptr,
-                                   num_seqs, block_tables, max_blocks, num_cache_blocks);
-    auto phys = [&](int i) { return __builtin_amdgcn_readlane(en.phys, min(i, cnt - 1)); };
-    // Start (or continue) the sequence of entry i, then fold its block in;
-    // i >= cnt is a fully masked no-op so process() always runs.
-    auto visit = [&](const uint4* kk, const uint4* vv, int i) {
-      const bool real = i < cnt;
-      const int sq = __builtin_amdgcn_readlane(en.seq, min(i, cnt - 1));
-      const int lb = __builtin_amdgcn_readlane(en.blk, min(i, cnt - 1));
-      if (real && sq != cur) {
-        if (cur >= 0) finish(cur);
-        cur = sq;
-        cur_end = min(max(ctx[sq], 0), max_tokens);
-        cur_skip = has_pfx ? s_skip[sq] : 0;
-        st.init(q + (int64_t)sq * q_stride + (int64_t)kvh * G * D, scale_log2, lane);
-      }
-      st.process(kk, vv, lb, real ? cur_end : -1);
-    };
-    // NBUF register buffers rotate: NBUF - 1 blocks are in flight while one
-    // is folded in.  Loads past the group end reload its last block (cache
-    // hit) and their visits are masked no-ops.
-    //
-    // Every sync_mask + 1 blocks the workgroup's wavefronts (one per kv
-    // head, all walking the same blocks) meet at a plain barrier (no memory
-    // fence: loads stay in flight across it).  Left alone they drift apart
-    // by up to a quarter of the kernel (the CU's memory pipeline does not
-    // serve its eight wavefronts evenly) and the last one finishes alone;
-    // in step, all of them end together.  Every wavefront runs the same
-    // loop trip counts, so each reaches the same barriers.
-    if constexpr (NBUF == 2) {
-      st.load(kbase, vbase, phys(0), blk_stride, tok_stride, k0, v0);
-      for (int i = 0; i < cnt; i += 2) {
-        if (sync_mask >= 0 && (i & sync_mask) == 0) __builtin_amdgcn_s_barrier();
-        st.load(kbase, vbase, phys(i + 1), blk_stride, tok_stride, k1, v1);
-        __builtin_amdgcn_sched_barrier(0);
-        visit(k0, v0, i);
-        st.load(kbase, vbase, phys(i + 2), blk_stride, tok_stride, k0, v0);
-        __builtin_amdgcn_sched_barrier(0);
-        visit(k1, v1, i + 1);
-      }
-    } else {
-      st.load(kbase, vbase, phys(0), blk_stride, tok_stride, k0, v0);
-      st.load(kbase, vbase, phys(1), blk_stride, tok_stride, k1, v1);
-      st.load(kbase, vbase, phys(2), blk_stride, tok_stride, k2, v2);
-      for (int i = 0; i < cnt; i += 4) {
-        if (sync_mask >= 0 && (i & sync_mask) == 0) __builtin_amdgcn_s_barrier();
-        st.load(kbase, vbase, phys(i + 3), blk_stride, tok_stride, k3, v3);
-        __builtin_amdgcn_sched_barrier(0);
-        visit(k0, v0, i);
-        st.load(kbase, vbase, phys(i + 4), blk_stride, tok_stride, k0, v0);
-        __builtin_amdgcn_sched_barrier(0);
-        visit(k1, v1, i + 1);
-        st.load(kbase, vbase, phys(i + 5), blk_stride, tok_stride, k1, v1);
-        __builtin_amdgcn_sched_barrier(0);
-        visit(k2, v2, i + 2);
-        st.load(kbase, vbase, phys(i + 6), blk_stride, tok_stride, k2, v2);
-        __builtin_amdgcn_sched_barrier(0);
-        visit(k3, v3, i + 3);
-      }
-    }
-  }
-  if (cur >= 0) finish(cur);
-}
-
 // Running merge of softmax partials (m, l in log2 units, O / l) for four
 // dims of one query head.  add() folds U partials at a time, so their loads
 // can all be in flight together.
@@ -1582,6 +901,797 @@ struct MergeSource {
   }
 };
 
+// Key split of the chunk units: workgroup (unit, split) takes key tiles
+// [split * per, (split + 1) * per) of the unit, per = split_tiles(tiles of the
+// unit, nsplit); a unit of more than one such range writes partials (m, l in
+// log2 units, O / l) for attn_chunk_merge_kernel.
+struct KeySplit {
+  int nsplit, units;   // nsplit = 1: none
+  float* ml;           // [units][nsplit][rows][2]
+  float* acc;          // [units][nsplit][D / 4][rows][4]
+};
+constexpr int kSplitMinTiles = 4;
+constexpr int kSplitRows = 64;
+__device__ __forceinline__ int split_tiles(int ntiles, int nsplit) {
+  return max(kSplitMinTiles, (ntiles + nsplit - 1) / nsplit);
+}
+
+// Arguments of the MFMA attention body (prefill chunks or shared-prefix
+// units).
+template <typename T>
+struct ChunkArgs {
+  const T* __restrict__ q; int64_t q_stride;
+  const T* __restrict__ kc; const T* __restrict__ vc; int num_kv_heads; int64_t num_cache_blocks;
+  const int32_t* __restrict__ block_tables; int max_blocks;
+  const int32_t* __restrict__ cu; const int32_t* __restrict__ ctx; int seq_begin;
+  int nq_tiles, num_groups; float scale_log2; T* __restrict__ out; int64_t out_stride;
+  PrefixArgs pfx;
+  KeySplit ks;
+};
+
+// A chunk unit's place in the step: its kv head, sequence, query tokens and
+// the keys [0, kend) they need (kend <= 0: nothing to do).
+struct ChunkUnit { int kvh, seq, q0, qlen, qt0, pos0, kend; };
+
+template <int BS, int QT, typename A>
+__device__ __forceinline__ ChunkUnit chunk_unit(const A& a, int unit, int pick) {
+  ChunkUnit u{0, 0, 0, 0, 0, 0, 0};
+  const int slot = unit / kXcds;
+  const int grp = (slot / a.nq_tiles) * kXcds + unit % kXcds;
+  if (grp >= a.num_groups) return u;
+  u.kvh = grp % a.num_kv_heads;
+  u.seq = a.seq_begin + pick;
+  u.q0 = a.cu[u.seq];
+  u.qlen = a.cu[u.seq + 1] - u.q0;
+  u.qt0 = (a.nq_tiles - 1 - slot % a.nq_tiles) * QT;
+  if (u.qt0 >= u.qlen) return u;
+  const int ctxlen = min(a.ctx[u.seq], a.max_blocks * BS);
+  u.pos0 = ctxlen - u.qlen;                                       // position of chunk row 0
+  u.kend = max(0, min(ctxlen, u.pos0 + min(u.qt0 + QT, u.qlen)));
+  return u;
+}
+
+// PFX = false: prefill chunks (causal, normalised output rows); `unit` is
+// the workgroup id and `kvh_sel` the chunk sequence (index from seq_begin)
+// the caller's longest-first order gives it.  PFX = true: one shared-prefix
+// unit -- `unit` is the work item, `kvh_sel` the kv head: up to QT group
+// members against one 128-key split of the group's prefix (no causal mask;
+// every prefix key precedes every member's query), writing prefix partials.
+// The body runs on one team of W wavefronts (`tid` = thread index in the
+// team) with its own four LDS tiles.  Every early exit before the last
+// barrier depends only on (unit, its item), never on the team or the lane,
+// and teams that share a workgroup run the same item, so all wavefronts of
+// the workgroup meet the same barriers.
+//
+// HK = 2 (chunks that leave the chip idle): the workgroup has half as many
+// rows, and wavefronts w and w + W / 2 share 32 of them, taking the first and
+// the second 32 keys of every 64-key tile; the second hands its O, maximum
+// and sum over through LDS at the end (in the tiles, and xml).  Twice the
+// workgroups, each with half the work per tile.
+template <typename T, int D, int G, int BS, int W, int BPW, bool PFX, int HK, bool KS>
+__device__ __forceinline__ void chunk_mfma_body(const ChunkArgs<T>& A, int unit, int kvh_sel,
+                                                int tid, uint16_t* Ks0, uint16_t* Ks1,
+                                                uint16_t* Vs0, uint16_t* Vs1,
+                                                float2* xml = nullptr, int part = 0) {
+  static_assert(!KS || HK == 2, "key split");
+  static_assert(HK == 1 || (HK == 2 && !PFX && W == 4 && BPW == 1), "split tiles");
+  using M = Mfma32<T>;
+  using v8 = typename M::v8;
+  using L = ChunkLds<D, W * BPW>;
+  constexpr int kThreads = 64 * W;
+  constexpr int RW = W / HK;           // wavefronts with rows of their own
+  constexpr int QT = 32 * RW / G;      // query tokens per workgroup
+  constexpr int KB = 2 / HK;           // 32-key halves of a sub-tile per wavefront
+  constexpr int KT = 16 * W * BPW;     // keys per LDS tile
+  constexpr int NSUB = KT / 64;        // 64-key sub-tiles per LDS tile
+  static_assert(NSUB == 1 || NSUB == 2, "one or two 64-key sub-tiles");
+  constexpr int QSTEPS = D / 16;       // k-steps of K Q^T
+  constexpr int DBLK = D / 32;         // 32-dim blocks of O^T
+  constexpr int CPR = L::CPR;
+  constexpr int RPI = 64 / CPR;        // key rows per wave-wide 1 KiB load
+  constexpr int LPW = BS / RPI;        // loads per wavefront per tile (one block each)
+  static_assert(BS == 16 && (W == 4 || W == 8), "each wavefront stages one 16-token block");
+  const T* __restrict__ q = A.q;
+  const int64_t q_stride = A.q_stride;
+  const T* __restrict__ kc = A.kc;
+  const T* __restrict__ vc = A.vc;
+  const int num_kv_heads = A.num_kv_heads;
+  const int64_t num_cache_blocks = A.num_cache_blocks;
+  const int max_blocks = A.max_blocks;
+  const float scale_log2 = A.scale_log2;
+  const PrefixArgs& pfx = A.pfx;
+
+  // XCD-aware, longest-first order (chunks): workgroups are dispatched
+  // round-robin over the XCDs (id % kXcds) and, on each XCD, in id order as
+  // slots free up.  Workgroup id w serves group g = (w / kXcds / nq) *
+  // kXcds + w % kXcds -- kv head g % Hkv of the (g / Hkv)-th longest chunk
+  // sequence (the caller ranks them) -- and query tile nq - 1 - (w / kXcds)
+  // % nq: all query tiles of one group run on one XCD and share its L2 copy
+  // of the group's K/V, and each XCD starts with the longest tiles, which
+  // shortens the tail of the last wave of workgroups.
+  int kvh, seq, q0, qlen, qt0, pos0, kb0, kend, mbeg = 0, split = 0;
+  if constexpr (PFX) {
+    const int item = unit;
+    kvh = kvh_sel;
+    if (item >= pfx.max_items) return;
+    const int4 it = *reinterpret_cast<const int4*>(pfx.items + 4 * item);
+    // unused item (leader < 0), leaders beyond the decode rows (num_groups),
+    // member slices outside `members` or wider than QT, splits beyond the
+    // partial buffers: skipped
+    if (it.x < 0 || it.x >= A.num_groups || it.w < 0 || it.w >= kPrefixMaxSplits || it.y < 0 ||
+        it.z < 1 || it.z > QT || it.y > pfx.num_members - it.z)
+      return;
+    seq = it.x;                                 // the group leader's block table
+    mbeg = it.y;
+    qlen = it.z;                                // members in this item (<= QT)
+    split = it.w;
+    q0 = 0;
+    qt0 = 0;
+    const int pkeys = min(min(pfx.blocks[seq], max_blocks), kPrefixMaxBlocks) * BS;
+    kb0 = split * kPrefixKeysPerSplit;
+    kend = min(pkeys, kb0 + kPrefixKeysPerSplit);
+    pos0 = 0x3fffffff;                          // queries follow every prefix key
+    if (kb0 >= kend) return;
+  } else {
+    // (chunk_unit()'s arithmetic, written out: through the struct this kernel
+    // is scheduled 5 % slower, 15 chunks of 512 tokens 143 against 136 us)
+    const int wg = unit;
+    const int slot = wg / kXcds;
+    const int grp = (slot / A.nq_tiles) * kXcds + wg % kXcds;
+    if (grp >= A.num_groups) return;
+    kvh = grp % num_kv_heads;
+    seq = A.seq_begin + kvh_sel;
+    q0 = A.cu[seq];
+    qlen = A.cu[seq + 1] - q0;
+    qt0 = (A.nq_tiles - 1 - slot % A.nq_tiles) * QT;
+    if (qt0 >= qlen) return;
+    const int ctxlen = min(A.ctx[seq], max_blocks * BS);
+    pos0 = ctxlen - qlen;                                      // position of chunk row 0
+    kb0 = 0;
+    kend = max(0, min(ctxlen, pos0 + min(qt0 + QT, qlen)));    // keys [0, kend)
+    if (kend <= 0) return;
+  }
+  bool partial = false;            // KS: the unit has other ranges
+  if constexpr (KS) {
+    const int tiles = (kend + KT - 1) / KT, per = split_tiles(tiles, A.ks.nsplit);
+    kb0 = part * per * KT;
+    if (kb0 >= kend) return;       // (the whole workgroup, before any barrier)
+    partial = per < tiles;
+    kend = min(kend, kb0 + per * KT);
+  }
+  const int ntiles = (kend - kb0 + KT - 1) / KT;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int lr = lane & 31;        // this lane's query column / key row
+  const int h = lane >> 5;         // half of the wavefront
+  const int64_t tok_stride = (int64_t)num_kv_heads * D;
+  const int32_t* __restrict__ bt = A.block_tables + (int64_t)seq * max_blocks;
+
+  // This lane's query row (the B-operand column of K Q^T).
+  const int row = 32 * (HK == 1 ? wave : wave % RW) + lr;
+  const int kh = HK == 1 ? 0 : wave / RW;   // HK = 2: this wavefront's half of each tile
+  const int qtok = qt0 + row % QT;
+  const int qg = row / QT;
+  const int qpos = PFX ? pos0 : pos0 + qtok;
+  int qrow = PFX ? pfx.members[mbeg + min(qtok, qlen - 1)] : q0 + min(qtok, qlen - 1);
+  bool qrow_ok = true;
+  if constexpr (PFX) {
+    qrow_ok = qrow >= 0 && qrow < A.num_groups;
+    qrow = qrow_ok ? qrow : seq;
+  }
+  v8 qf[QSTEPS];
+  {
+    const T* qp = q + (int64_t)qrow * q_stride + (int64_t)(kvh * G + qg) * D + 8 * h;
+#pragma unroll
+    for (int st = 0; st < QSTEPS; ++st) qf[st] = __builtin_bit_cast(v8, load16(qp + 16 * st));
+  }
+
+  // Staging: wavefront w loads block w of the tile (rows 16w..16w+15) with
+  // LPW wave-wide loads; lane l of load u fills LDS slot l % CPR of row
+  // 16w + RPI u + l / CPR, i.e. the row's chunk (l % CPR) ^ swz(row).
+  int64_t goff[LPW];
+#pragma unroll
+  for (int u = 0; u < LPW; ++u) {
+    const int r = RPI * u + lane / CPR;            // row inside the block
+    const int chunk = (lane % CPR) ^ L::swz(r);        // 16-row blocks keep row & 15
+    goff[u] = (int64_t)r * tok_stride + (int64_t)kvh * D + 8 * chunk;
+  }
+  const int last_blk = (kend - 1) / BS;
+  const int64_t blk_elems = (int64_t)BS * tok_stride;
+  // Chunks: physical ids of this wavefront's blocks (blocks wave + W j of
+  // each tile), 64 tiles at a time: lane l of bids[j] holds tile bid_tb + l,
+  // loaded ahead so staging a tile never waits for a block-table read.  (A
+  // shared-prefix unit has at most two tiles and reads its ids directly.)
+  int bids[BPW];
+  int bid_tb = 0;
+  auto load_bids = [&](int tb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < BPW; ++j) {
+      const int b = bt[min((kb0 + (tb + lane) * KT) / BS + wave + W * j, last_blk)];
+      const bool bad = b < 0 || b >= num_cache_blocks;   // clamped and reported
+      if (bad) report_device_error(LV_DEVERR_BLOCK_ID);
+      bids[j] = bad ? 0 : b;
+    }
+    bid_tb = tb;
+  };
+  if constexpr (!PFX) load_bids(0);
+  // Wavefront w stages blocks w, w + W, ... (BPW of them) of the tile.
+  auto stage = [&](uint16_t* Kst, uint16_t* Vst, int k0) {
+    const int tile = (k0 - kb0) / KT;
+    if constexpr (!PFX) {
+      if (tile - bid_tb >= 64) load_bids(tile);   // contexts beyond 64 tiles
+    }
+#pragma unroll
+    for (int j = 0; j < BPW; ++j) {
+      const int blk = wave + W * j;
+      int b;
+      if constexpr (PFX) {
+        b = bt[min(k0 / BS + blk, last_blk)];
+        if (b < 0 || b >= num_cache_blocks) {   // clamped and reported
+          report_device_error(LV_DEVERR_BLOCK_ID);
+          b = 0;
+        }
+      } else {
+        b = __builtin_amdgcn_readlane(bids[j], tile - bid_tb);
+      }
+      const T* kp = kc + (int64_t)b * blk_elems;
+      const T* vp = vc + (int64_t)b * blk_elems;
+      uint16_t* kd = Kst + 16 * blk * D;
+      uint16_t* vd = Vst + 16 * blk * D;
+#pragma unroll
+      for (int u = 0; u < LPW; ++u) {
+        load_lds16(kp + goff[u], kd + RPI * u * D);
+        load_lds16(vp + goff[u], vd + RPI * u * D);
+      }
+    }
+  };
+  // Rows at or past kend hold data of the clamped block: zero their V so a
+  // zero probability never meets a NaN (their scores are masked).
+  auto zero_tail = [&](uint16_t* Vst, int k0) {
+    for (int c = tid; c < KT * CPR; c += kThreads)
+      if (k0 + c / CPR >= kend) store16(Vst + (c / CPR) * D + 8 * (c % CPR), make_uint4(0, 0, 0, 0));
+  };
+
+  f32x16_t o[DBLK];
+#pragma unroll
+  for (int b = 0; b < DBLK; ++b)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[b][i] = 0.0f;
+  float m_run = kNegBig, l_run = 0.0f;
+
+
+  // Per-lane LDS offsets of the MFMA operands.  Rows 32 kb + lr share
+  // lr's swizzle (it depends on row % 16 only), so the K offset of step st
+  // is kx[st] plus the constant 32 kb D; the V rows 16 t + vrow (+ 8)
+  // likewise share a swizzle across t.
+  int kx[QSTEPS];
+  {
+    const int y = h ^ L::swz(lr);         // (2 st + h) ^ sw == 2 st ^ y
+#pragma unroll
+    for (int st = 0; st < QSTEPS; ++st) kx[st] = lr * D + 8 * ((2 * st) ^ y);
+  }
+  const int vrow = 4 * h + ((lane & 15) >> 2);
+  int voff[DBLK][2];
+#pragma unroll
+  for (int b = 0; b < DBLK; ++b) {
+    const int dim = 32 * b + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    voff[b][0] = L::at(vrow, dim >> 3) + (dim & 7);
+    voff[b][1] = L::at(vrow + 8, dim >> 3) + (dim & 7);
+  }
+
+  // S^T of one 64-key sub-tile (raw scores, two 32-key halves): 16 MFMAs,
+  // step j = (half j / 8, k-step j % 8), with four K operand reads in
+  // flight.  The order is pinned (read j + 4 goes out right after MFMA j
+  // frees its buffer): left to itself the scheduler, at this register
+  // budget, gives all reads one buffer and waits out each read in turn.
+  auto qk = [&](const uint16_t* kb_lds, f32x16_t* sv) {
+    auto kread = [&](int j) __attribute__((always_inline)) {
+      return *reinterpret_cast<const uint4*>(kb_lds + 32 * (j >> 3) * D + kx[j & 7]);
+    };
+    kb_lds += 32 * kh * D;
+    static_assert(QSTEPS == 8 || QSTEPS == 4, "head_dim 128 or 64");
+    constexpr int NJ = KB * QSTEPS;
+    uint4 ka[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) ka[j] = kread((j / QSTEPS) * 8 + j % QSTEPS);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      __builtin_amdgcn_sched_barrier(0);
+      const int kb = j / QSTEPS, st = j % QSTEPS;
+      sv[kb] = M::run(__builtin_bit_cast(v8, ka[j & 3]), qf[st], st ? sv[kb] : f32x16_t{});
+      if (j + 4 < NJ) ka[j & 3] = kread(((j + 4) / QSTEPS) * 8 + (j + 4) % QSTEPS);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Causal / range mask (MaskT = std::true_type on tiles that may need it;
+  // those run in a loop of their own so the mask is never straight-line code
+  // on the others): slot i of half kb holds key k0 + 32 kb + 8 (i/4) + 4 h + i%4.
+  const int lim = min(qpos, kend - 1);   // last key each row may see
+  auto mask = [&](auto MaskT, f32x16_t* sv, int k0) {
+    if constexpr (decltype(MaskT)::value) {
+      const int d = lim - k0 - 32 * kh - 4 * h;
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (32 * kb + 8 * (i >> 2) + (i & 3) > d) sv[kb][i] = kNegBig;
+    }
+  };
+  // Online softmax in log2 units with a lazily raised maximum: the running
+  // maximum m_run moves only when a row's maximum exceeds it by more than
+  // 2^8 (or on the first tile), so probabilities stay below 256 and the O
+  // rescale is rare.  Returns the factor O must be scaled by (1 = none).
+  auto soft = [&](const f32x16_t* sv, uint32_t (*pw)[8]) {
+    float mx = kNegBig;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sv[kb][i]);
+    mx = xor32_max(mx) * scale_log2;
+    float alpha = 1.0f;
+    // HK = 2: while every key of a row has been masked in this wavefront's
+    // halves, m_run stays kNegBig and the weights are 0
+    if (mx > m_run + 8.0f && (HK == 1 || mx > kNegBig * 0.01f)) {
+      alpha = fast_exp2(m_run - mx);
+      m_run = mx;
+    }
+    const float m_ref = HK == 2 && m_run == kNegBig ? 0.0f : m_run;
+    float psum = 0.0f;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) {
+        const float p0 = fast_exp2(fmaf(sv[kb][i], scale_log2, -m_ref));
+        const float p1 = fast_exp2(fmaf(sv[kb][i + 1], scale_log2, -m_ref));
+        psum += p0 + p1;
+        pw[kb][i >> 1] = M::pack2(p0, p1);
+      }
+    l_run = l_run * alpha + psum;
+    return alpha;
+  };
+  auto rescale = [&](float alpha) {
+    if (__ballot(alpha != 1.0f)) {   // uniform branch, rare after the first tile
+#pragma unroll
+      for (int b = 0; b < DBLK; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[b][i] *= alpha;
+    }
+  };
+  // O^T += V^T P^T over one 64-key sub-tile, four 16-key steps; each step's
+  // transpose reads are issued together ahead of its MFMAs.
+  auto pv = [&](const uint16_t* vb_lds, const uint32_t (*pw)[8]) {
+    vb_lds += 32 * kh * D;
+#pragma unroll
+    for (int t = 0; t < 2 * KB; ++t) {
+      const uint32_t* pp = &pw[t >> 1][4 * (t & 1)];
+      const v8 pb = __builtin_bit_cast(v8, make_uint4(pp[0], pp[1], pp[2], pp[3]));
+      i16x4_t lo[DBLK], hi[DBLK];
+#pragma unroll
+      for (int b = 0; b < DBLK; ++b) {
+        lo[b] = lds_read_tr16(vb_lds + 16 * t * D + voff[b][0]);
+        hi[b] = lds_read_tr16(vb_lds + 16 * t * D + voff[b][1]);
+      }
+#pragma unroll
+      for (int b = 0; b < DBLK; ++b) {
+        const i16x8_t a = __builtin_shufflevector(lo[b], hi[b], 0, 1, 2, 3, 4, 5, 6, 7);
+        o[b] = M::run(__builtin_bit_cast(v8, a), pb, o[b]);
+      }
+    }
+  };
+  // One LDS tile.  With two sub-tiles the code order lets the second
+  // half's K Q^T overlap the first half's softmax and the first half's
+  // P V overlap the second half's softmax (no branch between them).
+  auto compute = [&](auto MaskT, const uint16_t* kb_lds, const uint16_t* vb_lds, int k0) {
+    if constexpr (NSUB == 1) {
+      f32x16_t sv[2];
+      uint32_t pw[2][8];
+      qk(kb_lds, sv);
+      mask(MaskT, sv, k0);
+      rescale(soft(sv, pw));
+      pv(vb_lds, pw);
+    } else {
+      f32x16_t s0[2], s1[2];
+      uint32_t p0[2][8], p1[2][8];
+      qk(kb_lds, s0);
+      mask(MaskT, s0, k0);
+      qk(kb_lds + 64 * D, s1);
+      mask(MaskT, s1, k0 + 64);
+      rescale(soft(s0, p0));
+      pv(vb_lds, p0);
+      rescale(soft(s1, p1));
+      pv(vb_lds + 64 * D, p1);
+    }
+  };
+
+  // One step: start loading the next tile into the other stage, compute
+  // this one, then wait for the loads and make them visible to all.
+  auto step = [&](auto MaskT, uint16_t* Kc, uint16_t* Vc, uint16_t* Kn, uint16_t* Vn, int it) {
+    const int k0 = kb0 + it * KT;
+    const bool more = it + 1 < ntiles;
+    if (more) stage(Kn, Vn, k0 + KT);
+    compute(MaskT, Kc, Vc, k0);
+    __builtin_amdgcn_s_waitcnt(0);   // this thread's LDS loads have landed
+    __syncthreads();                 // ... and everyone's; the current stage is free
+    if (more && k0 + 2 * KT > kend) {
+      zero_tail(Vn, k0 + KT);
+      __syncthreads();
+    }
+  };
+  stage(Ks0, Vs0, kb0);
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (kb0 + KT > kend) {
+    zero_tail(Vs0, kb0);
+    __syncthreads();
+  }
+  // Tiles [0, nfull) need no mask for any row of the workgroup (its
+  // earliest row sits at position pos0 + qt0); the rest may.
+  const int nfull = PFX ? (kend - kb0) / KT
+                   : KS ? min(ntiles, max(0, min(kend, pos0 + qt0 + 1) - kb0) / KT)
+                        : min(ntiles, min(kend, pos0 + qt0 + 1) / KT);
+  const std::false_type plain{};
+  const std::true_type masked{};
+  int it = 0;
+  for (; it + 1 < nfull; it += 2) {
+    step(plain, Ks0, Vs0, Ks1, Vs1, it);
+    step(plain, Ks1, Vs1, Ks0, Vs0, it + 1);
+  }
+  if (it < nfull) {
+    step(plain, Ks0, Vs0, Ks1, Vs1, it);
+    ++it;
+  }
+  for (; it < ntiles; ++it) {
+    if (it & 1)
+      step(masked, Ks1, Vs1, Ks0, Vs0, it);
+    else
+      step(masked, Ks0, Vs0, Ks1, Vs1, it);
+  }
+
+  // Row sum over both halves of the wavefront, then write this lane's
+  // query row: O^T slot i of block b is dim 32 b + 8 (i / 4) + 4 h + i % 4.
+  l_run = xor32_sum(l_run);
+  if constexpr (HK == 2) {
+    // (past the last step's barrier nobody reads the tiles)
+    uint16_t* const tiles[4] = {Ks0, Ks1, Vs0, Vs1};
+    constexpr int RT = 64 * RW;          // threads with rows of their own
+    static_assert(2 * L::TILE >= 4 * RT * 16 && DBLK <= 4, "O exchange fits the tiles");
+    const int rt = tid % RT;
+    if (kh == 1) {
+#pragma unroll
+      for (int b = 0; b < DBLK; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          reinterpret_cast<float*>(tiles[b])[i * RT + rt] = o[b][i];
+      xml[rt] = make_float2(m_run, l_run);
+    }
+    __syncthreads();
+    if (kh == 1) return;
+    const float2 other = xml[rt];
+    const float mx = fmaxf(m_run, other.x);
+    const float f0 = fast_exp2(m_run - mx), f1 = fast_exp2(other.x - mx);
+    l_run = l_run * f0 + other.y * f1;
+    m_run = mx;
+#pragma unroll
+    for (int b = 0; b < DBLK; ++b)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        o[b][i] = o[b][i] * f0 + reinterpret_cast<const float*>(tiles[b])[i * RT + rt] * f1;
+  }
+  if (qtok >= qlen || !qrow_ok) return;
+  const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
+  if constexpr (PFX) {
+    const int H = num_kv_heads * G;
+    const int64_t base = ((int64_t)qrow * H + kvh * G + qg) * kPrefixMaxSplits + split;
+    if (h == 0) {
+      pfx.ml[base * 2] = m_run;
+      pfx.ml[base * 2 + 1] = l_run;
+    }
+    float* ap = pfx.acc + base * D + 4 * h;
+#pragma unroll
+    for (int b = 0; b < DBLK; ++b)
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4)
+        *reinterpret_cast<float4*>(ap + 32 * b + 8 * g4) =
+            make_float4(o[b][4 * g4] * inv, o[b][4 * g4 + 1] * inv, o[b][4 * g4 + 2] * inv,
+                        o[b][4 * g4 + 3] * inv);
+    return;
+  }
+  if constexpr (KS) {
+    if (partial) {
+      const int64_t slot = (int64_t)unit * A.ks.nsplit + part;
+      if (h == 0)
+        *reinterpret_cast<float2*>(A.ks.ml + (slot * kSplitRows + row) * 2) =
+            make_float2(m_run, l_run);
+      float* ap = A.ks.acc + slot * (D * kSplitRows) + 4 * row;
+#pragma unroll
+      for (int b = 0; b < DBLK; ++b)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4)   // dims 32 b + 8 g4 + 4 h ..
+          *reinterpret_cast<float4*>(ap + (8 * b + 2 * g4 + h) * (4 * kSplitRows)) =
+              make_float4(o[b][4 * g4] * inv, o[b][4 * g4 + 1] * inv, o[b][4 * g4 + 2] * inv,
+                          o[b][4 * g4 + 3] * inv);
+      return;
+    }
+  }
+  T* op = A.out + (int64_t)(q0 + qtok) * A.out_stride + (int64_t)(kvh * G + qg) * D + 4 * h;
+#pragma unroll
+  for (int b = 0; b < DBLK; ++b)
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4)
+      *reinterpret_cast<uint2*>(op + 32 * b + 8 * g4) =
+          make_uint2(M::pack2(o[b][4 * g4] * inv, o[b][4 * g4 + 1] * inv),
+                     M::pack2(o[b][4 * g4 + 2] * inv, o[b][4 * g4 + 3] * inv));
+}
+
+
+// The chunk sequence a chunk workgroup of group g serves: group rank
+// r = g / Hkv names the r-th chunk sequence by descending context length
+// (ties by index), so the longest sequences' tiles are dispatched first.
+// Every workgroup ranks the sequences itself (kChunkRankMax of them at
+// most; beyond that the order is the index order).  All threads of the
+// workgroup call it (it may hold two barriers).
+template <typename T>
+__device__ __forceinline__ int chunk_rank_pick(const ChunkArgs<T>& a, int grp, int* s_ctx,
+                                               int* s_pick) {
+  const int nseq = a.num_groups / a.num_kv_heads;
+  int pick = grp / a.num_kv_heads;
+  if (grp < a.num_groups && nseq > 1 && nseq <= kChunkRankMax) {
+    for (int t = threadIdx.x; t < nseq; t += blockDim.x) s_ctx[t] = a.ctx[a.seq_begin + t];
+    __syncthreads();
+    for (int t = threadIdx.x; t < nseq; t += blockDim.x) {
+      const int c = s_ctx[t];
+      int rank = 0;
+      for (int u = 0; u < nseq; ++u) {
+        const int cu = s_ctx[u];
+        rank += (cu > c || (cu == c && u < t)) ? 1 : 0;
+      }
+      if (rank == pick) *s_pick = t;
+    }
+    __syncthreads();
+    pick = *s_pick;
+  }
+  return pick;
+}
+
+// Prefill chunks (PFX = false) or the shared-prefix pass as a launch of its
+// own (PFX = true: workgroup = (item, kv head)).
+template <typename T, int D, int G, int BS, int W, int BPW, bool PFX, int HK, bool KS>
+__global__ __launch_bounds__(64 * W, PFX ? 1 : 8 / (W * BPW)) void attn_chunk_mfma_kernel(
+    ChunkArgs<T> a) {
+  using L = ChunkLds<D, W * BPW>;
+  // One LDS object per stage and operand: a load in flight into one stage
+  // provably does not alias the reads of the other, so the compiler does not
+  // make those reads wait for it.
+  __shared__ __align__(16) uint16_t Ks0[L::TILE], Ks1[L::TILE], Vs0[L::TILE], Vs1[L::TILE];
+  const int wg = KS ? (int)(blockIdx.x % a.ks.units) : (int)blockIdx.x;
+  if constexpr (PFX) {
+    chunk_mfma_body<T, D, G, BS, W, BPW, true, 1, false>(a, wg / a.num_kv_heads, wg % a.num_kv_heads,
+                                                  (int)threadIdx.x, Ks0, Ks1, Vs0, Vs1);
+  } else {
+    __shared__ int s_ctx[kChunkRankMax];
+    __shared__ int s_pick;
+    const int grp = (wg / kXcds / a.nq_tiles) * kXcds + wg % kXcds;
+    const int pick = chunk_rank_pick(a, grp, s_ctx, &s_pick);
+    __shared__ float2 s_ml[HK == 2 ? 32 * W : 1];
+    chunk_mfma_body<T, D, G, BS, W, BPW, false, HK, KS>(
+        a, wg, pick, (int)threadIdx.x, Ks0, Ks1, Vs0, Vs1, s_ml,
+        KS ? (int)(blockIdx.x / a.ks.units) : 0);
+  }
+}
+
+// Merge of the key-split chunk units: workgroup = (unit, 16 dims), thread =
+// (row, 4 dims), splits four loads at a time in key order.
+template <typename T, int D, int G, int BS>
+__global__ __launch_bounds__(256) void attn_chunk_merge_kernel(ChunkArgs<T> a) {
+  __shared__ int s_ctx[kChunkRankMax];
+  __shared__ int s_pick;
+  const int unit = blockIdx.x;
+  const int pick = chunk_rank_pick(a, (unit / kXcds / a.nq_tiles) * kXcds + unit % kXcds, s_ctx,
+                                   &s_pick);
+  const ChunkUnit u = chunk_unit<BS, kSplitRows / G>(a, unit, pick);
+  if (u.kend <= 0) return;
+  const int tiles = (u.kend + 63) / 64, per = split_tiles(tiles, a.ks.nsplit);
+  if (per >= tiles) return;            // one range: already in `out`
+  const int n = (tiles + per - 1) / per;
+  const int row = threadIdx.x & (kSplitRows - 1);
+  const int d4 = blockIdx.y * 4 + (int)threadIdx.x / kSplitRows;   // dims 4 d4 ..
+  const int qtok = u.qt0 + row % (kSplitRows / G), qg = row / (kSplitRows / G);
+  if (qtok >= u.qlen) return;
+  const int64_t slot = (int64_t)unit * a.ks.nsplit;
+  MergeState st;
+  for (int i = 0; i < n; i += 4) {
+    float2 ml[4]; float4 v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int64_t sp = slot + min(i + j, n - 1);
+      ml[j] = *reinterpret_cast<const float2*>(a.ks.ml + (sp * kSplitRows + row) * 2);
+      v[j] = *reinterpret_cast<const float4*>(a.ks.acc + sp * (D * kSplitRows) +
+                                              (d4 * kSplitRows + row) * 4);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (i + j >= n) ml[j] = make_float2(kNegBig, 0.0f);
+    st.add(ml, v);
+  }
+  const float inv = st.l > 0.0f ? 1.0f / st.l : 0.0f;
+  T* op = a.out + (int64_t)(u.q0 + qtok) * a.out_stride + (int64_t)(u.kvh * G + qg) * D + 4 * d4;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) elem<T>::store(op + j, st.o[j] * inv);
+}
+
+template <typename T, int D, int G, int BS, bool NT, int NBUF>
+__global__ __launch_bounds__(kPersistMaxWaves * 64) void attn_decode_persistent_kernel(
+    const T* __restrict__ q, int64_t q_stride,
+    const T* __restrict__ kc, const T* __restrict__ vc, int num_kv_heads, int64_t num_cache_blocks,
+    const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ ctx,
+    int num_seqs, float scale_log2, T* __restrict__ out, int64_t out_stride,
+    int32_t* __restrict__ ws_off, float* __restrict__ ws_acc, float* __restrict__ ws_ml,
+    PrefixArgs pfx, int sync_mask) {
+  using S = HeadState<T, D, G, BS, NT>;
+  constexpr int VEC = S::VEC;
+  // LDS: s_off [num_seqs + 1], then (shared prefixes only) s_skip [num_seqs]
+  extern __shared__ int32_t s_off[];
+  int32_t* s_skip = s_off + num_seqs + 1;
+  __shared__ int32_t s_part[kPersistMaxWaves];
+  const int max_tokens = max_blocks * BS;
+  const bool has_pfx = pfx.blocks != nullptr;
+  scan_block_counts<BS>(ctx, pfx.blocks, num_seqs, max_tokens, s_off, s_part, s_skip);
+  const int total = s_off[num_seqs];
+  const int H = num_kv_heads * G;
+  const RangeSplit rs = make_range_split(total, (int)gridDim.x);
+  if (blockIdx.x == 0) write_row_headers<BS>(ws_off, s_off, has_pfx ? s_skip : nullptr, num_seqs, rs);
+  if (total == 0) return;
+  const int r0 = rs.start((int)blockIdx.x);
+  const int r1 = rs.start((int)blockIdx.x + 1);
+  if (r0 >= r1) return;
+
+  const int lane = threadIdx.x & 63;
+  const int kvh = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (kvh >= num_kv_heads) return;
+  const int64_t tok_stride = (int64_t)num_kv_heads * D;
+  const int64_t blk_stride = (int64_t)BS * tok_stride;
+
+  S st;
+  st.tg = lane / S::RL;
+  st.dc = lane % S::RL;
+  const int64_t lane_off = (int64_t)kvh * D + st.dc * VEC + st.tg * tok_stride;
+  const T* kbase = kc + lane_off;
+  const T* vbase = vc + lane_off;
+
+  int cur = -1;     // sequence whose state st holds (uniform)
+  int cur_end = 0;  // its context length
+  int cur_skip = 0; // its leading blocks attended by the shared-prefix units
+
+  // Finish sequence sq: a piece covering the whole sequence goes straight
+  // to `out` (merged with the row's shared-prefix partials, which the
+  // prefix launch before this one wrote), any other piece to its workspace
+  // slot (piece_slot), for the reduce kernel.
+  auto finish = [&](int sq) __attribute__((always_inline)) {
+    st.merge_token_groups();
+    const int a = s_off[sq], b = s_off[sq + 1];
+    const bool whole = a >= r0 && b <= r1;
+    if (st.tg != 0) return;
+    {
+      if (whole && cur_skip > 0) {
+        // fold in the prefix partials (splits of 128 keys), then normalise
+        const int nsplit = (cur_skip * BS + kPrefixKeysPerSplit - 1) / kPrefixKeysPerSplit;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const int hq = kvh * G + g;
+          const int64_t pb = ((int64_t)sq * H + hq) * kPrefixMaxSplits;
+          float mx = st.m[g];
+          for (int sp = 0; sp < nsplit; ++sp) mx = fmaxf(mx, pfx.ml[(pb + sp) * 2]);
+          const float fs = fast_exp2(st.m[g] - mx);
+          float L = st.l[g] * fs;
+          float o[S::VEC];
+#pragma unroll
+          for (int j = 0; j < S::VEC; ++j) o[j] = st.acc[g][j] * fs;
+          for (int sp = 0; sp < nsplit; ++sp) {
+            const float f = pfx.ml[(pb + sp) * 2 + 1] * fast_exp2(pfx.ml[(pb + sp) * 2] - mx);
+            L += f;
+            const float* ap = pfx.acc + (pb + sp) * D + st.dc * VEC;
+#pragma unroll
+            for (int j = 0; j < S::VEC; ++j) o[j] = fmaf(ap[j], f, o[j]);
+          }
+          const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+          T* op = out + (int64_t)sq * out_stride + (int64_t)hq * D + st.dc * VEC;
+#pragma unroll
+          for (int j = 0; j < VEC; ++j) elem<T>::store(op + j, o[j] * inv);
+        }
+        return;
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int hq = kvh * G + g;
+      const float inv = st.l[g] > 0.0f ? 1.0f / st.l[g] : 0.0f;
+      if (whole) {
+        T* op = out + (int64_t)sq * out_stride + (int64_t)hq * D + st.dc * VEC;
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) elem<T>::store(op + j, st.acc[g][j] * inv);
+      } else {
+        const int slot = piece_slot(sq, rs.piece_rank(a, (int)blockIdx.x), (int)blockIdx.x,
+                                    num_seqs);
+        const int64_t base = (int64_t)slot * H + hq;
+        float* wp = ws_acc + base * D + st.dc * VEC;
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) wp[j] = st.acc[g][j] * inv;
+        if (st.dc == 0) { ws_ml[base * 2] = st.m[g]; ws_ml[base * 2 + 1] = st.l[g]; }
+      }
+    }
+  };
+
+  static_assert(NBUF == 2 || NBUF == 4, "NBUF");
+  uint4 k0[S::LOADS], v0[S::LOADS], k1[S::LOADS], v1[S::LOADS];
+  uint4 k2[NBUF == 4 ? S::LOADS : 1], v2[NBUF == 4 ? S::LOADS : 1];
+  uint4 k3[NBUF == 4 ? S::LOADS : 1], v3[NBUF == 4 ? S::LOADS : 1];
+  for (int base = r0; base < r1; base += 64) {
+    const int cnt = min(64, r1 - base);
+    // Lane i resolves flattened entry base + i.
+    const Entry en = resolve_entry(base + lane, lane < cnt, s_off, has_pfx ? s_skip : nullptr,
+                                   num_seqs, block_tables, max_blocks, num_cache_blocks);
+    auto phys = [&](int i) { return __builtin_amdgcn_readlane(en.phys, min(i, cnt - 1)); };
+    // Start (or continue) the sequence of entry i, then fold its block in;
+    // i >= cnt is a fully masked no-op so process() always runs.
+    auto visit = [&](const uint4* kk, const uint4* vv, int i) {
+      const bool real = i < cnt;
+      const int sq = __builtin_amdgcn_readlane(en.seq, min(i, cnt - 1));
+      const int lb = __builtin_amdgcn_readlane(en.blk, min(i, cnt - 1));
+      if (real && sq != cur) {
+        if (cur >= 0) finish(cur);
+        cur = sq;
+        cur_end = min(max(ctx[sq], 0), max_tokens);
+        cur_skip = has_pfx ? s_skip[sq] : 0;
+        st.init(q + (int64_t)sq * q_stride + (int64_t)kvh * G * D, scale_log2, lane);
+      }
+      st.process(kk, vv, lb, real ? cur_end : -1);
+    };
+    // NBUF register buffers rotate: NBUF - 1 blocks are in flight while one
+    // is folded in.  Loads past the group end reload its last block (cache
+    // hit) and their visits are masked no-ops.
+    //
+    // Every sync_mask + 1 blocks the workgroup's wavefronts (one per kv
+    // head, all walking the same blocks) meet at a plain barrier (no memory
+    // fence: loads stay in flight across it).  Left alone they drift apart
+    // by up to a quarter of the kernel (the CU's memory pipeline does not
+    // serve its eight wavefronts evenly) and the last one finishes alone;
+    // in step, all of them end together.  Every wavefront runs the same
+    // loop trip counts, so each reaches the same barriers.
+    if constexpr (NBUF == 2) {
+      st.load(kbase, vbase, phys(0), blk_stride, tok_stride, k0, v0);
+      for (int i = 0; i < cnt; i += 2) {
+        if (sync_mask >= 0 && (i & sync_mask) == 0) __builtin_amdgcn_s_barrier();
+        st.load(kbase, vbase, phys(i + 1), blk_stride, tok_stride, k1, v1);
+        __builtin_amdgcn_sched_barrier(0);
+        visit(k0, v0, i);
+        st.load(kbase, vbase, phys(i + 2), blk_stride, tok_stride, k0, v0);
+        __builtin_amdgcn_sched_barrier(0);
+        visit(k1, v1, i + 1);
+      }
+    } else {
+      st.load(kbase, vbase, phys(0), blk_stride, tok_stride, k0, v0);
+      st.load(kbase, vbase, phys(1), blk_stride, tok_stride, k1, v1);
+      st.load(kbase, vbase, phys(2), blk_stride, tok_stride, k2, v2);
+      for (int i = 0; i < cnt; i += 4) {
+        if (sync_mask >= 0 && (i & sync_mask) == 0) __builtin_amdgcn_s_barrier();
+        st.load(kbase, vbase, phys(i + 3), blk_stride, tok_stride, k3, v3);
+        __builtin_amdgcn_sched_barrier(0);
+        visit(k0, v0, i);
+        st.load(kbase, vbase, phys(i + 4), blk_stride, tok_stride, k0, v0);
+        __builtin_amdgcn_sched_barrier(0);
+        visit(k1, v1, i + 1);
+        st.load(kbase, vbase, phys(i + 5), blk_stride, tok_stride, k1, v1);
+        __builtin_amdgcn_sched_barrier(0);
+        visit(k2, v2, i + 2);
+        st.load(kbase, vbase, phys(i + 6), blk_stride, tok_stride, k2, v2);
+        __builtin_amdgcn_sched_barrier(0);
+        visit(k3, v3, i + 3);
+      }
+    }
+  }
+  if (cur >= 0) finish(cur);
+}
+
 // Merge the pieces of every sequence that spans several workgroup ranges
 // (same flattened split as the persistent kernel), together with its
 // shared-prefix partials if it has any; write zeros for a sequence with no
@@ -1901,8 +2011,8 @@ static void launch_persistent(const void* q, int64_t q_stride, const void* kc, c
       // shared prefixes first: their partials are read by the two kernels below
       const ChunkArgs<T> ca{(const T*)q, q_stride, (const T*)kc, (const T*)vc, num_kv_heads,
                             num_cache_blocks, bt, max_blocks, nullptr, ctx, 0, 1, num_seqs,
-                            scale_log2, (T*)out, out_stride, pfx};
-      hipLaunchKernelGGL((attn_chunk_mfma_kernel<T, D, G, 16, 4, 1, true, 1>),
+                            scale_log2, (T*)out, out_stride, pfx, KeySplit{1, 0, nullptr, nullptr}};
+      hipLaunchKernelGGL((attn_chunk_mfma_kernel<T, D, G, 16, 4, 1, true, 1, false>),
                          dim3((unsigned)(pfx.max_items * num_kv_heads)), dim3(256), 0, st, ca);
     }
   }
@@ -2024,25 +2134,39 @@ static int dispatch(lv_dtype dt, int D, int G, int BS, const LaunchArgs& a, cons
   }
 }
 
-template <typename T, int D, int G, int HK>
+static int64_t chunk_units(int groups, int nq) {   // the XCD-ordered grid
+  return (int64_t)((groups + kXcds - 1) / kXcds) * kXcds * nq;
+}
+
+template <typename T, int D, int G, int HK, bool KS>
 static void launch_chunk_kernel_h(const LaunchArgs& a, const int32_t* cu, int seq_begin,
-                                  int groups, int nq) {
-  const int64_t wgs = (int64_t)((groups + kXcds - 1) / kXcds) * kXcds * nq;
+                                  int groups, int nq, const KeySplit& ks) {
+  const int64_t wgs = chunk_units(groups, nq);
   const ChunkArgs<T> ca{(const T*)a.q, a.q_stride, (const T*)a.kc, (const T*)a.vc,
                         a.num_kv_heads, a.num_cache_blocks, a.bt, a.max_blocks, cu, a.ctx,
                         seq_begin, nq, groups, a.scale_log2, (T*)a.out, a.out_stride,
-                        PrefixArgs{}};
-  hipLaunchKernelGGL((attn_chunk_mfma_kernel<T, D, G, 16, 4, 1, false, HK>), dim3((unsigned)wgs),
-                     dim3(256), 0, a.st, ca);
+                        PrefixArgs{}, ks};
+  hipLaunchKernelGGL((attn_chunk_mfma_kernel<T, D, G, 16, 4, 1, false, HK, KS>),
+                     dim3((unsigned)(wgs * ks.nsplit)), dim3(256), 0, a.st, ca);
+  if constexpr (KS)
+    hipLaunchKernelGGL((attn_chunk_merge_kernel<T, D, G, 16>), dim3((unsigned)wgs, D / 16),
+                       dim3(256), 0, a.st, ca);
 }
 
-// Chunk workgroups: 4 wavefronts, 64-key tiles, two workgroups per CU, 128
-// (query token, head) rows or, split tiles, 64.
-template <typename T, int D, int G>
-static void launch_chunk_kernel(const LaunchArgs& a, const int32_t* cu, int seq_begin, int n_seqs,
-                                int max_query_len) {
-  const int groups = a.num_kv_heads * n_seqs;
-  const int nq = (max_query_len + 128 / G - 1) / (128 / G);
+// How the chunk rows of a call are cut: 64-row workgroups with split tiles
+// (else 128 rows), and into how many key ranges at most.
+struct ChunkPlan {
+  bool half;
+  int nsplit;
+  int64_t units;
+  size_t ml_bytes, acc_bytes;
+};
+
+static ChunkPlan plan_chunks(int n_seqs, int num_kv_heads, int G, int head_dim, int block_size,
+                             int max_blocks, int max_query_len) {
+  ChunkPlan p{};
+  const int64_t groups = (int64_t)num_kv_heads * n_seqs;
+  const int cus = device_cu_count();
   // Split tiles while 128-row workgroups would leave half the slots (two per
   // CU) empty: 64 rows each, every wavefront with half the dependent chain
   // (K Q^T, softmax, P V) per tile.  Calls as graph replays, 128-row / split
@@ -2050,22 +2174,60 @@ static void launch_chunk_kernel(const LaunchArgs& a, const int32_t* cu, int seq_
   // 16.8 us, of 2000 (256) 43.3 / 35.5, 6 chunks of 512 at up to 3000 (384)
   // 76.6 / 68.9; 8 chunks (512) 87.3 / 87.4, 15 chunks (960) 146 / 157.
   // Four tiles in flight, or 128-key tiles over eight wavefronts, were slower
-  // but for a few workgroups on long contexts.
-  if ((int64_t)groups * nq * 2 <= 3 * (int64_t)device_cu_count())
-    launch_chunk_kernel_h<T, D, G, 2>(a, cu, seq_begin, groups,
-                                      (max_query_len + 64 / G - 1) / (64 / G));
-  else
-    launch_chunk_kernel_h<T, D, G, 1>(a, cu, seq_begin, groups, nq);
+  // but for a few workgroups on long contexts (next rule).
+  p.half = groups * ((max_query_len + 128 / G - 1) / (128 / G)) * 2 <= 3 * (int64_t)cus;
+  p.nsplit = 1;
+  if (!p.half || groups > 0x7fffffff) return p;
+  p.units = chunk_units((int)groups, (max_query_len + 64 / G - 1) / (64 / G));
+  const int tiles = (int)std::min<int64_t>((int64_t)max_blocks * block_size / 64, 1 << 20);
+  // Key ranges while even those workgroups fill an eighth of the slots, and the
+  // table is wide enough for contexts of 16 tiles.  Unsplit / split: 20 tokens
+  // at 3000 (2 kv heads, 8 query heads each) 41.2 / 13.7 us, at 1000 18.7 /
+  // 12.6; 512 tokens (64 workgroups) at 1500 32.1 / 25.9, at 3000 50.1 / 33.0,
+  // at 16000 201 / 95.9; with 104 or more workgroups the merge costs what the
+  // shorter chains save (777 tokens in 4 ranges 16.9 / 19.1, 2 chunks of 512
+  // at up to 3000 41.4 / 42.7).
+  const int want = (int)std::min<int64_t>(16, 2 * (int64_t)cus / p.units);
+  if (want >= 8 && tiles >= 16) {
+    p.nsplit = std::min(want, std::max(1, tiles / kSplitMinTiles));
+    const size_t slots = (size_t)p.units * p.nsplit * kSplitRows;
+    p.ml_bytes = align256(slots * 2 * sizeof(float));
+    p.acc_bytes = align256(slots * head_dim * sizeof(float));
+  }
+  return p;
+}
+
+// Chunk workgroups: 4 wavefronts, 64-key tiles, two workgroups per CU.  `ws`
+// (ws_bytes of it) is scratch for key splits; without enough of it a unit's
+// keys stay in one range.
+template <typename T, int D, int G>
+static void launch_chunk_kernel(const LaunchArgs& a, const int32_t* cu, int seq_begin, int n_seqs,
+                                int max_query_len, char* ws, size_t ws_bytes) {
+  const int groups = a.num_kv_heads * n_seqs;
+  const ChunkPlan p = plan_chunks(n_seqs, a.num_kv_heads, G, D, 16, a.max_blocks, max_query_len);
+  KeySplit ks{1, 0, nullptr, nullptr};
+  if (!p.half) {
+    launch_chunk_kernel_h<T, D, G, 1, false>(a, cu, seq_begin, groups,
+                                             (max_query_len + 128 / G - 1) / (128 / G), ks);
+    return;
+  }
+  const int nq = (max_query_len + 64 / G - 1) / (64 / G);
+  if (p.nsplit > 1 && ws != nullptr && ws_bytes >= p.ml_bytes + p.acc_bytes) {
+    ks = KeySplit{p.nsplit, (int)p.units, (float*)ws, (float*)(ws + p.ml_bytes)};
+    launch_chunk_kernel_h<T, D, G, 2, true>(a, cu, seq_begin, groups, nq, ks);
+  } else {
+    launch_chunk_kernel_h<T, D, G, 2, false>(a, cu, seq_begin, groups, nq, ks);
+  }
 }
 
 template <typename T, int D>
 static int launch_chunks_g(int G, const LaunchArgs& a, const int32_t* cu, int seq_begin,
-                           int n_seqs, int max_query_len) {
+                           int n_seqs, int max_query_len, char* ws, size_t ws_bytes) {
   switch (G) {
-    case 1: launch_chunk_kernel<T, D, 1>(a, cu, seq_begin, n_seqs, max_query_len); return LV_OK;
-    case 2: launch_chunk_kernel<T, D, 2>(a, cu, seq_begin, n_seqs, max_query_len); return LV_OK;
-    case 4: launch_chunk_kernel<T, D, 4>(a, cu, seq_begin, n_seqs, max_query_len); return LV_OK;
-    case 8: launch_chunk_kernel<T, D, 8>(a, cu, seq_begin, n_seqs, max_query_len); return LV_OK;
+    case 1: launch_chunk_kernel<T, D, 1>(a, cu, seq_begin, n_seqs, max_query_len, ws, ws_bytes); return LV_OK;
+    case 2: launch_chunk_kernel<T, D, 2>(a, cu, seq_begin, n_seqs, max_query_len, ws, ws_bytes); return LV_OK;
+    case 4: launch_chunk_kernel<T, D, 4>(a, cu, seq_begin, n_seqs, max_query_len, ws, ws_bytes); return LV_OK;
+    case 8: launch_chunk_kernel<T, D, 8>(a, cu, seq_begin, n_seqs, max_query_len, ws, ws_bytes); return LV_OK;
     default:
       set_error("lv_paged_attention: num_heads/num_kv_heads=%d not in {1,2,4,8}", G);
       return LV_ERR_UNSUPPORTED;
@@ -2073,12 +2235,12 @@ static int launch_chunks_g(int G, const LaunchArgs& a, const int32_t* cu, int se
 }
 
 static int launch_chunks(lv_dtype dt, int D, int G, const LaunchArgs& a, const int32_t* cu,
-                         int seq_begin, int n_seqs, int max_query_len) {
+                         int seq_begin, int n_seqs, int max_query_len, char* ws, size_t ws_bytes) {
   if (dt == LV_BF16)
-    return D == 128 ? launch_chunks_g<bf16, 128>(G, a, cu, seq_begin, n_seqs, max_query_len)
-                    : launch_chunks_g<bf16, 64>(G, a, cu, seq_begin, n_seqs, max_query_len);
-  return D == 128 ? launch_chunks_g<f16, 128>(G, a, cu, seq_begin, n_seqs, max_query_len)
-                  : launch_chunks_g<f16, 64>(G, a, cu, seq_begin, n_seqs, max_query_len);
+    return D == 128 ? launch_chunks_g<bf16, 128>(G, a, cu, seq_begin, n_seqs, max_query_len, ws, ws_bytes)
+                    : launch_chunks_g<bf16, 64>(G, a, cu, seq_begin, n_seqs, max_query_len, ws, ws_bytes);
+  return D == 128 ? launch_chunks_g<f16, 128>(G, a, cu, seq_begin, n_seqs, max_query_len, ws, ws_bytes)
+                  : launch_chunks_g<f16, 64>(G, a, cu, seq_begin, n_seqs, max_query_len, ws, ws_bytes);
 }
 
 LV_ERROR_WORD_READER(read_errors_attention)
@@ -2100,6 +2262,25 @@ extern "C" size_t lv_paged_attention_workspace_size(int32_t num_seqs, int32_t nu
   const lv::AttnPlan b = lv::plan_decode(num_decodes, num_heads, lv::kPersistMaxWaves + 1, head_dim,
                                          block_size, max_blocks, dtype);
   return a.bytes() > b.bytes() ? a.bytes() : b.bytes();
+}
+
+extern "C" size_t lv_paged_attention_split_workspace_size(
+    int32_t num_seqs, int32_t num_decodes, int64_t num_tokens, int32_t num_heads,
+    int32_t num_kv_heads, int32_t head_dim, int32_t block_size, int32_t max_blocks,
+    int32_t max_query_len, lv_dtype dtype) {
+  using namespace lv;
+  const size_t base = lv_paged_attention_workspace_size(num_seqs, num_decodes, num_tokens,
+                                                        num_heads, head_dim, block_size,
+                                                        max_blocks, max_query_len, dtype);
+  if (num_decodes < 0 || num_seqs <= num_decodes || num_heads <= 0 || num_kv_heads <= 0 ||
+      num_heads % num_kv_heads != 0 || max_blocks <= 0 || max_query_len < 1 || block_size != 16 ||
+      (head_dim != 64 && head_dim != 128) || (dtype != LV_BF16 && dtype != LV_F16))
+    return base;
+  const int G = num_heads / num_kv_heads;
+  if (G != 1 && G != 2 && G != 4 && G != 8) return base;
+  const ChunkPlan p = plan_chunks(num_seqs - num_decodes, num_kv_heads, G, head_dim, block_size,
+                                  max_blocks, max_query_len);
+  return p.nsplit > 1 ? align256(base) + p.ml_bytes + p.acc_bytes : base;
 }
 
 static int paged_attention_impl(const void* query_dev, int64_t q_stride_t,
@@ -2175,8 +2356,17 @@ static int paged_attention_impl(const void* query_dev, int64_t q_stride_t,
       block_size == 16 && (G == 1 || G == 2 || G == 4 || G == 8) &&
       !env_is("LV_ATTN_CHUNK_KERNEL", 'r')) {
     LV_REQUIRE(max_query_len >= 1, "lv_paged_attention: max_query_len must be >= 1");
+    // scratch for key splits: what the caller gave beyond the decode rows' part
+    const size_t used = align256(pd.bytes());
+    char* ws = nullptr;
+    size_t ws_left = 0;
+    if (workspace_dev && (reinterpret_cast<uintptr_t>(workspace_dev) & 255) == 0 &&
+        workspace_bytes > used) {
+      ws = (char*)workspace_dev + used;
+      ws_left = workspace_bytes - used;
+    }
     const int rc = launch_chunks(dtype, head_dim, G, a, cu_seqlens_dev, num_decodes,
-                                 num_seqs - num_decodes, max_query_len);
+                                 num_seqs - num_decodes, max_query_len, ws, ws_left);
     if (rc != LV_OK) return rc;
   } else if (num_decodes < num_seqs) {
     // Prefill-chunk rows without an MFMA path (fp32): one row per query

@@ -63,6 +63,12 @@ SIGNATURES: dict[str, tuple] = {
         _c_p, _c_sz,                  # workspace, workspace_bytes
         ctypes.c_int, _c_p,           # dtype, stream
     ]),
+    "lv_paged_attention_split_workspace_size": (_c_sz, [
+        _c_i32, _c_i32, _c_i64,       # num_seqs, num_decodes, num_tokens
+        _c_i32, _c_i32, _c_i32,       # num_heads, num_kv_heads, head_dim
+        _c_i32, _c_i32, _c_i32,       # block_size, max_blocks, max_query_len
+        ctypes.c_int,                 # dtype
+    ]),
     "lv_paged_attention_prefix_workspace_size": (_c_sz, [_c_i32, _c_i32, _c_i32]),
     "lv_paged_attention_prefix": (ctypes.c_int, [
         _c_p, _c_i64,                 # query, q_stride_t

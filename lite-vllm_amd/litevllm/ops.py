@@ -72,7 +72,8 @@ def _native():
     """The native call module, bound to the loaded library on first use."""
     global _native_module
     if _native_module is None:
-        lib = _hip.load()
+        _hip.load()
+        lib = ctypes.CDLL(str(_hip.LIB_PATH))   # its own symbols, whoever wraps load()'s
         try:
             from . import _native as module
         except ImportError as e:
@@ -394,8 +395,13 @@ def paged_attention(query: torch.Tensor, key_cache: torch.Tensor, value_cache: t
         if workspace.dtype != torch.uint8 or not workspace.is_contiguous() or \
                 workspace.numel() < ws_bytes:
             raise RuntimeError(f"workspace must be a contiguous uint8 tensor of >= {ws_bytes} bytes")
-        ws = workspace if ws_bytes > 0 else None
+        ws = workspace if workspace.numel() > 0 else None
     else:
+        # chunk rows may use more; a graph under capture must not come to
+        # depend on the per-stream buffer for it
+        if num_decodes < B and not torch.cuda.is_current_stream_capturing():
+            ws_bytes = lib.lv_paged_attention_split_workspace_size(
+                B, num_decodes, T, H, hkv, D, bs, max_blocks, max_query_len, dt)
         ws = _workspace(dev, ws_bytes)
     if prefix is None:
         rc = lib.lv_paged_attention(

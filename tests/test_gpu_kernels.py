@@ -209,15 +209,45 @@ def test_decode_matrix_cores_one_rounding(device, dtype, heads, kind):
             assert (err <= bound).all(), (r, h, n, float((err / bound).max()))
 
 
+@torch.inference_mode()
+def test_chunks_under_capture_use_no_pooled_scratch(device):
+    """A captured chunk call keeps its keys in one range (the per-stream
+    scratch may be replaced after the capture); replays, with eager split
+    calls between them, equal the eager unsplit call."""
+    _say("chunk call under capture")
+    step = workloads.mixed_step(seed=3, num_decodes=0, num_chunks=1, chunk_len=33, off_lo=1500,
+                                off_hi=1500, num_cache_slots=16 * 300).batch.to(device)
+
+    def call(**kw):
+        return ops.paged_attention(step.query, step.key_cache, step.value_cache,
+                                   step.block_tables, step.context_lens, scale=step.scale,
+                                   cu_seqlens=step.cu_seqlens, num_decodes=0, max_query_len=33,
+                                   **kw)
+    want = call(workspace=torch.empty(0, dtype=torch.uint8, device=device))
+    split = call()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for _ in range(3):
+        out.zero_()
+        ops._workspaces.clear()
+        graph.replay()
+        again = call()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(again, split)
+    assert (split.float() - want.float()).norm() <= 2.0 ** -8 * want.float().norm()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("heads", [(16, 8, 128), (4, 2, 64), (16, 2, 128), (8, 8, 64)])
 @pytest.mark.parametrize("lens", [[(1, 0), (2, 700)], [(31, 33), (32, 0), (33, 31)],
                                   [(63, 1), (64, 64), (65, 0), (129, 900)], [(5, 4200)],
-                                  "full"])
+                                  [(64, 960)], [(65, 1100), (3, 2300), (1, 0)], "full"])
 def test_chunks_of_few_workgroups(device, dtype, heads, lens):
     """Chunks whose grid leaves the chip idle run on split key tiles (two
-    wavefronts share 32 rows, 32 keys of each tile apiece), fuller grids on
-    whole ones: lengths around a tile, rows with all keys in the first half of
+    wavefronts share 32 rows, 32 keys of each tile apiece), the emptiest with
+    their keys in several ranges where scratch allows, fuller grids on whole
+    tiles: lengths around a tile, rows with all keys in the first half of
     a tile, more than 64 tiles, NaN past the context.  Weights and outputs
     are rounded to 16 bits once each: 1.5 units in the last place of the
     largest |value| a row can see, and 2^-8 (2^-11) relative L2."""
@@ -247,6 +277,12 @@ def test_chunks_of_few_workgroups(device, dtype, heads, lens):
                               max_query_len=max(q for q, _ in lens)).float().cpu()
     ref = oatt.mixed_attention(query, kc, vc, bt, cu, ctx, scale)
     ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    # no scratch beyond what the call must have: keys in one range
+    whole = ops.paged_attention(*(t.to(device) for t in (query, kc, vc, bt, ctx)), scale=scale,
+                                cu_seqlens=cu.to(device), num_decodes=0,
+                                max_query_len=max(q for q, _ in lens),
+                                workspace=torch.empty(0, dtype=torch.uint8, device=device))
+    assert (whole.float().cpu() - ref).norm() <= ulp * ref.norm()
     assert torch.isfinite(got).all()
     assert (got - ref).norm() <= ulp * ref.norm()
     assert (got - ref).abs().max() <= 1.5 * ulp * float(vc.nan_to_num(0).abs().max())
