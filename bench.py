@@ -174,7 +174,7 @@ def bench_decode(args):
             "workload": "config2 paged decode attention: 256 seqs, ctx U[128,2048] (seed 0), "
                         "16 q / 8 kv heads, head_dim 128, block_size 16, bf16 in / fp32 accumulate",
             "num_seqs": 256, "sum_ctx": int(cpu_batch.context_lens.sum()),
-            "kernel": "lv_paged_attention (attn_decode_persistent_kernel + "
+            "kernel": "lv_paged_attention (attn_decode_mfma_kernel + "
                       "attn_persist_reduce_kernel)",
         },
         "roofline": {
@@ -447,7 +447,7 @@ def mixed_kernel_rooflines(steps: int = 20, warmup: int = 5):
                       "avg_launch_us": round(us["chunks"], 2), "timing": in_step},
          "config": wl},
         {"metric": "paged-decode attn HBM GB/s (config 3 decode rows)",
-         "kernel": "lv_paged_attention decode rows (attn_decode_persistent_kernel + "
+         "kernel": "lv_paged_attention decode rows (attn_decode_mfma_kernel + "
                    "attn_persist_reduce_kernel)",
          "value": round(dec_bytes / (us["decodes"] * 1e-6) / 1e9, 1), "unit": "GB/s",
          "roofline": hbm(dec_bytes, us["decodes"], us["decodes"], in_step,
@@ -462,7 +462,9 @@ def bench_e2e(args):
     time.  The decode-attention launches of decode-only steps are bracketed
     by HIP events on the launch stream for the roofline."""
     import torch
-    from litevllm import LLM, SamplingParams, _hip, workloads
+    import types
+
+    from litevllm import LLM, SamplingParams, _hip, ops, workloads
     from litevllm.engine import model_runner as mr
 
     mc = workloads.QWEN3_06B_SHAPE
@@ -612,6 +614,11 @@ def bench_e2e(args):
     mr.ModelRunner.execute_model = exec_probe
     for n in orig_c:
         setattr(lib, n, c_probe(n))
+    # the probes sit on the ctypes symbols: attention calls go through them
+    native = ops._native()
+    ops._native_module = types.SimpleNamespace(
+        **{n: getattr(native, n) for n in dir(native) if not n.startswith("_")})
+    ops._native_module.paged_attention = lambda *a: None
     mr.DecodeGraphs.accepts = accepts_probe
     llm = LLM("qwen3-0.6b-shape", dtype="bfloat16", load_format="dummy", hf_overrides=mc,
               skip_tokenizer_init=True, enable_prefix_caching=True, max_num_batched_tokens=8192,
@@ -651,6 +658,7 @@ def bench_e2e(args):
     mr.ModelRunner.execute_model = orig_exec
     for n, fn in orig_c.items():
         setattr(lib, n, fn)
+    ops._native_module = native
     mr.DecodeGraphs.accepts = orig_accepts
     durs = [a.elapsed_time(b) for a, b in probe["durs"]]
     if args.no_graph_timing:          # (keeps a kernel trace of this run to the serving run)
@@ -688,7 +696,7 @@ def bench_e2e(args):
             "output_tokens": n_out, "prefix_hit_tokens": eng.prefix_cache.hit_tokens - hits0,
             "num_gpu_blocks": eng.config.cache_config.num_gpu_blocks,
             "kernel": "lv_paged_attention_prefix decode (shared-prefix pass "
-                      "attn_chunk_mfma_kernel<PFX> + attn_decode_persistent_kernel + "
+                      "attn_chunk_mfma_kernel<PFX> + attn_decode_mfma_kernel + "
                       "attn_persist_reduce_kernel), decode-only steps",
             "decode_graphs": not args.eager,
             "roofline_sample": ("every decode-only step" if args.eager else

@@ -24,6 +24,11 @@ import statistics
 from pathlib import Path
 
 
+def _is_decode(name: str) -> bool:
+    """The kernel that walks the decode rows' blocks (matrix-core or vector form)."""
+    return "attn_decode_mfma_kernel" in name or "attn_decode_persistent_kernel" in name
+
+
 def _rows(db: str) -> list[tuple[str, int, int]]:
     cur = sqlite3.connect(db).cursor()
     return cur.execute("select name, start, end from kernels order by start").fetchall()
@@ -89,7 +94,7 @@ def _decode_only(rows) -> dict:
     acc: dict[str, list[int]] = {}
     for st in keep:
         for n, d in st:
-            if "attn_decode_persistent_kernel" in n or "attn_persist_reduce_kernel" in n:
+            if _is_decode(n) or "attn_persist_reduce" in n:
                 acc.setdefault(_short(n, 80), []).append(d)
     if not acc:
         return {}
@@ -125,9 +130,9 @@ def summarize_counters(pmc_dir: str) -> str:
     if cur:
         steps.append(cur)
     def is_prefix_pass(n: str) -> bool:
-        # attn_chunk_mfma_kernel<T, D, G, BS, W, BPW, true> (names may carry
-        # the argument list after the template arguments)
-        return re.search(r"attn_chunk_mfma_kernel<[^<>]*,\s*true>", n) is not None
+        # attn_chunk_mfma_kernel<T, D, G, BS, W, BPW, true, HK, KS> (names may
+        # carry the argument list after the template arguments)
+        return re.search(r"attn_chunk_mfma_kernel<[^<>]*,\s*true,\s*\d+,\s*\w+>", n) is not None
 
     def is_chunk(n: str) -> bool:
         return "attn_chunk_mfma_kernel" in n and not is_prefix_pass(n)
@@ -140,14 +145,12 @@ def summarize_counters(pmc_dir: str) -> str:
             continue
         acc, walked = None, False
         for n, vals in st:
-            if is_prefix_pass(n) or ("attn_decode_persistent_kernel" in n and walked) or \
-                    ("attn_decode_persistent_kernel" in n and acc is None):
+            if is_prefix_pass(n) or (_is_decode(n) and (walked or acc is None)):
                 if acc is not None:
                     pairs.append(acc)
-                acc, walked = dict(vals), "attn_decode_persistent_kernel" in n
-            elif acc is not None and ("attn_decode_persistent_kernel" in n
-                                      or "attn_persist_reduce_kernel" in n):
-                walked = walked or "attn_decode_persistent_kernel" in n
+                acc, walked = dict(vals), _is_decode(n)
+            elif acc is not None and (_is_decode(n) or "attn_persist_reduce" in n):
+                walked = walked or _is_decode(n)
                 for c, v in vals.items():
                     acc[c] = acc.get(c, 0.0) + v
         if acc is not None:
