@@ -58,21 +58,6 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
 
-// 16 bytes per lane from global memory into LDS at wave base + 16 lane
-// (global_load_lds_dwordx4), issued from inline assembly so that the
-// compiler does not track it: its own tracking of loads into LDS across the
-// staging loop's back edge waits for all of them before the first LDS read
-// of each iteration.  The loads a batch needs are waited for with
-// wait_vmcnt before that batch's barrier.
-// lds_wave_base is an LDS byte address, the same in every lane.  M0 is
-// written here and nowhere else in this file's kernels (no other
-// instruction of theirs reads it).
-__device__ __forceinline__ void load_lds16_async(const void* g, uint32_t lds_wave_base) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g),
-               "s"(lds_wave_base)
-               : "memory", "m0");
-}
-
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }

@@ -77,24 +77,38 @@ template <> struct Mfma16<f16> {
   __device__ __forceinline__ static uint16_t head_bits(float x) { return float_to_f16_bits(x); }
 };
 
-// 16 bytes per lane from global memory (base + the lane's byte offset) into
-// LDS at byte address lds + 16 lane, issued from inline assembly: the
-// compiler does not track it, so nothing waits for it but wait_vmcnt.
-// lds and base are the same in every lane.  Kernels that use this read M0
-// nowhere else.
-__device__ __forceinline__ void load_lds16_stream(uint64_t base, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, %2 nt" ::"v"(offset), "s"(lds),
-               "s"(base)
-               : "memory", "m0");
+// 16 bytes per lane from global memory into LDS at byte address lds + 16 lane
+// (global_load_lds_dwordx4), issued from inline assembly: the compiler does
+// not track it, so nothing waits for it but a wait on the vector-memory count
+// (its own tracking of loads into LDS would wait for all of them before the
+// first LDS read of a loop's next iteration).  lds is the same in every lane.
+// The load takes its LDS address from M0.  The hardware needs one wait state
+// between a scalar write of M0 and a load that reads it, and the compiler's
+// hazard pass does not look into inline assembly: s_nop 0 is that state.  M0
+// is not on the clobber lists: the compiler allocates no value to it and
+// writes it itself only ahead of instructions of its own that read it
+// (load_lds16 below), so a kernel uses either these loads or load_lds16.
+#define LV_SET_M0(ARG) "s_mov_b32 m0, " ARG "\n\ts_nop 0\n\t"
+// Any address per lane.
+__device__ __forceinline__ void load_lds16_async(const void* g, uint32_t lds) {
+  asm volatile(LV_SET_M0("%1") "global_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds) : "memory");
 }
+// base (the same in every lane) + the lane's byte offset; read once, so not
+// kept in the caches.
+__device__ __forceinline__ void load_lds16_stream(uint64_t base, uint32_t offset, uint32_t lds) {
+  asm volatile(LV_SET_M0("%1") "global_load_lds_dwordx4 %0, %2 nt" ::"v"(offset), "s"(lds),
+               "s"(base)
+               : "memory");
+}
+#undef LV_SET_M0
 
 // Waits until at most N of the wavefront's vector-memory operations are
-// outstanding (they complete in order) (wait_lds: until
-// its LDS operations are done).
+// outstanding; loads complete in order.
 template <int N>
 __device__ __forceinline__ void wait_vmem() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
+// Waits until all of the wavefront's LDS operations are done.
 __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // 16 bytes per lane from global memory straight into LDS at wave base + 16 lane.

@@ -66,7 +66,17 @@ def _compile(src: Path, hipcc: str) -> Path:
             f"hipcc failed for {src.name} (exit {proc.returncode}):\n{' '.join(cmd)}\n"
             f"{proc.stdout}\n{proc.stderr}"
         )
+    _print_warnings(src, proc.stderr)
     return obj
+
+
+def _print_warnings(src: Path, stderr: str) -> None:
+    """The compiler's messages, but for the host pass's that it does not know
+    the device-only target feature."""
+    text = [line for line in stderr.splitlines()
+            if "packed-fp32-ops" not in line and line.strip()]
+    if text:
+        print(f"[litevllm] {src.name}:", *text, sep="\n", file=sys.stderr)
 
 
 def _build_native() -> Path:
@@ -88,6 +98,7 @@ def _build_native() -> Path:
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"g++ failed for {src.name}:\n{' '.join(cmd)}\n{proc.stderr}")
+    _print_warnings(src, proc.stderr)
     os.replace(tmp, out)
     return out
 
