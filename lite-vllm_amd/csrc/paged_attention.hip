@@ -579,7 +579,9 @@ struct MergeState {
 //     element type in three columns of the same product (G = 8: the third
 //     in a second product), so O sums the fp32 weights' products in fp32.
 // Column c of a tile is head c % G, part c / G of P (parts past the third
-// are zero).
+// are zero).  An infinite V makes NaN of every zero among them, so a sum that
+// is not finite is taken from the leading part's column, whose weights are
+// not zero, alone (finish).
 //
 // LDS row r of a block holds its 16-byte chunk j at j ^ swz(r); the token of
 // tile row 4 g + e is 4 perm(g) + e, perm = 0 2 1 3.  With D = 128 swz is
@@ -707,6 +709,7 @@ __global__ __launch_bounds__(kPersistMaxWaves * 64) void attn_decode_mfma_kernel
 
   uint4 qf[QS];
   f32x4_t o[NB];
+  f32x4_t o2[G == 8 ? NB : 1];               // the third part's sums, if it has its own product
   float m = kNegBig, l = 0.0f;
   int cur = -1, cur_end = 0, cur_skip = 0;   // as in the kernel above
 
@@ -718,7 +721,10 @@ __global__ __launch_bounds__(kPersistMaxWaves * 64) void attn_decode_mfma_kernel
 #pragma unroll
     for (int s = 0; s < QS; ++s) qf[s] = load16(qp + 32 * s);
 #pragma unroll
-    for (int b = 0; b < NB; ++b) o[b] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int b = 0; b < NB; ++b) {
+      o[b] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      if constexpr (G == 8) o2[b] = o[b];
+    }
     m = kNegBig;
     l = 0.0f;
   };
@@ -759,17 +765,43 @@ __global__ __launch_bounds__(kPersistMaxWaves * 64) void attn_decode_mfma_kernel
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) o[b][e] *= alpha;
+          for (int e = 0; e < 4; ++e) {
+            o[b][e] *= alpha;
+            if constexpr (G == 8) o2[b][e] *= alpha;
+          }
+      }
+    }
+    float p[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool in = !(left < BS && tok0 + e >= left);
+      p[e] = in ? fast_exp2(x[e] - m) : 0.0f;
+      l += p[e];
+    }
+    if constexpr (std::is_same<T, f16>::value) {
+      // A weight under 2^-25 has no leading part in fp16.  In a block that
+      // holds a value that is not finite such weights are raised to 2^-24
+      // (2^-34 of the row's largest) to keep the leading part's column right.
+      if (__ballot(fminf(fminf(p[0], p[1]), fminf(p[2], p[3])) < 0x1p-25f)) {
+        uint32_t top = 0;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const uint2 w = __builtin_bit_cast(uint2, vf[b]);
+          top |= (w.x & 0x7c007c00u) + 0x04000400u;   // bits 15, 31: exponents all ones
+          top |= (w.y & 0x7c007c00u) + 0x04000400u;
+        }
+        if (__ballot((top & 0x80008000u) != 0)) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (p[e] > 0.0f) p[e] = fmaxf(p[e], 0x1p-24f);
+        }
       }
     }
     uint16_t w0[4], w1[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const bool in = !(left < BS && tok0 + e >= left);
-      const float p = in ? fast_exp2(x[e] - m) : 0.0f;
-      l += p;
-      const float r1 = p - M::head(p), r2 = r1 - M::head(r1);
-      const uint16_t b0 = M::head_bits(p), b1 = M::head_bits(r1), b2 = M::head_bits(r2);
+      const float r1 = p[e] - M::head(p[e]), r2 = r1 - M::head(r1);
+      const uint16_t b0 = M::head_bits(p[e]), b1 = M::head_bits(r1), b2 = M::head_bits(r2);
       w0[e] = part == 0 ? b0 : part == 1 ? b1 : part == 2 ? b2 : (uint16_t)0;
       w1[e] = part == 0 ? b2 : (uint16_t)0;
     }
@@ -779,7 +811,7 @@ __global__ __launch_bounds__(kPersistMaxWaves * 64) void attn_decode_mfma_kernel
     if constexpr (G == 8) {
       const i16x4_t p1 = {(short)w1[0], (short)w1[1], (short)w1[2], (short)w1[3]};
 #pragma unroll
-      for (int b = 0; b < NB; ++b) o[b] = M::run16(vf[b], p1, o[b]);
+      for (int b = 0; b < NB; ++b) o2[b] = M::run16(vf[b], p1, o2[b]);
     }
   };
 
@@ -792,6 +824,27 @@ __global__ __launch_bounds__(kPersistMaxWaves * 64) void attn_decode_mfma_kernel
     const int hq = kvh * G + head;
     float L = l + __shfl_xor(l, 16);
     L = xor32_sum(L);
+    float all = 0.0f;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        all += o[b][e];
+        if constexpr (G == 8) all += o2[b][e];
+      }
+    if (__ballot(!(fabsf(all) < __builtin_inff()))) {   // uniform, rare
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (!(fabsf(__shfl(o[b][e], (lane & 48) | head)) < __builtin_inff())) {
+            if (part != 0) o[b][e] = 0.0f;
+            if constexpr (G == 8) o2[b][e] = 0.0f;
+          }
+    }
+    if constexpr (G == 8)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) o[b] += o2[b];
     if (whole && cur_skip > 0) {
       const int nsplit = (cur_skip * BS + kPrefixKeysPerSplit - 1) / kPrefixKeysPerSplit;
       const int64_t pb = ((int64_t)sq * H + hq) * kPrefixMaxSplits;
@@ -874,7 +927,8 @@ struct MergeSource {
   int sq, np, nsplit, g0, num_seqs, num_heads, hq;
 
   // Entries i, i + step, ... (U of them); those past the last count nothing
-  // (m = kNegBig, l = 0; the loads re-read the last).
+  // (m = kNegBig, l = 0, values 0: the loads re-read the last, which may be
+  // infinite).
   template <int D, int U>
   __device__ __forceinline__ void load(int i, int step, int d, float2 (&ml)[U],
                                        float4 (&v)[U]) const {
@@ -897,7 +951,10 @@ struct MergeSource {
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (i + u * step >= np + nsplit) ml[u] = make_float2(kNegBig, 0.0f);
+      if (i + u * step >= np + nsplit) {
+        ml[u] = make_float2(kNegBig, 0.0f);
+        v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      }
   }
 };
 
@@ -1510,7 +1567,10 @@ __global__ __launch_bounds__(256) void attn_chunk_merge_kernel(ChunkArgs<T> a) {
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      if (i + j >= n) ml[j] = make_float2(kNegBig, 0.0f);
+      if (i + j >= n) {                // (the last again, which may be infinite)
+        ml[j] = make_float2(kNegBig, 0.0f);
+        v[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      }
     st.add(ml, v);
   }
   const float inv = st.l > 0.0f ? 1.0f / st.l : 0.0f;

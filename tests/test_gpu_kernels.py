@@ -209,6 +209,78 @@ def test_decode_matrix_cores_one_rounding(device, dtype, heads, kind):
             assert (err <= bound).all(), (r, h, n, float((err / bound).max()))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("heads", [(16, 8, 128), (8, 8, 64), (16, 4, 64), (16, 2, 128)])
+@pytest.mark.parametrize("kind", ["few rows", "many rows", "prefix", "chunks"])
+def test_infinite_values(device, dtype, heads, kind):
+    """An infinite V element the row can see makes its own dim of the row
+    infinite (NaN where both signs meet) and touches no other dim: decode rows
+    of one and of many pieces, rows with a shared prefix, and chunk rows in one
+    and in several key ranges, each with a weight far below the row's largest
+    among the infinite tokens (fp16 decode: under 2^-40)."""
+    H, Hkv, D = heads
+    G = H // Hkv
+    _say(f"infinite values {dtype} {heads} {kind}")
+    if kind == "chunks":
+        batch = workloads.mixed_step(seed=5, num_decodes=0, num_chunks=1, chunk_len=20,
+                                     off_lo=1500, off_hi=1500, num_heads=H, num_kv_heads=Hkv,
+                                     head_dim=D, num_cache_slots=16 * 400, dtype=dtype).batch
+    else:
+        batch = workloads.paged_decode(seed=6, num_seqs=300 if kind == "many rows" else 5,
+                                       num_heads=H, num_kv_heads=Hkv, head_dim=D, ctx_lo=90,
+                                       ctx_hi=400, dtype=dtype, scale_inputs=False,
+                                       ctx_head=[3000, 100, 97])
+    plan = None
+    if kind == "prefix":
+        batch.block_tables[1:3, :4] = batch.block_tables[0, :4]
+        plan = ops.prefix_plan([([0, 1, 2], 4)], 5, G, device) if dtype != torch.float32 else None
+
+    def call():
+        b = batch.to(device)
+        cu = dict(cu_seqlens=b.cu_seqlens, max_query_len=b.max_query_len) if kind == "chunks" else {}
+        return ops.paged_attention(b.query, b.key_cache, b.value_cache, b.block_tables,
+                                   b.context_lens, scale=b.scale, num_decodes=b.num_decodes,
+                                   prefix=plan, **cu).float().cpu()
+    want = call()
+    assert torch.isfinite(want).all()
+    bt, kc, vc = batch.block_tables, batch.key_cache, batch.value_cache
+    inf = float("inf")
+    for r in range(bt.shape[0]):
+        if kind == "prefix" and r == 0:
+            continue                       # (its first blocks are the others' too)
+        n = int(batch.context_lens[r]) - (19 if kind == "chunks" else 0)
+        b0, b1, b2 = (int(bt[r, t // 16]) for t in (70, n - 1, 81))
+        vc[b0, 70 % 16, :, 3] = inf
+        vc[b1, (n - 1) % 16, :, 5] = -inf
+        vc[b0, 70 % 16, 0, 7] = -inf
+        vc[b1, (n - 1) % 16, 0, 7] = inf
+        if kind not in ("chunks", "prefix"):
+            # a token of little weight: its key against the row's first query head
+            q = batch.query[r].float().view(Hkv, G, D).sum(1)
+            kc[b2, 81 % 16] = (-q * 40 / q.square().sum(-1, keepdim=True).sqrt()).to(dtype)
+            vc[b2, 81 % 16, :, 9] = inf
+    want = want if kind in ("chunks", "prefix") else None
+    got = call()
+    if want is None:                       # the same keys with finite values
+        vc.nan_to_num_(0.0, 0.0, 0.0)
+        want = call()
+    rows = slice(1, None) if kind == "prefix" else slice(None)
+    got, want = got[rows], want[rows]
+    assert (got[:, :, 3] == inf).all() and (got[:, :, 5] == -inf).all()
+    assert got[:, :G, 7].isnan().all()
+    special = torch.zeros(D, dtype=torch.bool)
+    special[[3, 5]] = True
+    if kind not in ("chunks", "prefix"):
+        assert (got[:, :, 9] == inf).all()
+        special[9] = True
+    special = special.expand(H, D).clone()
+    special[:G, 7] = True
+    # other dims: the same weights and values, so one rounding of the output apart
+    a, b = got[:, ~special], want[:, ~special]
+    assert torch.isfinite(a).all()
+    assert (a - b).norm() <= 2.0 ** -8 * b.norm()
+
+
 @torch.inference_mode()
 def test_chunks_under_capture_use_no_pooled_scratch(device):
     """A captured chunk call keeps its keys in one range (the per-stream
