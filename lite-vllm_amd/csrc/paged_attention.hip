@@ -1278,7 +1278,11 @@ __device__ __forceinline__ void chunk_mfma_body(const ChunkArgs<T>& A, int unit,
   // maximum m_run moves only when a row's maximum exceeds it by more than
   // 2^8 (or on the first tile), so probabilities stay below 256 and the O
   // rescale is rare.  Returns the factor O must be scaled by (1 = none).
-  auto soft = [&](const f32x16_t* sv, uint32_t (*pw)[8]) {
+  // HK = 2: a row may have all of this wavefront's keys of a tile masked; its
+  // maximum then stays and its weights are 0.
+  auto soft = [&](auto MaskT, const f32x16_t* sv, uint32_t (*pw)[8], int k0) {
+    bool seen = true;
+    if constexpr (HK == 2 && decltype(MaskT)::value) seen = lim >= k0 + 32 * kh;
     float mx = kNegBig;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
@@ -1286,13 +1290,11 @@ __device__ __forceinline__ void chunk_mfma_body(const ChunkArgs<T>& A, int unit,
       for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sv[kb][i]);
     mx = xor32_max(mx) * scale_log2;
     float alpha = 1.0f;
-    // HK = 2: while every key of a row has been masked in this wavefront's
-    // halves, m_run stays kNegBig and the weights are 0
-    if (mx > m_run + 8.0f && (HK == 1 || mx > kNegBig * 0.01f)) {
+    if (mx > m_run + 8.0f && seen) {
       alpha = fast_exp2(m_run - mx);
       m_run = mx;
     }
-    const float m_ref = HK == 2 && m_run == kNegBig ? 0.0f : m_run;
+    const float m_ref = seen ? m_run : 0.0f;
     float psum = 0.0f;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
@@ -1344,7 +1346,7 @@ __device__ __forceinline__ void chunk_mfma_body(const ChunkArgs<T>& A, int unit,
       uint32_t pw[2][8];
       qk(kb_lds, sv);
       mask(MaskT, sv, k0);
-      rescale(soft(sv, pw));
+      rescale(soft(MaskT, sv, pw, k0));
       pv(vb_lds, pw);
     } else {
       f32x16_t s0[2], s1[2];
@@ -1353,9 +1355,9 @@ __device__ __forceinline__ void chunk_mfma_body(const ChunkArgs<T>& A, int unit,
       mask(MaskT, s0, k0);
       qk(kb_lds + 64 * D, s1);
       mask(MaskT, s1, k0 + 64);
-      rescale(soft(s0, p0));
+      rescale(soft(MaskT, s0, p0, k0));
       pv(vb_lds, p0);
-      rescale(soft(s1, p1));
+      rescale(soft(MaskT, s1, p1, k0 + 64));
       pv(vb_lds + 64 * D, p1);
     }
   };

@@ -281,6 +281,29 @@ def test_infinite_values(device, dtype, heads, kind):
     assert (a - b).norm() <= 2.0 ** -8 * b.norm()
 
 
+@pytest.mark.parametrize("chunk,off", [(70, 0), (20, 1500)])
+def test_chunk_scores_of_any_finite_size(device, chunk, off):
+    """Split tiles tell a masked key by its position, not by its score: with
+    every score -2^99 (and a scale that is 1/8 in log2 units, so its products
+    are exact) a row's output is the mean of the values it sees."""
+    _say(f"chunk scores of -2^99, {chunk} tokens at {off}")
+    batch = workloads.mixed_step(seed=5, num_decodes=0, num_chunks=1, chunk_len=chunk, off_lo=off,
+                                 off_hi=off, num_cache_slots=16 * 400).batch
+    batch.query.fill_(2.0 ** 49)
+    batch.key_cache.fill_(-2.0 ** 43)
+    log2e = np.float32(1.4426950408889634)
+    scale = np.float32(0.125) / log2e
+    assert scale * log2e == np.float32(0.125)
+    b = batch.to(device)
+    got = ops.paged_attention(b.query, b.key_cache, b.value_cache, b.block_tables, b.context_lens,
+                              scale=float(scale), cu_seqlens=b.cu_seqlens, num_decodes=0,
+                              max_query_len=chunk).float().cpu()
+    v = oatt.gather_sequence(batch.value_cache, batch.block_tables[0], chunk + off).float()
+    mean = v.cumsum(0)[off:] / torch.arange(off + 1, off + chunk + 1)[:, None, None]
+    want = mean.repeat_interleave(2, 1)
+    assert (got - want).norm() <= 2.0 ** -8 * want.norm()
+
+
 @torch.inference_mode()
 def test_chunks_under_capture_use_no_pooled_scratch(device):
     """A captured chunk call keeps its keys in one range (the per-stream
