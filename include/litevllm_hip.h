@@ -201,7 +201,8 @@ size_t lv_paged_attention_workspace_size(int32_t num_seqs, int32_t num_decodes,
 /* lv_paged_attention_workspace_size plus what lets the prefill-chunk rows of
  * such a call split their keys over more workgroups (few chunks at long
  * offsets leave most of the GPU idle otherwise).  Optional: with less
- * workspace the chunk rows run unsplit, with results equal to fp32 rounding. */
+ * workspace the chunk rows run unsplit.  The results differ by the rounding of
+ * the softmax weights to `dtype`, which is against another running maximum. */
 size_t lv_paged_attention_split_workspace_size(int32_t num_seqs, int32_t num_decodes,
                                                int64_t num_tokens, int32_t num_heads,
                                                int32_t num_kv_heads, int32_t head_dim,

@@ -259,28 +259,29 @@ FAST(paged_attention, 14) {
   if (!ws && nd < B &&
       c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None)
     ws_bytes = api.split_ws(B, nd, T, H, hkv, D, bs, max_blocks, max_q, dt);
-  if (ws_bytes > 0 && !ws && !(ws = scratch(dev, st, ws_bytes, kind_attn))) NOT_PLAIN();
+  if (ws) ws_bytes = ws->numel();
+  else if (ws_bytes > 0 && !(ws = scratch(dev, st, ws_bytes, kind_attn))) NOT_PLAIN();
   if (pb && !pws && pws_bytes > 0 && !(pws = scratch(dev, st, pws_bytes, kind_prefix)))
     NOT_PLAIN();
   // held past the GIL's release: another thread may grow the pool's entry
   const at::Tensor ws_held = ws ? *ws : at::Tensor(), pws_held = pws ? *pws : at::Tensor();
   const at::Tensor out = given ? *given : empty(q->sizes(), *q);
   void *wp = ptr(ws), *pwp = ptr(pws);
-  const size_t wn = ws ? ws->numel() : 0, pwn = pws ? pws->numel() : 0;
+  const size_t pwn = pws ? pws->numel() : 0;
   int rc;
   Py_BEGIN_ALLOW_THREADS
   if (pb)
     rc = api.attention_prefix(ptr(q), q->stride(0), ptr(kc), ptr(vc), n_blocks,
                               (const int32_t*)ptr(bt), max_blocks, (const int32_t*)ptr(cu),
                               (const int32_t*)ptr(ctx), B, nd, T, max_q, H, hkv, D, bs,
-                              (float)scale, out.data_ptr(), out.stride(0), wp, wn,
+                              (float)scale, out.data_ptr(), out.stride(0), wp, ws_bytes,
                               (const int32_t*)ptr(pb), (const int32_t*)ptr(pi), pi->size(0),
                               (const int32_t*)ptr(pm), pm->size(0), pwp, pwn, dt, st);
   else
     rc = api.attention(ptr(q), q->stride(0), ptr(kc), ptr(vc), n_blocks, (const int32_t*)ptr(bt),
                        max_blocks, (const int32_t*)ptr(cu), (const int32_t*)ptr(ctx), B, nd, T,
-                       max_q, H, hkv, D, bs, (float)scale, out.data_ptr(), out.stride(0), wp, wn,
-                       dt, st);
+                       max_q, H, hkv, D, bs, (float)scale, out.data_ptr(), out.stride(0), wp,
+                       ws_bytes, dt, st);
   Py_END_ALLOW_THREADS
   return done(rc, pb ? "lv_paged_attention_prefix" : "lv_paged_attention", &out);
 }

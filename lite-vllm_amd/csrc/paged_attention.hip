@@ -2418,8 +2418,12 @@ static int paged_attention_impl(const void* query_dev, int64_t q_stride_t,
       block_size == 16 && (G == 1 || G == 2 || G == 4 || G == 8) &&
       !env_is("LV_ATTN_CHUNK_KERNEL", 'r')) {
     LV_REQUIRE(max_query_len >= 1, "lv_paged_attention: max_query_len must be >= 1");
-    // scratch for key splits: what the caller gave beyond the decode rows' part
-    const size_t used = align256(pd.bytes());
+    // scratch for key splits: what the caller gave beyond the plain call's
+    // (not beyond this grid's decode part, which may be less: a workspace of
+    // the plain size must not split)
+    const size_t used = align256(lv_paged_attention_workspace_size(
+        num_seqs, num_decodes, num_tokens, num_heads, head_dim, block_size, max_blocks,
+        max_query_len, dtype));
     char* ws = nullptr;
     size_t ws_left = 0;
     if (workspace_dev && (reinterpret_cast<uintptr_t>(workspace_dev) & 255) == 0 &&

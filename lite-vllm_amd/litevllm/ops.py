@@ -396,9 +396,12 @@ def paged_attention(query: torch.Tensor, key_cache: torch.Tensor, value_cache: t
                 workspace.numel() < ws_bytes:
             raise RuntimeError(f"workspace must be a contiguous uint8 tensor of >= {ws_bytes} bytes")
         ws = workspace if workspace.numel() > 0 else None
+        ws_bytes = workspace.numel()
     else:
         # chunk rows may use more; a graph under capture must not come to
-        # depend on the per-stream buffer for it
+        # depend on the per-stream buffer for it.  (The library is told of the
+        # bytes asked for, not of all that the buffer has grown to: whether the
+        # chunk rows are split depends on the call alone.)
         if num_decodes < B and not torch.cuda.is_current_stream_capturing():
             ws_bytes = lib.lv_paged_attention_split_workspace_size(
                 B, num_decodes, T, H, hkv, D, bs, max_blocks, max_query_len, dt)
@@ -408,7 +411,7 @@ def paged_attention(query: torch.Tensor, key_cache: torch.Tensor, value_cache: t
             _ptr(query), query.stride(0), _ptr(key_cache), _ptr(value_cache), n_blocks,
             _ptr(block_tables), max_blocks, _ptr(cu_seqlens), _ptr(context_lens),
             B, num_decodes, T, max_query_len, H, hkv, D, bs, float(scale),
-            _ptr(out), out.stride(0), _ptr(ws), 0 if ws is None else ws.numel(), dt,
+            _ptr(out), out.stride(0), _ptr(ws), ws_bytes, dt,
             _stream(dev))
         _hip.check(rc, "lv_paged_attention")
         return out
@@ -433,7 +436,7 @@ def paged_attention(query: torch.Tensor, key_cache: torch.Tensor, value_cache: t
         _ptr(query), query.stride(0), _ptr(key_cache), _ptr(value_cache), n_blocks,
         _ptr(block_tables), max_blocks, _ptr(cu_seqlens), _ptr(context_lens),
         B, num_decodes, T, max_query_len, H, hkv, D, bs, float(scale),
-        _ptr(out), out.stride(0), _ptr(ws), 0 if ws is None else ws.numel(),
+        _ptr(out), out.stride(0), _ptr(ws), ws_bytes,
         _ptr(prefix.blocks), _ptr(prefix.items), prefix.items.shape[0], _ptr(prefix.members),
         prefix.members.shape[0], _ptr(pws), 0 if pws is None else pws.numel(), dt, _stream(dev))
     _hip.check(rc, "lv_paged_attention_prefix")

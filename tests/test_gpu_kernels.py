@@ -11,6 +11,7 @@ from __future__ import annotations
 import json
 import math
 import sys
+import types
 from pathlib import Path
 
 import numpy as np
@@ -381,6 +382,49 @@ def test_chunks_of_few_workgroups(device, dtype, heads, lens):
     assert torch.isfinite(got).all()
     assert (got - ref).norm() <= ulp * ref.norm()
     assert (got - ref).abs().max() <= 1.5 * ulp * float(vc.nan_to_num(0).abs().max())
+
+
+@pytest.mark.parametrize("path", ["native", "python"])
+@torch.inference_mode()
+def test_mixed_batch_under_capture_does_not_split(device, path, monkeypatch):
+    """A captured mixed batch keeps its chunk's keys in one range whatever the
+    per-stream scratch has grown to, as a call with a workspace of
+    lv_paged_attention_workspace_size bytes does; with a larger one, and in
+    eager calls, it splits."""
+    _say(f"mixed batch under capture, {path}")
+    if path == "python":
+        monkeypatch.setattr(ops, "_native_module",
+                            types.SimpleNamespace(paged_attention=lambda *a: None))
+    step = workloads.mixed_step(seed=3, num_decodes=3, dec_lo=100, dec_hi=900, num_chunks=1,
+                                chunk_len=20, off_lo=3000, off_hi=3000,
+                                num_cache_slots=16 * 600).batch.to(device)
+    geom = (4, 3, 23, 16, 128, 16, step.block_tables.shape[1], 20, step.query.dtype)
+    plain = ops.paged_attention_workspace_size(*geom)
+
+    def call(nbytes=None):
+        ws = None if nbytes is None else torch.empty(nbytes, dtype=torch.uint8, device=device)
+        return ops.paged_attention(step.query, step.key_cache, step.value_cache,
+                                   step.block_tables, step.context_lens, scale=step.scale,
+                                   cu_seqlens=step.cu_seqlens, num_decodes=3, max_query_len=20,
+                                   workspace=ws)
+    want, split = call(plain), call(plain + (1 << 24))
+    assert not torch.equal(want, split)             # (another rounding of the weights)
+    assert torch.equal(call(), split)
+    ops._workspace(device, 1 << 26)                 # a pool grown by larger calls
+    assert torch.equal(call(), split)
+    graph = torch.cuda.CUDAGraph()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        pool = ops._workspace(device, 1 << 26)
+    with torch.cuda.graph(graph, stream=stream):
+        out = call()
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        again = call()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(again, split)
+    del pool
 
 
 @pytest.mark.parametrize("rows,heads", [(1, (16, 8, 128)), (3, (16, 2, 128)), (7, (8, 8, 64)),
