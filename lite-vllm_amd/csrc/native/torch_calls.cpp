@@ -15,6 +15,10 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -40,6 +44,7 @@ struct Api {
   decltype(&lv_add_rms_norm) add_rms_norm;
   decltype(&lv_qk_norm_rope_cache) qk_norm_rope_cache;
   decltype(&lv_silu_mul) silu_mul;
+  decltype(&lv_linear_supported) linear_supported;
   decltype(&lv_linear) linear;
   decltype(&lv_linear_f32) linear_f32;
 };
@@ -50,7 +55,7 @@ constexpr const char* kNames[] = {
     "lv_paged_attention_split_workspace_size", "lv_paged_attention",
     "lv_paged_attention_prefix_workspace_size", "lv_paged_attention_prefix",
     "lv_sample_workspace_size", "lv_sample", "lv_add_rms_norm", "lv_qk_norm_rope_cache",
-    "lv_silu_mul", "lv_linear", "lv_linear_f32"};
+    "lv_silu_mul", "lv_linear_supported", "lv_linear", "lv_linear_f32"};
 constexpr size_t kNumNames = sizeof(kNames) / sizeof(kNames[0]);
 static_assert(sizeof(Api) == kNumNames * sizeof(void*), "one pointer per name");
 
@@ -425,8 +430,7 @@ FAST(linear, 4) {
   return done(rc, "lv_linear", &out);
 }
 
-// (x, weight, out) -> out.  Rows off 16-byte boundaries are not plain either:
-// the layer that asks has a library product to fall back on.
+// (x, weight, out) -> out
 FAST(linear_f32, 3) {
   const at::Tensor *x = A.tensor(0), *w = A.tensor(1), *given = A.maybe(2);
   if (!A.ok || !x->is_cuda() || x->scalar_type() != at::kFloat || x->dim() != 2 || w->dim() != 2)
@@ -434,8 +438,7 @@ FAST(linear_f32, 3) {
   const at::Device dev = x->device();
   const int64_t M = x->size(0), K = x->size(1), N = w->size(0);
   if (M == 0 || !on(x, dev) || !on(w, dev) || !on(given, dev) || !is_rows(*x, K, at::kFloat) ||
-      !is_rows(*w, K, at::kFloat) || w->size(1) != K || K == 0 || K % 4 || N == 0 ||
-      x->stride(0) % 4 || w->stride(0) % 4 || ((uintptr_t)ptr(x) | (uintptr_t)ptr(w)) % 16 ||
+      !is_rows(*w, K, at::kFloat) || w->size(1) != K ||
       (given && (!is_rows(*given, N, at::kFloat) || given->size(0) != M)))
     NOT_PLAIN();
   const at::Tensor out = given ? *given : empty({M, N}, *x);
@@ -448,6 +451,68 @@ FAST(linear_f32, 3) {
   return done(rc, "lv_linear_f32", &out);
 }
 
+// No tangent of forward-mode differentiation, and nothing between the tensor
+// and the values in its storage: no transform's wrapper, lazy conjugate or
+// negation.
+bool is_direct(const at::Tensor& t) {
+  using K = at::DispatchKey;
+  static const uint64_t plain =
+      at::DispatchKeySet({K::CUDA, K::AutogradCUDA, K::AutocastCUDA, K::ADInplaceOrView}).raw_repr();
+  return (t.key_set().raw_repr() & ~plain) == 0 && !t._fw_grad(/*level=*/0).defined();
+}
+
+// Nobody but the dispatcher's CUDA kernel would see a call made now: neither
+// autograd, autocast, a trace, a transform nor a Python mode.
+bool calls_are_direct() {
+  if (at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) ||
+      at::impl::torch_function_mode_enabled() ||
+      c10::impl::TorchDispatchModeTLS::any_modes_set())
+    return false;
+  const auto tls = c10::impl::tls_local_dispatch_key_set();
+  return (tls.included_.raw_repr() & ~c10::default_included_set.raw_repr()) == 0;
+}
+
+// Rows of `width` elements, each on a 16-byte boundary and none overlapping
+// the next.
+bool is_aligned_rows(const at::Tensor& t, int64_t width, at::ScalarType type) {
+  return is_rows(t, width, type) && t.stride(0) >= width &&
+         t.stride(0) * t.element_size() % 16 == 0 && (uintptr_t)ptr(&t) % 16 == 0;
+}
+
+// (x, weight, silu_mul) -> out: nn.Linear's product for a layer that falls
+// back on nn.Linear itself, so everything the library's kernels ask for or
+// nn.Linear answers differently is not plain here.
+FAST(layer_linear, 3) {
+  const at::Tensor *x = A.tensor(0), *w = A.tensor(1);
+  const int64_t act = A.integer(2);
+  lv_dtype dt;
+  if (!A.ok || !x->is_cuda() || !dtype_of(*x, dt) || x->dim() != 2 || w->dim() != 2 ||
+      !calls_are_direct())
+    NOT_PLAIN();
+  const at::Device dev = x->device();
+  const at::ScalarType type = x->scalar_type();
+  const int64_t M = x->size(0), K = x->size(1), rows = w->size(0);
+  const bool silu = act == LV_ACT_SILU_MUL;
+  const int64_t N = silu ? rows / 2 : rows;
+  if (M == 0 || N == 0 || K == 0 || !on(x, dev) || !on(w, dev) || !is_direct(*x) ||
+      !is_direct(*w) || w->size(1) != K || (silu && rows % 2) || !is_aligned_rows(*x, K, type) ||
+      !is_aligned_rows(*w, K, type) ||
+      (dt == LV_F32 ? silu || K % 4 != 0 : !api.linear_supported(M, N, K, act, dt)))
+    NOT_PLAIN();
+  const at::Tensor out = empty({M, N}, *x);
+  void* st = stream_of(dev);
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  if (dt == LV_F32)
+    rc = api.linear_f32((const float*)ptr(x), x->stride(0), (const float*)ptr(w), w->stride(0),
+                        (float*)out.data_ptr(), out.stride(0), M, N, K, st);
+  else
+    rc = api.linear(ptr(x), x->stride(0), ptr(w), w->stride(0), out.data_ptr(), out.stride(0), M,
+                    N, K, act, dt, st);
+  Py_END_ALLOW_THREADS
+  return done(rc, dt == LV_F32 ? "lv_linear_f32" : "lv_linear", &out);
+}
+
 #define METHOD(NAME) {#NAME, (PyCFunction)(void (*)(void))NAME, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {{"bind", bind, METH_VARARGS, nullptr},
                          METHOD(kv_scatter),
@@ -458,6 +523,7 @@ PyMethodDef methods[] = {{"bind", bind, METH_VARARGS, nullptr},
                          METHOD(silu_mul),
                          METHOD(linear),
                          METHOD(linear_f32),
+                         METHOD(layer_linear),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods};
 

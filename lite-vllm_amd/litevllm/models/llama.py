@@ -19,28 +19,27 @@ from litevllm.models.base import BaseModelForCausalLM
 
 
 # Rows up to which a projection runs on lv_linear (decode-sized batches);
-# larger batches (prefill chunks) use the library GEMM.  0 disables it.
+# larger batches (prefill chunks) use the library GEMM.  0 disables it, and the
+# next two.
 DECODE_GEMM_ROWS = int(os.environ.get("LV_DECODE_GEMM_ROWS", "256"))
-# Without autograd, layers of up to SMALL_LAYER weights take lv_linear to twice
-# as many rows.  The library's call alone costs 19 us of host time against 4
+# Where nothing but the product itself would see the call (linear_if_plain),
+# layers of up to SMALL_LAYER weights take lv_linear to twice as many rows.  The library's call alone costs 19 us of host time against 4
 # (an eager step of that many tokens is bound by the host), and on the GPU the
 # two are level: 512 rows of 4096x1024 10.5 us (library 10.8), 1024x2048 8.5
 # (9.8), 1024x3072 10.6 (12.5), 6144x1024 16.5 (13.4, plus 5 for the SiLU that
 # lv_linear has in its epilogue); at 768 rows 16.5 against 12.1.
 SMALL_LAYER = 1 << 23
 # fp32 products of up to SMALL_F32 multiply-adds (k up to 1024) run on
-# lv_linear_f32, again without autograd: 4 us of host time, and 4-10 us on the
+# lv_linear_f32, under the same condition: 4 us of host time, and 4-10 us on the
 # GPU where the library takes 4-8 us on its good shapes and up to 133 on others
 # (200 rows of 256x688); 2x slower than the library past the line.
 SMALL_F32 = 1 << 27
 
 
-def _half_rows(weights: int) -> int:
-    """Rows up to which a bf16 / fp16 layer of that many weights runs on
-    lv_linear."""
-    if weights <= SMALL_LAYER and not torch.is_grad_enabled():
-        return 2 * DECODE_GEMM_ROWS
-    return DECODE_GEMM_ROWS
+def _has_forward_hooks(module: nn.Module) -> bool:
+    return bool(module._forward_hooks or module._forward_pre_hooks
+                or nn.modules.module._global_forward_hooks
+                or nn.modules.module._global_forward_pre_hooks)
 
 
 class Linear(nn.Linear):
@@ -49,20 +48,24 @@ class Linear(nn.Linear):
     MFMA kernel and whose small fp32 calls on lv_linear_f32; other shapes,
     biases and dtypes use the library GEMM."""
 
-    half_rows: Optional[int] = None     # instead of _half_rows()
+    half_on_lv_linear = True     # False: bf16 / fp16 calls use the library GEMM
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         m = x.shape[0] if x.dim() == 2 else 0
-        if m > 0 and self.bias is None and x.is_cuda:
+        if m > 0 and self.bias is None and x.is_cuda and DECODE_GEMM_ROWS > 0:
             n, k = self.out_features, self.in_features
             if x.dtype is torch.float32:
-                if m * n * k <= SMALL_F32 and k <= 1024 and not torch.is_grad_enabled():
-                    y = ops.linear_f32_if_plain(x, self.weight)
-                    if y is not None:
-                        return y
-            elif (m <= (_half_rows(n * k) if self.half_rows is None else self.half_rows)
-                    and ops.linear_supported(m, n, k, x.dtype)):
+                small = m * n * k <= SMALL_F32 and k <= 1024
+            elif not self.half_on_lv_linear:
+                small = False
+            elif m <= DECODE_GEMM_ROWS and ops.linear_supported(m, n, k, x.dtype):
                 return ops.linear(x, self.weight)
+            else:
+                small = m <= 2 * DECODE_GEMM_ROWS and n * k <= SMALL_LAYER
+            if small and not torch.is_grad_enabled():
+                y = ops.linear_if_plain(x, self.weight)
+                if y is not None:
+                    return y
         return super().forward(x)
 
 
@@ -102,11 +105,17 @@ class GatedMLP(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         m = x.shape[0] if x.dim() == 2 else 0
         up = self.gate_up_proj
-        if (0 < m <= _half_rows(up.out_features * up.in_features) and x.is_cuda and up.bias is None
+        # decode-sized: gate|up projection with SiLU * up in its epilogue
+        if (0 < m <= 2 * DECODE_GEMM_ROWS and x.is_cuda and up.bias is None
                 and ops.linear_supported(m, self.intermediate_size, up.in_features, x.dtype,
                                          "silu_mul")):
-            # decode-sized: gate|up projection with SiLU * up in its epilogue
-            return self.down_proj(ops.linear(x, up.weight, activation="silu_mul"))
+            if m <= DECODE_GEMM_ROWS:
+                return self.down_proj(ops.linear(x, up.weight, activation="silu_mul"))
+            if (up.out_features * up.in_features <= SMALL_LAYER
+                    and not torch.is_grad_enabled() and not _has_forward_hooks(up)):
+                y = ops.linear_if_plain(x, up.weight, "silu_mul")
+                if y is not None:
+                    return self.down_proj(y)
         return self.down_proj(ops.silu_mul(up(x)))
 
 
@@ -223,7 +232,7 @@ class LlamaForCausalLM(BaseModelForCausalLM):
         self.model = DecoderModel(config, self._qk_norm(config))
         # (a vocabulary-wide bf16 / fp16 product stays on the library GEMM)
         self.lm_head = Linear(config.hidden_size, config.vocab_size, bias=False)
-        self.lm_head.half_rows = 0
+        self.lm_head.half_on_lv_linear = False
         if config.tie_word_embeddings:
             self.lm_head.weight = self.model.embed_tokens.weight
 

@@ -790,7 +790,18 @@ def linear_f32(x: torch.Tensor, weight: torch.Tensor,
     return out
 
 
+def linear_if_plain(x: torch.Tensor, weight: torch.Tensor,
+                    activation: Optional[str] = None) -> Optional[torch.Tensor]:
+    """linear (bf16 / fp16) or linear_f32 (fp32, no activation), or None,
+    having done nothing, where nn.Linear has to make the product: operands the
+    kernels do not take (rows that overlap or lie off 16-byte boundaries, other
+    sizes), grad mode, autocast, forward-mode tangents, traces, transforms and
+    Python modes."""
+    if torch.compiler.is_compiling():
+        return None
+    return (_native_module or _native()).layer_linear(x, weight, _ACTIVATIONS[activation])
+
+
 def linear_f32_if_plain(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
-    """linear_f32, or None for operands it has no kernel for (for callers with
-    another product to fall back on)."""
-    return (_native_module or _native()).linear_f32(x, weight, None)
+    """linear_if_plain for fp32 operands; None for others."""
+    return linear_if_plain(x, weight) if x.dtype is torch.float32 else None

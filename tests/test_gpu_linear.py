@@ -154,3 +154,110 @@ def test_linear_f32_forms_left_to_the_library():
         assert (got.double() - ref).norm() <= 1e-6 * ref.norm()
     lin(x[:, :256].contiguous()).sum().backward()
     assert lin.weight.grad is not None
+
+
+def _layer_and_reference(dtype, k=256, n=64):
+    from litevllm.models.llama import Linear
+    torch.manual_seed(3)
+    lin = Linear(k, n, bias=False).to(device="cuda", dtype=dtype)
+    ref = torch.nn.Linear(k, n, bias=False).to(device="cuda", dtype=dtype)
+    ref.load_state_dict(lin.state_dict())
+    return lin, ref
+
+
+@pytest.mark.parametrize("dtype,m", [(torch.float32, 9), (torch.bfloat16, 300)])
+def test_layer_is_nn_linear_to_autograd_autocast_and_transforms(dtype, m):
+    """Without reverse-mode gradients too, whatever else follows a call by the
+    dispatcher gets nn.Linear's product: tangents, autocast's type, traces that
+    record the product, vmap, dispatch and function modes, lazy negation."""
+    import torch.autograd.forward_ad as fwd
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    lin, ref = _layer_and_reference(dtype)
+    x, t = (torch.randn(m, 256, device="cuda", dtype=dtype) for _ in range(2))
+    tol = 1e-5 if dtype == torch.float32 else 2.0 ** -7
+
+    def close(a, b):
+        assert a.dtype == b.dtype and (a - b).float().norm() <= tol * b.float().norm()
+    with torch.no_grad():
+        close(lin(x), ref(x))
+        with fwd.dual_level():
+            d = fwd.unpack_dual(lin(fwd.make_dual(x, t)))
+            close(d.primal, ref(x))
+            close(d.tangent, ref(t))
+        y, dy = torch.func.jvp(lin, (x,), (t,))
+        close(dy, ref(t))
+        other = torch.float16 if dtype == torch.bfloat16 else torch.bfloat16
+        with torch.autocast("cuda", dtype=other):
+            assert lin(x).dtype == ref(x).dtype == other
+        traced = torch.jit.trace(lin, (x,))
+        close(traced(t), ref(t))
+        batch = torch.stack([x, t])
+        close(torch.func.vmap(lin)(batch), torch.func.vmap(ref)(batch))
+        seen = []
+
+        class Functions(TorchFunctionMode):
+            def __torch_function__(self, func, types, args=(), kwargs=None):
+                seen.append(func)
+                return func(*args, **(kwargs or {}))
+
+        class Ops(TorchDispatchMode):
+            def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+                seen.append(func)
+                return func(*args, **(kwargs or {}))
+        with Functions():
+            lin(x)
+        assert torch.nn.functional.linear in seen
+        seen.clear()
+        with Ops():
+            lin(x)
+        assert seen
+        if dtype == torch.float32:
+            z = torch.complex(t, x).conj().imag          # -x, not yet negated
+            assert z.is_neg()
+            close(lin(z), ref(z))
+
+
+@pytest.mark.parametrize("dtype,m", [(torch.float32, 9), (torch.bfloat16, 300),
+                                     (torch.float16, 300)])
+@torch.inference_mode()
+def test_layer_takes_every_row_layout_of_nn_linear(dtype, m, monkeypatch):
+    """Rows that overlap, lie off 16-byte boundaries or are columns, and a
+    weight that is a view: the library's product, as nn.Linear has it.  With
+    LV_DECODE_GEMM_ROWS = 0 every call is."""
+    from litevllm.models import llama
+    lin, ref = _layer_and_reference(dtype)
+    wide = torch.randn(m, 260, device="cuda", dtype=dtype)
+    forms = {"contiguous": wide[:, :256].contiguous(), "strided": wide[:, :256],
+             "off 16 bytes": wide[:, 1:257], "one row repeated": wide[:1, :256].expand(m, 256),
+             "overlapping": wide.flatten().as_strided((m, 256), (8, 1)),
+             "columns": wide[:, :256].t().contiguous().t()}
+    for name, x in forms.items():
+        print(f"[case] {dtype} {name}", flush=True)
+        a, b = lin(x), ref(x)
+        assert (a - b).float().norm() <= 2.0 ** (-20 if dtype == torch.float32 else -7) * \
+            b.float().norm()
+        mlp = llama.GatedMLP(256, 128).to(device="cuda", dtype=dtype)
+        up = torch.nn.functional.linear(x, mlp.gate_up_proj.weight)
+        want = torch.nn.functional.linear(
+            torch.nn.functional.silu(up[:, :128]) * up[:, 128:], mlp.down_proj.weight)
+        if m > 256 or dtype == torch.float32:
+            got = mlp(x)
+            assert (got - want).float().norm() <= 2.0 ** -6 * want.float().norm()
+    calls = []
+    monkeypatch.setattr(llama.ops, "linear", lambda *a, **k: calls.append(a))
+    monkeypatch.setattr(llama.ops, "linear_if_plain", lambda *a, **k: calls.append(a))
+    monkeypatch.setattr(llama, "DECODE_GEMM_ROWS", 0)
+    assert torch.equal(lin(forms["contiguous"]), ref(forms["contiguous"])) and not calls
+
+
+@torch.inference_mode()
+def test_gated_mlp_runs_the_hooks_of_its_projection():
+    from litevllm.models.llama import GatedMLP
+    mlp = GatedMLP(256, 128).cuda().bfloat16()
+    x = torch.randn(300, 256, device="cuda", dtype=torch.bfloat16)
+    want, seen = mlp(x), []
+    mlp.gate_up_proj.register_forward_hook(lambda mod, args, out: seen.append(out.shape))
+    got = mlp(x)
+    assert seen == [(300, 256)]
+    assert (got - want).float().norm() <= 2.0 ** -6 * want.float().norm()
