@@ -82,10 +82,10 @@ class RMSNorm(nn.Module):
         self.eps = eps
 
     def forward(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None):
-        if x.dim() == 2:
+        n = self.weight.shape[0]
+        if x.dim() == 2 and x.shape[1] == n:
             out = ops.add_rms_norm(x, self.weight, self.eps, residual=residual)
             return out if residual is None else (out, residual)
-        n = self.weight.shape[0]
         rows = x.reshape(-1, n)
         if residual is None:
             return ops.add_rms_norm(rows, self.weight, self.eps).view(x.shape)

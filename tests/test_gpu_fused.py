@@ -187,3 +187,21 @@ def test_qk_norm_rope_cache_forms(device, dtype, H, Hkv, D, form):
     gk, wk = kc_d.cpu().view(-1, Hkv, D)[rest], kc.view(-1, Hkv, D)[rest]
     _close(gk, wk, dtype, scale=pair_mag(wk))
     assert torch.equal(vc_d.cpu(), vc)
+
+
+@torch.inference_mode()
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_rms_norm_layer_folds_rows(device, dtype):
+    """The layer normalises the last n elements whatever the input's shape is:
+    [T, 4 n], with a residual of [4 T, n] rows too, as its rows on their own."""
+    from litevllm.models.llama import RMSNorm
+    norm = RMSNorm(64, 1e-6).to(device=device, dtype=dtype)
+    norm.weight.copy_(torch.rand(64) + 0.5)
+    x = torch.randn(5, 256, device=device).to(dtype)
+    rows = x.reshape(20, 64)
+    assert torch.equal(norm(x), norm(rows).reshape(5, 256))
+    assert torch.equal(norm(x.view(5, 4, 64)), norm(rows).reshape(5, 4, 64))
+    r0, r1 = (torch.ones(20, 64, device=device, dtype=dtype) for _ in range(2))
+    a, ra = norm(x, r0)
+    b, rb = norm(rows, r1)
+    assert torch.equal(a.reshape(20, 64), b) and ra is r0 and torch.equal(ra, rb)
