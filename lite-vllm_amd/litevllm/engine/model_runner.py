@@ -17,7 +17,11 @@ forward: decodes first, then prefill chunks; only the rows that are sampled
 
 from __future__ import annotations
 
+import contextlib
+import gc
 import os
+import sys
+import threading
 from dataclasses import dataclass
 from typing import Optional
 
@@ -282,6 +286,32 @@ GRAPH_BATCHES = (1, 2, 4, 8, 16, 24, 32, 48, 64, 80, 96, 112, 128, 144, 160, 176
                  224, 240, 256, 320, 384, 448, 512)
 
 
+# A CUDAGraph's destructor waits for the device, which the runtime refuses
+# while a stream of the thread (or, in the captures made here, of any thread)
+# is capturing; the error ends the process, since it is raised in a destructor.
+# So no graph may be freed inside a capture: not by the cyclic collector, which
+# runs wherever Python happens to allocate, and not by a thread that drops an
+# engine meanwhile.
+_capture_lock = threading.RLock()
+_retired: list[dict] = []     # graphs dropped while their thread was capturing
+
+
+@contextlib.contextmanager
+def _graph_capture():
+    """No DecodeGraphs is freed inside: garbage is collected first, the
+    collector is off until the end, and drops on other threads wait."""
+    with _capture_lock:
+        _retired.clear()
+        gc.collect()
+        was_on = gc.isenabled()
+        gc.disable()
+        try:
+            yield
+        finally:
+            if was_on:
+                gc.enable()
+
+
 class DecodeGraphs:
     """HIP graphs of the decode-only forward, one per padded batch size.
 
@@ -294,13 +324,16 @@ class DecodeGraphs:
     (the reference's convention, cache/block_manager.py:20-27) -- and their
     logits are dropped.  The attention workspace is sized for the largest
     batch and owned here, so no replay reads memory another call may free.
+    Nothing here refers to the runner: with its last reference the graphs go
+    too, at once and not when the cyclic collector comes by.
     """
 
     def __init__(self, runner: "ModelRunner", max_batch: int) -> None:
         mc = runner.model_config
         cc = runner.config.cache_config
         dev = torch.device(runner.device)
-        self.runner = runner
+        self.model: Optional[BaseModelForCausalLM] = None    # set by capture()
+        self.kv_cache: Optional[KVCache] = None
         self.block_size = cc.block_size
         self.max_blocks = (mc.max_model_len + cc.block_size - 1) // cc.block_size
         self.batches = [b for b in GRAPH_BATCHES if b < max_batch] + [max_batch]
@@ -366,12 +399,11 @@ class DecodeGraphs:
             p = self.pfx_plan
             meta.prefix = ops.PrefixPlan(p.blocks[:b], p.items, p.members)
             meta.prefix_workspace = self.pfx_workspace
-        r = self.runner
-        kv = [r.kv_cache.get_kv(i) for i in range(r.model_config.num_hidden_layers)]
-        return r.model(input_ids=v["input_ids"], positions=v["positions"], kv_caches=kv,
-                       slot_mapping=v["slot_mapping"], block_tables=v["block_tables"],
-                       context_lens=v["context_lens"], is_prefill=False, attn_metadata=meta,
-                       logits_indices=None)
+        kv = [self.kv_cache.get_kv(i) for i in range(self.kv_cache.num_layers)]
+        return self.model(input_ids=v["input_ids"], positions=v["positions"], kv_caches=kv,
+                          slot_mapping=v["slot_mapping"], block_tables=v["block_tables"],
+                          context_lens=v["context_lens"], is_prefill=False, attn_metadata=meta,
+                          logits_indices=None)
 
     def _pack(self, b: int, num_block_ids: int,
               device_tokens: Optional[torch.Tensor] = None) -> None:
@@ -380,21 +412,34 @@ class DecodeGraphs:
                         device_tokens=device_tokens, out=self._views(b))
 
     @torch.inference_mode()
-    def capture(self) -> None:
+    def capture(self, runner: "ModelRunner") -> None:
+        self.model, self.kv_cache = runner.model, runner.kv_cache
         pool = torch.cuda.graph_pool_handle()
-        for b in sorted(self.batches, reverse=True):
-            self._pad_rows(0, b)
-            self._pack(b, 1)
-            side = torch.cuda.Stream()
-            side.wait_stream(torch.cuda.current_stream())
-            with torch.cuda.stream(side):
-                self._forward(b)
-            torch.cuda.current_stream().wait_stream(side)
-            g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g, pool=pool):
-                self.logits[b] = self._forward(b)
-            self.graphs[b] = g
-        torch.cuda.synchronize()
+        with _graph_capture():
+            for b in sorted(self.batches, reverse=True):
+                self._pad_rows(0, b)
+                self._pack(b, 1)
+                side = torch.cuda.Stream()
+                side.wait_stream(torch.cuda.current_stream())
+                with torch.cuda.stream(side):
+                    self._forward(b)
+                torch.cuda.current_stream().wait_stream(side)
+                g = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(g, pool=pool):
+                    self.logits[b] = self._forward(b)
+                self.graphs[b] = g
+            torch.cuda.synchronize()
+
+    def __del__(self) -> None:
+        graphs = self.__dict__.get("graphs")
+        if not graphs or sys.is_finalizing():
+            return
+        with _capture_lock:
+            if torch.cuda.is_current_stream_capturing():   # e.g. in a program's own capture
+                _retired.append(graphs)
+                return
+            graphs.clear()
+            _retired.clear()
 
     def accepts(self, st: StepDescriptors) -> bool:
         B = st.descs.shape[0]
@@ -504,8 +549,12 @@ class ModelRunner:
         the scheduler's max_num_seqs (block 0 must be reserved as scratch)."""
         max_batch = min(self.config.max_graph_batch, self.config.scheduler_config.max_num_seqs)
         graphs = DecodeGraphs(self, max_batch)
-        graphs.capture()
+        graphs.capture(self)
         self.graphs = graphs
+
+    def release_decode_graphs(self) -> None:
+        """Free the captured graphs; later decode steps run eagerly."""
+        self.graphs = None
 
     # ------------------------------------------------------------------
     def prepare_inputs(self, seq_groups: list[SequenceGroup], block_manager,

@@ -72,6 +72,9 @@ class AsyncLLM:
             self._post("stop", None)
             await self._loop.run_in_executor(None, self._thread.join)
             self._thread = None
+            runner = getattr(self._engine, "model_runner", None)
+            if runner is not None:      # not whenever the last reference goes
+                runner.release_decode_graphs()
 
     # -- requests ------------------------------------------------------------
     async def add_request(self, prompt: Optional[str], sampling_params: SamplingParams,
