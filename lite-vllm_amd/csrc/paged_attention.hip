@@ -309,7 +309,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_rows_kernel(
 //
 // The blocks of all decode sequences form one flattened list (sequence-major:
 // sequence s owns entries off[s] .. off[s+1]-1, off = exclusive scan of
-// ceil(ctx / bs)).  A fixed grid of workgroups (about two per CU) splits the
+// ceil(ctx / bs)).  A fixed grid of workgroups (plan_decode) splits the
 // list into equal contiguous ranges, so every workgroup streams the same
 // number of blocks however ragged the contexts are.  Wavefront w of a
 // workgroup owns kv head w; all wavefronts walk the same blocks, so the K/V
@@ -574,10 +574,13 @@ struct MergeState {
 //   * softmax in fp32, one reference maximum per column, raised only when a
 //     score exceeds it by 2^4;
 //   * O^T += V^T P^T, D / 16 products of 16x16x16 with V^T by the LDS
-//     transpose read.  P stays fp32-exact: its leading, middle and trailing
-//     bits (8 each in bf16, 11 each in fp16) are three values of the
-//     element type in three columns of the same product (G = 8: the third
-//     in a second product), so O sums the fp32 weights' products in fp32.
+//     transpose read.  P is not rounded to the element type: its leading,
+//     middle and trailing bits (8 each in bf16, 11 each in fp16) are three
+//     values of that type in three columns of the same product (G = 8: the
+//     third in a second product), so O sums the fp32 weights' products in
+//     fp32.  In bf16 the three parts are the weight exactly; in fp16, whose
+//     smallest step is 2^-24, they are within 2^-25 of it, against a largest
+//     weight of the row of 2^10 or more (kLift).
 // Column c of a tile is head c % G, part c / G of P (parts past the third
 // are zero).  An infinite V makes NaN of every zero among them, so a sum that
 // is not finite is taken from the leading part's column, whose weights are
@@ -642,8 +645,10 @@ __global__ __launch_bounds__(kPersistMaxWaves * 64) void attn_decode_mfma_kernel
   static_assert(BS == B::BS, "16-token blocks");
   constexpr int QS = D / 32;                   // k-steps of K Q^T
   constexpr int NB = D / 16;                   // 16-dim blocks of O^T
-  // fp16 weights are kept between 2^-14 and 2^15: the reference maximum sits
-  // 2^10 under the score that set it
+  // fp16: the reference maximum sits 10 (in log2 units) under the score that
+  // set it and is raised when a score passes that by 4, so a row's largest
+  // weight is between 2^10 and 2^14 and the fixed steps of the smallest fp16
+  // values weigh little against it
   constexpr float kLift = std::is_same<T, f16>::value ? 10.0f : 0.0f;
   // LDS: the wavefronts' stages, s_off [num_seqs + 1], then (shared prefixes
   // only) s_skip [num_seqs]
@@ -1952,8 +1957,9 @@ __global__ __launch_bounds__(D) void attn_reduce_kernel(
 // Decode kernel choice.  Default: the persistent kernel with non-temporal
 // K/V loads.  Tuning knobs (environment): LV_ATTN_DECODE_KERNEL=rows selects
 // the workgroup-per-(row, kv head, partition) kernel, LV_ATTN_PART_TOKENS its
-// partition length, LV_ATTN_NT=0 plain loads, LV_ATTN_PERSIST_WGS the
-// persistent grid size.
+// partition length, LV_ATTN_PERSIST_WGS the persistent grid size.  Of the row
+// and vector kernels only: LV_ATTN_NT=0 plain loads, LV_ATTN_NBUF=4 four
+// register buffers.
 static bool env_is(const char* name, char c) {
   const char* e = getenv(name);
   return e != nullptr && e[0] == c;
