@@ -583,13 +583,18 @@ def bench_e2e(args):
             del g
         return times, nbytes
 
+    def sampled():
+        """Whether the step at hand is one the probe times: decodes only."""
+        meta = probe["meta"]
+        return probe["on"] and meta is not None and meta.num_decodes == len(meta.seq_ids)
+
     def c_probe(name):
         fn = orig_c[name]
 
         def call(*args):
-            meta = probe["meta"]
-            if not probe["on"] or meta is None or meta.num_decodes != len(meta.seq_ids):
+            if not sampled():
                 return fn(*args)
+            meta = probe["meta"]
             e0 = torch.cuda.Event(enable_timing=True)
             e1 = torch.cuda.Event(enable_timing=True)
             e0.record()
@@ -614,11 +619,13 @@ def bench_e2e(args):
     mr.ModelRunner.execute_model = exec_probe
     for n in orig_c:
         setattr(lib, n, c_probe(n))
-    # the probes sit on the ctypes symbols: attention calls go through them
+    # the probes sit on the ctypes symbols: the sampled steps' attention calls
+    # go through them, all others take the product's own path
     native = ops._native()
     ops._native_module = types.SimpleNamespace(
         **{n: getattr(native, n) for n in dir(native) if not n.startswith("_")})
-    ops._native_module.paged_attention = lambda *a: None
+    ops._native_module.paged_attention = \
+        lambda *a: None if sampled() else native.paged_attention(*a)
     mr.DecodeGraphs.accepts = accepts_probe
     llm = LLM("qwen3-0.6b-shape", dtype="bfloat16", load_format="dummy", hf_overrides=mc,
               skip_tokenizer_init=True, enable_prefix_caching=True, max_num_batched_tokens=8192,
