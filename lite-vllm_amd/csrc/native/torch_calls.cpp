@@ -479,21 +479,23 @@ bool is_aligned_rows(const at::Tensor& t, int64_t width, at::ScalarType type) {
          t.stride(0) * t.element_size() % 16 == 0 && (uintptr_t)ptr(&t) % 16 == 0;
 }
 
-// (x, weight, silu_mul) -> out: nn.Linear's product for a layer that falls
+// (x, weight, None or "silu_mul") -> out: nn.Linear's product for a layer that falls
 // back on nn.Linear itself, so everything the library's kernels ask for or
 // nn.Linear answers differently is not plain here.
 FAST(layer_linear, 3) {
   const at::Tensor *x = A.tensor(0), *w = A.tensor(1);
-  const int64_t act = A.integer(2);
+  const bool silu = A.a[2] != Py_None;
   lv_dtype dt;
   if (!A.ok || !x->is_cuda() || !dtype_of(*x, dt) || x->dim() != 2 || w->dim() != 2 ||
+      (silu && (!PyUnicode_Check(A.a[2]) ||
+                PyUnicode_CompareWithASCIIString(A.a[2], "silu_mul") != 0)) ||
       !calls_are_direct())
     NOT_PLAIN();
   const at::Device dev = x->device();
   const at::ScalarType type = x->scalar_type();
   const int64_t M = x->size(0), K = x->size(1), rows = w->size(0);
-  const bool silu = act == LV_ACT_SILU_MUL;
   const int64_t N = silu ? rows / 2 : rows;
+  const int32_t act = silu ? LV_ACT_SILU_MUL : LV_ACT_NONE;
   if (M == 0 || N == 0 || K == 0 || !on(x, dev) || !on(w, dev) || !is_direct(*x) ||
       !is_direct(*w) || w->size(1) != K || (silu && rows % 2) || !is_aligned_rows(*x, K, type) ||
       !is_aligned_rows(*w, K, type) ||

@@ -62,7 +62,7 @@ class Linear(nn.Linear):
                 return ops.linear(x, self.weight)
             else:
                 small = m <= 2 * DECODE_GEMM_ROWS and n * k <= SMALL_LAYER
-            if small and not torch.is_grad_enabled():
+            if small:
                 y = ops.linear_if_plain(x, self.weight)
                 if y is not None:
                     return y
@@ -82,14 +82,15 @@ class RMSNorm(nn.Module):
         self.eps = eps
 
     def forward(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None):
-        n = self.weight.shape[0]
-        if x.dim() == 2 and x.shape[1] == n:
-            out = ops.add_rms_norm(x, self.weight, self.eps, residual=residual)
+        weight = self.weight
+        n = weight.size(0)
+        if x.dim() == 2 and x.size(1) == n:
+            out = ops.add_rms_norm(x, weight, self.eps, residual)
             return out if residual is None else (out, residual)
         rows = x.reshape(-1, n)
         if residual is None:
-            return ops.add_rms_norm(rows, self.weight, self.eps).view(x.shape)
-        out = ops.add_rms_norm(rows, self.weight, self.eps, residual=residual)
+            return ops.add_rms_norm(rows, weight, self.eps).view(x.shape)
+        out = ops.add_rms_norm(rows, weight, self.eps, residual=residual)
         return out.view(x.shape), residual
 
 
@@ -112,7 +113,7 @@ class GatedMLP(nn.Module):
             if m <= DECODE_GEMM_ROWS:
                 return self.down_proj(ops.linear(x, up.weight, activation="silu_mul"))
             if (up.out_features * up.in_features <= SMALL_LAYER
-                    and not torch.is_grad_enabled() and not _has_forward_hooks(up)):
+                    and not _has_forward_hooks(up)):
                 y = ops.linear_if_plain(x, up.weight, "silu_mul")
                 if y is not None:
                     return self.down_proj(y)

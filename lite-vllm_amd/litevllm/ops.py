@@ -797,9 +797,9 @@ def linear_if_plain(x: torch.Tensor, weight: torch.Tensor,
     kernels do not take (rows that overlap or lie off 16-byte boundaries, other
     sizes), grad mode, autocast, forward-mode tangents, traces, transforms and
     Python modes."""
-    if torch.compiler.is_compiling():
+    if torch.compiler.is_dynamo_compiling():
         return None
-    return (_native_module or _native()).layer_linear(x, weight, _ACTIVATIONS[activation])
+    return (_native_module or _native()).layer_linear(x, weight, activation)
 
 
 def linear_f32_if_plain(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:

@@ -192,6 +192,8 @@ def test_layer_is_nn_linear_to_autograd_autocast_and_transforms(dtype, m):
             assert lin(x).dtype == ref(x).dtype == other
         traced = torch.jit.trace(lin, (x,))
         close(traced(t), ref(t))
+        compiled = torch.compile(lin, backend="eager", fullgraph=True)
+        close(compiled(t), ref(t))
         batch = torch.stack([x, t])
         close(torch.func.vmap(lin)(batch), torch.func.vmap(ref)(batch))
         seen = []
