@@ -2235,15 +2235,27 @@ static ChunkPlan plan_chunks(int n_seqs, int num_kv_heads, int G, int head_dim, 
   ChunkPlan p{};
   const int64_t groups = (int64_t)num_kv_heads * n_seqs;
   const int cus = device_cu_count();
-  // Split tiles while 128-row workgroups would leave half the slots (two per
-  // CU) empty: 64 rows each, every wavefront with half the dependent chain
-  // (K Q^T, softmax, P V) per tile.  Calls as graph replays, 128-row / split
-  // (16 / 8 heads, D = 128): one prompt of 777 tokens (104 workgroups) 21.6 /
-  // 16.8 us, of 2000 (256) 43.3 / 35.5, 6 chunks of 512 at up to 3000 (384)
-  // 76.6 / 68.9; 8 chunks (512) 87.3 / 87.4, 15 chunks (960) 146 / 157.
+  // Split tiles while the 64-row workgroups all run at once (two per CU): 64
+  // rows each, every wavefront with half the dependent chain (K Q^T, softmax,
+  // P V) per tile.  A (sequence, kv head) group's workgroups share one XCD, so
+  // what counts is the XCD with the most of them: with one kv head and one
+  // sequence that is all of them, on 32 CUs.  Past that line the last of them
+  // start when the first end, which pays only where they get shorter: one
+  // prompt from (nearly) its start, whose query tiles run longest first.
+  // 128-row / split, us, for 128-row workgroups on the fullest XCD (bf16, D =
+  // 128): 13 (777 tokens, 16 / 8 heads) 20.7 / 15.9, 32 (2048) 42.5 / 36.5, 48
+  // (3072) 65.5 / 54.4; 32 (6 chunks of 320) 14.6 / 14.8; past the line at an
+  // offset or of many short chunks 38 (2432 at 2000) 94.6 / 103, 44 (1408 at
+  // 2000, 16 / 4 heads) 82.8 / 95.0, 48 (12 chunks of 128, 32 / 8 heads) 14.6 /
+  // 19.3, 188 (3000 tokens, 16 / 2 heads) 152 / 180.  Over 963 shapes within
+  // 1.5 times the line: 0.93 of the whole tiles' time, at most 1.06.
   // Four tiles in flight, or 128-key tiles over eight wavefronts, were slower
   // but for a few workgroups on long contexts (next rule).
-  p.half = groups * ((max_query_len + 128 / G - 1) / (128 / G)) * 2 <= 3 * (int64_t)cus;
+  const int64_t fullest = (groups + kXcds - 1) / kXcds * ((max_query_len + 128 / G - 1) / (128 / G));
+  const int64_t line = cus / kXcds;
+  const bool triangle = max_query_len >= 1024 &&
+                        (int64_t)max_blocks * block_size <= max_query_len + max_query_len / 4;
+  p.half = fullest <= line || (2 * fullest <= 3 * line && triangle);
   p.nsplit = 1;
   if (!p.half || groups > 0x7fffffff) return p;
   p.units = chunk_units((int)groups, (max_query_len + 64 / G - 1) / (64 / G));
