@@ -2012,9 +2012,16 @@ static AttnPlan plan_decode(int num_decodes, int num_heads, int num_kv_heads, in
     // stages each at head_dim 128.  Measured (1 / 2 / 3 / 4 per CU, us): 4 kv
     // heads 59.4 / 55.4 / 65.8 / 63.9; 2 kv heads, 256 rows 85.2 / 63.2 /
     // 59.8 / 62.2; 1 kv head 41.3 / 27.5 / 22.7 / 21.8; 8 kv heads 179.7 / 193.
+    // head_dim 64 halves a block, so with one or two query heads per kv head a
+    // CU needs twice the wavefronts to cover HBM (300 rows of up to 2000
+    // tokens, 1 / 2 per CU, vector kernel: 5 kv heads 125.6 / 85.2 / 89.7, 6
+    // 129.5 / 102.0 / 100.1, 7 137.1 / 117.3 / 115.3, 8 142.3 / 131.4 / 129.8);
+    // with more the matrix cores' work does it (8 kv heads of 8: 143.7 / 147.1 /
+    // 237.3, 256 rows of up to 100 tokens 19.9 / 33.8 / 48.3).
     p.nbuf = env_int("LV_ATTN_NBUF", 2) == 4 ? 4 : 2;
+    const int wide = head_dim == 64 && num_heads <= 2 * num_kv_heads ? 2 : 1;
     const int per_cu = dtype == LV_F32 ? (num_kv_heads == 1 ? 4 : 1)
-                       : num_kv_heads >= 5 ? 1 : num_kv_heads >= 3 ? 2 : num_kv_heads == 2 ? 3 : 4;
+                       : num_kv_heads >= 5 ? wide : num_kv_heads >= 3 ? 2 : num_kv_heads == 2 ? 3 : 4;
     p.num_wgs = env_int("LV_ATTN_PERSIST_WGS", device_cu_count() * per_cu);
     // wavefront lockstep interval in blocks (LV_ATTN_SYNC=0: none)
     int sync = env_is("LV_ATTN_SYNC", '0') ? 0 : env_int("LV_ATTN_SYNC", 4);

@@ -428,6 +428,25 @@ def test_mixed_batch_under_capture_does_not_split(device, path, monkeypatch):
     del pool
 
 
+@pytest.mark.parametrize("heads,chunk,off", [
+    ((16, 8, 128), 2048, 0), ((16, 8, 128), 2049, 0), ((16, 8, 128), 2049, 600),
+    ((16, 8, 128), 3073, 0), ((8, 1, 128), 512, 0), ((8, 1, 128), 513, 0), ((4, 2, 64), 3000, 0)])
+def test_chunks_around_the_line_of_split_tiles(device, heads, chunk, off):
+    """One prompt just inside and past the sizes at which its workgroups stop
+    running all at once (split tiles, from there on whole tiles unless the
+    prompt is long and near its start), and past the last of them.  Weights
+    and outputs are rounded to bf16 once each: 2^-8 relative L2."""
+    H, Hkv, D = heads
+    _say(f"chunks around the line {heads} {chunk} at {off}")
+    batch = workloads.mixed_step(seed=chunk, num_decodes=0, num_chunks=1, chunk_len=chunk,
+                                 off_lo=off, off_hi=off, num_heads=H, num_kv_heads=Hkv,
+                                 head_dim=D, num_cache_slots=16 * 400).batch
+    got = _run_attention(batch, device, use_cu=True).float().cpu()
+    ref = _oracle(batch)
+    assert torch.isfinite(got).all()
+    assert (got - ref).norm() <= 2.0 ** -8 * ref.norm()
+
+
 @pytest.mark.parametrize("rows,heads", [(1, (16, 8, 128)), (3, (16, 2, 128)), (7, (8, 8, 64)),
                                         (128, (16, 8, 128)), (129, (16, 8, 128))])
 def test_decode_few_rows_of_many_pieces(device, rows, heads):
