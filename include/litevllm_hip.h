@@ -408,6 +408,11 @@ typedef enum lv_activation {
 
 int lv_linear_supported(int64_t m, int64_t n, int64_t k, int32_t activation, lv_dtype dtype);
 
+/* Whether the workgroups of such a call all run at once (0 also where there is
+ * no kernel): past that the last of them start when the first end, and a
+ * library GEMM with larger tiles is the faster one. */
+int lv_linear_one_round(int64_t m, int64_t n, int64_t k, int32_t activation);
+
 int lv_linear(const void* x_dev, int64_t x_stride_t, const void* weight_dev,
               int64_t weight_stride_n, void* y_dev, int64_t y_stride_t, int64_t m, int64_t n,
               int64_t k, int32_t activation, lv_dtype dtype, void* stream);

@@ -331,8 +331,8 @@ __global__ __launch_bounds__(64 * kF32Waves) void linear_f32_kernel(
 // make more (two resident per CU cover the second round), else the narrower
 // tiles.  LV_LINEAR_CFG forces one.
 // ---------------------------------------------------------------------------
-struct LinCfg { int tm, tn; };
-constexpr LinCfg kLinCfgs[] = {{64, 64}, {64, 64}, {32, 32}, {32, 64}};
+struct LinCfg { int tm, tn, ns; };
+constexpr LinCfg kLinCfgs[] = {{64, 64, 3}, {64, 64, 2}, {32, 32, 4}, {32, 64, 4}};
 constexpr int kLinNumCfgs = 4;
 
 // silu_mul: tiles of 64 x 32 outputs (64 staged weight rows: 32 gate, 32 up),
@@ -401,6 +401,19 @@ extern "C" int lv_linear_supported(int64_t m, int64_t n, int64_t k, int32_t acti
   if (activation != LV_ACT_NONE && activation != LV_ACT_SILU_MUL) return 0;
   if (m < 1 || m > 0x7fffffff || n < 1 || n > 0x3fffffff || k < 1 || k > 0x7fffffff) return 0;
   return (activation == LV_ACT_SILU_MUL ? lin_pick_silu(m, n, k) : lin_pick(m, n, k)) >= 0;
+}
+
+extern "C" int lv_linear_one_round(int64_t m, int64_t n, int64_t k, int32_t activation) {
+  using namespace lv;
+  if (!lv_linear_supported(m, n, k, activation, LV_BF16)) return 0;
+  const bool silu = activation == LV_ACT_SILU_MUL;
+  const int cfg = silu ? lin_pick_silu(m, n, k) : lin_pick(m, n, k);
+  const LinCfg c = silu ? LinCfg{64, 32, cfg == 1 ? 2 : 3} : kLinCfgs[cfg];
+  const int staged_rows = c.tm + (silu ? 2 : 1) * c.tn;
+  const int per_cu = 160 * 1024 / (c.ns * staged_rows * kLinK * 2);
+  // the n tiles are dealt out over the XCDs; all m tiles of one follow it
+  const int64_t fullest = (n / c.tn + kXcds - 1) / kXcds * ((m + c.tm - 1) / c.tm);
+  return fullest <= 256 / kXcds * per_cu;
 }
 
 extern "C" int lv_linear(const void* x_dev, int64_t x_stride_t, const void* weight_dev,

@@ -44,7 +44,7 @@ struct Api {
   decltype(&lv_add_rms_norm) add_rms_norm;
   decltype(&lv_qk_norm_rope_cache) qk_norm_rope_cache;
   decltype(&lv_silu_mul) silu_mul;
-  decltype(&lv_linear_supported) linear_supported;
+  decltype(&lv_linear_one_round) linear_one_round;
   decltype(&lv_linear) linear;
   decltype(&lv_linear_f32) linear_f32;
 };
@@ -55,7 +55,7 @@ constexpr const char* kNames[] = {
     "lv_paged_attention_split_workspace_size", "lv_paged_attention",
     "lv_paged_attention_prefix_workspace_size", "lv_paged_attention_prefix",
     "lv_sample_workspace_size", "lv_sample", "lv_add_rms_norm", "lv_qk_norm_rope_cache",
-    "lv_silu_mul", "lv_linear_supported", "lv_linear", "lv_linear_f32"};
+    "lv_silu_mul", "lv_linear_one_round", "lv_linear", "lv_linear_f32"};
 constexpr size_t kNumNames = sizeof(kNames) / sizeof(kNames[0]);
 static_assert(sizeof(Api) == kNumNames * sizeof(void*), "one pointer per name");
 
@@ -479,9 +479,16 @@ bool is_aligned_rows(const at::Tensor& t, int64_t width, at::ScalarType type) {
          t.stride(0) * t.element_size() % 16 == 0 && (uintptr_t)ptr(&t) % 16 == 0;
 }
 
-// (x, weight, None or "silu_mul") -> out: nn.Linear's product for a layer that falls
-// back on nn.Linear itself, so everything the library's kernels ask for or
-// nn.Linear answers differently is not plain here.
+// (x, weight, None or "silu_mul") -> out: nn.Linear's product for a layer that
+// falls back on nn.Linear itself, so everything the library's kernels ask for
+// or nn.Linear answers differently is not plain here.  Nor is a call under
+// graph capture: what these products save is host time, on the GPU the library
+// GEMM is often the faster (fp32, 16 rows of 1024x512: 7.2 us against 4.5;
+// 4096x1024 11.9 and 6.0).  bf16 / fp16, 257-512 rows, GPU time against the
+// library: 0.65-1.13 where the workgroups run at once and k is at least 512
+// (4096x1024 1.01-1.10, 1024x3072 0.83-0.91), 1.2-1.7 where they do not
+// (6144x1024 from 384 rows on, 2048x2048 up to 384, 384 rows of 1280x5120); with
+// SiLU 0.64-0.85 where the layer widens, up to 1.35 where it does not.
 FAST(layer_linear, 3) {
   const at::Tensor *x = A.tensor(0), *w = A.tensor(1);
   const bool silu = A.a[2] != Py_None;
@@ -499,7 +506,9 @@ FAST(layer_linear, 3) {
   if (M == 0 || N == 0 || K == 0 || !on(x, dev) || !on(w, dev) || !is_direct(*x) ||
       !is_direct(*w) || w->size(1) != K || (silu && rows % 2) || !is_aligned_rows(*x, K, type) ||
       !is_aligned_rows(*w, K, type) ||
-      (dt == LV_F32 ? silu || K % 4 != 0 : !api.linear_supported(M, N, K, act, dt)))
+      (dt == LV_F32 ? silu || K % 4 != 0
+                    : (silu ? N < K : K < 512) || !api.linear_one_round(M, N, K, act)) ||
+      c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None)
     NOT_PLAIN();
   const at::Tensor out = empty({M, N}, *x);
   void* st = stream_of(dev);

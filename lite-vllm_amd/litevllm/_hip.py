@@ -119,6 +119,7 @@ SIGNATURES: dict[str, tuple] = {
         ctypes.c_int, _c_p,            # dtype, stream
     ]),
     "lv_linear_supported": (ctypes.c_int, [_c_i64, _c_i64, _c_i64, _c_i32, ctypes.c_int]),
+    "lv_linear_one_round": (ctypes.c_int, [_c_i64, _c_i64, _c_i64, _c_i32]),
     "lv_linear": (ctypes.c_int, [
         _c_p, _c_i64, _c_p, _c_i64,    # x, x_stride, weight, weight_stride
         _c_p, _c_i64,                  # y, y_stride

@@ -23,16 +23,18 @@ from litevllm.models.base import BaseModelForCausalLM
 # next two.
 DECODE_GEMM_ROWS = int(os.environ.get("LV_DECODE_GEMM_ROWS", "256"))
 # Where nothing but the product itself would see the call (linear_if_plain),
-# layers of up to SMALL_LAYER weights take lv_linear to twice as many rows.  The library's call alone costs 19 us of host time against 4
-# (an eager step of that many tokens is bound by the host), and on the GPU the
-# two are level: 512 rows of 4096x1024 10.5 us (library 10.8), 1024x2048 8.5
-# (9.8), 1024x3072 10.6 (12.5), 6144x1024 16.5 (13.4, plus 5 for the SiLU that
-# lv_linear has in its epilogue); at 768 rows 16.5 against 12.1.
+# layers of up to SMALL_LAYER weights take lv_linear to twice as many rows.  The
+# library's call alone costs 19 us of host time against 4 (an eager step of that
+# many tokens is bound by the host), and on the GPU the two are level while
+# lv_linear's workgroups all run at once, which linear_if_plain asks for: 512
+# rows of 4096x1024 10.3 us (library 10.1), 1024x2048 7.9 (8.9), 1024x3072 10.5
+# (11.6), 320 of 6144x1024 with SiLU 10.1 (13.6); past that 512 rows of
+# 6144x1024 15.7 (12.5).
 SMALL_LAYER = 1 << 23
 # fp32 products of up to SMALL_F32 multiply-adds (k up to 1024) run on
-# lv_linear_f32, under the same condition: 4 us of host time, and 4-10 us on the
-# GPU where the library takes 4-8 us on its good shapes and up to 133 on others
-# (200 rows of 256x688); 2x slower than the library past the line.
+# lv_linear_f32, under the same condition and outside graph capture: 4 us of
+# host time, and 4-13 us on the GPU where the library takes 4-8 us on its good
+# shapes and up to 133 on others (200 rows of 256x688).
 SMALL_F32 = 1 << 27
 
 

@@ -795,8 +795,9 @@ def linear_if_plain(x: torch.Tensor, weight: torch.Tensor,
     """linear (bf16 / fp16) or linear_f32 (fp32, no activation), or None,
     having done nothing, where nn.Linear has to make the product: operands the
     kernels do not take (rows that overlap or lie off 16-byte boundaries, other
-    sizes), grad mode, autocast, forward-mode tangents, traces, transforms and
-    Python modes."""
+    sizes), bf16 / fp16 sizes at which the library GEMM is clearly faster on the
+    GPU (lv_linear_one_round), graph capture, grad mode, autocast, forward-mode
+    tangents, traces, transforms and Python modes."""
     if torch.compiler.is_dynamo_compiling():
         return None
     return (_native_module or _native()).layer_linear(x, weight, activation)

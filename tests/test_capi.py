@@ -168,3 +168,17 @@ def test_check_device_errors_message(monkeypatch):
                         _hip.LV_DEVERR_SLOT)
     with pytest.raises(RuntimeError, match="block-table entry.*slot_mapping entry"):
         ops.check_device_errors()
+
+
+def test_linear_one_round():
+    """Workgroups on the fullest XCD against its 32 CUs: 64 x 64 tiles, two a CU
+    from 257 of them on; 32 x 64 tiles, one a CU; with SiLU 64 x 32."""
+    from litevllm import _hip
+    lib = _hip.load()
+    one = lambda m, n, k, act=0: lib.lv_linear_one_round(m, n, k, act)
+    assert one(320, 6144, 1024) == 1 and one(321, 6144, 1024) == 0     # 12 x 5, 12 x 6 of 64
+    assert one(512, 2048, 2048) == 1 and one(384, 2048, 2048) == 0     # 4 x 8 of 32, 4 x 12
+    assert one(320, 1280, 5120) == 1 and one(384, 1280, 5120) == 0     # 3 x 10, 3 x 12 of 32
+    assert one(320, 3072, 1024, 1) == 1 and one(384, 3072, 1024, 1) == 0
+    assert one(0, 64, 128) == 0 and one(8, 33, 128) == 0 and one(8, 64, 100) == 0
+    assert one(8, 64, 128, 7) == 0 and one(8, 64, 128) == 1

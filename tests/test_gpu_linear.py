@@ -156,7 +156,7 @@ def test_linear_f32_forms_left_to_the_library():
     assert lin.weight.grad is not None
 
 
-def _layer_and_reference(dtype, k=256, n=64):
+def _layer_and_reference(dtype, k=512, n=64):
     from litevllm.models.llama import Linear
     torch.manual_seed(3)
     lin = Linear(k, n, bias=False).to(device="cuda", dtype=dtype)
@@ -174,7 +174,7 @@ def test_layer_is_nn_linear_to_autograd_autocast_and_transforms(dtype, m):
     from torch.overrides import TorchFunctionMode
     from torch.utils._python_dispatch import TorchDispatchMode
     lin, ref = _layer_and_reference(dtype)
-    x, t = (torch.randn(m, 256, device="cuda", dtype=dtype) for _ in range(2))
+    x, t = (torch.randn(m, 512, device="cuda", dtype=dtype) for _ in range(2))
     tol = 1e-5 if dtype == torch.float32 else 2.0 ** -7
 
     def close(a, b):
@@ -229,20 +229,20 @@ def test_layer_takes_every_row_layout_of_nn_linear(dtype, m, monkeypatch):
     LV_DECODE_GEMM_ROWS = 0 every call is."""
     from litevllm.models import llama
     lin, ref = _layer_and_reference(dtype)
-    wide = torch.randn(m, 260, device="cuda", dtype=dtype)
-    forms = {"contiguous": wide[:, :256].contiguous(), "strided": wide[:, :256],
-             "off 16 bytes": wide[:, 1:257], "one row repeated": wide[:1, :256].expand(m, 256),
-             "overlapping": wide.flatten().as_strided((m, 256), (8, 1)),
-             "columns": wide[:, :256].t().contiguous().t()}
+    wide = torch.randn(m, 520, device="cuda", dtype=dtype)
+    forms = {"contiguous": wide[:, :512].contiguous(), "strided": wide[:, :512],
+             "off 16 bytes": wide[:, 1:513], "one row repeated": wide[:1, :512].expand(m, 512),
+             "overlapping": wide.flatten().as_strided((m, 512), (8, 1)),
+             "columns": wide[:, :512].t().contiguous().t()}
     for name, x in forms.items():
         print(f"[case] {dtype} {name}", flush=True)
         a, b = lin(x), ref(x)
         assert (a - b).float().norm() <= 2.0 ** (-20 if dtype == torch.float32 else -7) * \
             b.float().norm()
-        mlp = llama.GatedMLP(256, 128).to(device="cuda", dtype=dtype)
+        mlp = llama.GatedMLP(512, 512).to(device="cuda", dtype=dtype)
         up = torch.nn.functional.linear(x, mlp.gate_up_proj.weight)
         want = torch.nn.functional.linear(
-            torch.nn.functional.silu(up[:, :128]) * up[:, 128:], mlp.down_proj.weight)
+            torch.nn.functional.silu(up[:, :512]) * up[:, 512:], mlp.down_proj.weight)
         if m > 256 or dtype == torch.float32:
             got = mlp(x)
             assert (got - want).float().norm() <= 2.0 ** -6 * want.float().norm()
@@ -256,10 +256,35 @@ def test_layer_takes_every_row_layout_of_nn_linear(dtype, m, monkeypatch):
 @torch.inference_mode()
 def test_gated_mlp_runs_the_hooks_of_its_projection():
     from litevllm.models.llama import GatedMLP
-    mlp = GatedMLP(256, 128).cuda().bfloat16()
+    mlp = GatedMLP(256, 256).cuda().bfloat16()
     x = torch.randn(300, 256, device="cuda", dtype=torch.bfloat16)
     want, seen = mlp(x), []
     mlp.gate_up_proj.register_forward_hook(lambda mod, args, out: seen.append(out.shape))
     got = mlp(x)
-    assert seen == [(300, 256)]
+    assert seen == [(300, 512)]
     assert (got - want).float().norm() <= 2.0 ** -6 * want.float().norm()
+
+
+@torch.inference_mode()
+def test_layer_products_leave_graphs_and_slow_sizes_to_the_library():
+    """Under capture the library's product is recorded (host time, all the own
+    kernels save there, is not spent on replays), equal on every replay to the
+    library's eager one; so are sizes whose workgroups do not run at once."""
+    lin, ref = _layer_and_reference(torch.float32)
+    x = torch.randn(9, 512, device="cuda")
+    assert ops.linear_if_plain(x, lin.weight) is not None
+    ref(x)
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=stream):
+        assert ops.linear_if_plain(x, lin.weight) is None
+        y = lin(x)
+    for _ in range(3):
+        x.normal_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.allclose(y, ref(x), rtol=0, atol=1e-5 * float(x.abs().max()))
+    for m, n, k, act, own in ((320, 6144, 1024, None, True), (384, 6144, 1024, None, False),
+                              (300, 512, 256, None, False), (300, 1024, 512, "silu_mul", True),
+                              (300, 512, 512, "silu_mul", False)):
+        x, w = (torch.randn(r, k, device="cuda", dtype=torch.bfloat16) for r in (m, n))
+        assert (ops.linear_if_plain(x, w, act) is not None) == own, (m, n, k, act)
