@@ -53,19 +53,24 @@ class Linear(nn.Linear):
     half_on_lv_linear = True     # False: bf16 / fp16 calls use the library GEMM
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        m = x.shape[0] if x.dim() == 2 else 0
-        if m > 0 and self.bias is None and x.is_cuda and DECODE_GEMM_ROWS > 0:
+        m = x.size(0) if x.dim() == 2 else 0
+        # (registered parameters, not a parametrization's attributes, without
+        # the module's attribute search)
+        params = self._parameters
+        weight = params.get("weight")
+        if (m > 0 and weight is not None and params.get("bias", self) is None and x.is_cuda
+                and DECODE_GEMM_ROWS > 0):
             n, k = self.out_features, self.in_features
             if x.dtype is torch.float32:
                 small = m * n * k <= SMALL_F32 and k <= 1024
             elif not self.half_on_lv_linear:
                 small = False
             elif m <= DECODE_GEMM_ROWS and ops.linear_supported(m, n, k, x.dtype):
-                return ops.linear(x, self.weight)
+                return ops.linear(x, weight)
             else:
                 small = m <= 2 * DECODE_GEMM_ROWS and n * k <= SMALL_LAYER
             if small:
-                y = ops.linear_if_plain(x, self.weight)
+                y = ops.linear_if_plain(x, weight)
                 if y is not None:
                     return y
         return super().forward(x)

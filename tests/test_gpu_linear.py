@@ -288,3 +288,21 @@ def test_layer_products_leave_graphs_and_slow_sizes_to_the_library():
                               (300, 512, 512, "silu_mul", False)):
         x, w = (torch.randn(r, k, device="cuda", dtype=torch.bfloat16) for r in (m, n))
         assert (ops.linear_if_plain(x, w, act) is not None) == own, (m, n, k, act)
+
+
+@torch.inference_mode()
+@pytest.mark.parametrize("dtype,m", [(torch.float32, 9), (torch.bfloat16, 9), (torch.bfloat16, 300)])
+def test_layer_with_a_bias_or_a_parametrized_weight(dtype, m):
+    from torch.nn.utils import parametrize
+    from litevllm.models.llama import Linear
+
+    class Half(torch.nn.Module):
+        def forward(self, w):
+            return w * 0.5
+    x = torch.randn(m, 512, device="cuda", dtype=dtype)
+    for bias in (False, True):
+        lin = Linear(512, 64, bias=bias).to(device="cuda", dtype=dtype)
+        want = torch.nn.functional.linear(x, lin.weight * 0.5, lin.bias)
+        parametrize.register_parametrization(lin, "weight", Half())
+        got = lin(x)
+        assert (got - want).float().norm() <= 2.0 ** -7 * want.float().norm()
