@@ -300,9 +300,9 @@ _retired: list[dict] = []     # graphs dropped while their thread was capturing
 def _graph_capture():
     """No DecodeGraphs is freed inside: garbage is collected first, the
     collector is off until the end, and drops on other threads wait."""
+    gc.collect()     # not under the lock: other objects' finalizers may wait for threads
     with _capture_lock:
         _retired.clear()
-        gc.collect()
         was_on = gc.isenabled()
         gc.disable()
         try:
