@@ -461,10 +461,13 @@ bool is_direct(const at::Tensor& t) {
   return (t.key_set().raw_repr() & ~plain) == 0 && !t._fw_grad(/*level=*/0).defined();
 }
 
+// This thread's layers leave their products to nn.Linear (library_products).
+thread_local bool products_by_library = false;
+
 // Nobody but the dispatcher's CUDA kernel would see a call made now: neither
 // autograd, autocast, a trace, a transform nor a Python mode.
 bool calls_are_direct() {
-  if (at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) ||
+  if (products_by_library || at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) ||
       at::impl::torch_function_mode_enabled() ||
       c10::impl::TorchDispatchModeTLS::any_modes_set())
     return false;
@@ -481,10 +484,13 @@ bool is_aligned_rows(const at::Tensor& t, int64_t width, at::ScalarType type) {
 
 // (x, weight, None or "silu_mul") -> out: nn.Linear's product for a layer that
 // falls back on nn.Linear itself, so everything the library's kernels ask for
-// or nn.Linear answers differently is not plain here.  Nor is a call under
-// graph capture: what these products save is host time, on the GPU the library
-// GEMM is often the faster (fp32, 16 rows of 1024x512: 7.2 us against 4.5;
-// 4096x1024 11.9 and 6.0).  bf16 / fp16, 257-512 rows, GPU time against the
+// or nn.Linear answers differently is not plain here.  What these products save
+// is host time; on the GPU the library GEMM is often the faster (fp32, 16 rows
+// of 1024x512: 7.2 us against 4.5; 4096x1024 11.9 and 6.0), so the decode graphs
+// switch them off (library_products).  That a stream is capturing does not: the
+// warm-up before a capture has to take the capture's route, or the library's
+// handle for the thread would be made inside it, which the runtime does not
+// survive.  bf16 / fp16, 257-512 rows, GPU time against the
 // library: 0.65-1.13 where the workgroups run at once and k is at least 512
 // (4096x1024 1.01-1.10, 1024x3072 0.83-0.91), 1.2-1.7 where they do not
 // (6144x1024 from 384 rows on, 2048x2048 up to 384, 384 rows of 1280x5120); with
@@ -507,8 +513,7 @@ FAST(layer_linear, 3) {
       !is_direct(*w) || w->size(1) != K || (silu && rows % 2) || !is_aligned_rows(*x, K, type) ||
       !is_aligned_rows(*w, K, type) ||
       (dt == LV_F32 ? silu || K % 4 != 0
-                    : (silu ? N < K : K < 512) || !api.linear_one_round(M, N, K, act)) ||
-      c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None)
+                    : (silu ? N < K : K < 512) || !api.linear_one_round(M, N, K, act)))
     NOT_PLAIN();
   const at::Tensor out = empty({M, N}, *x);
   void* st = stream_of(dev);
@@ -524,8 +529,18 @@ FAST(layer_linear, 3) {
   return done(rc, dt == LV_F32 ? "lv_linear_f32" : "lv_linear", &out);
 }
 
+// (on) -> whether it was: layer_linear answers None to this thread from here on.
+PyObject* library_products(PyObject*, PyObject* on) {
+  const int v = PyObject_IsTrue(on);
+  if (v < 0) return nullptr;
+  const bool was = products_by_library;
+  products_by_library = v != 0;
+  return PyBool_FromLong(was);
+}
+
 #define METHOD(NAME) {#NAME, (PyCFunction)(void (*)(void))NAME, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {{"bind", bind, METH_VARARGS, nullptr},
+                         {"library_products", library_products, METH_O, nullptr},
                          METHOD(kv_scatter),
                          METHOD(paged_attention),
                          METHOD(sample),

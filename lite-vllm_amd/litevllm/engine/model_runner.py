@@ -400,10 +400,11 @@ class DecodeGraphs:
             meta.prefix = ops.PrefixPlan(p.blocks[:b], p.items, p.members)
             meta.prefix_workspace = self.pfx_workspace
         kv = [self.kv_cache.get_kv(i) for i in range(self.kv_cache.num_layers)]
-        return self.model(input_ids=v["input_ids"], positions=v["positions"], kv_caches=kv,
-                          slot_mapping=v["slot_mapping"], block_tables=v["block_tables"],
-                          context_lens=v["context_lens"], is_prefill=False, attn_metadata=meta,
-                          logits_indices=None)
+        with ops.library_products():    # (in the warm-up before the capture too)
+            return self.model(input_ids=v["input_ids"], positions=v["positions"], kv_caches=kv,
+                              slot_mapping=v["slot_mapping"], block_tables=v["block_tables"],
+                              context_lens=v["context_lens"], is_prefill=False,
+                              attn_metadata=meta, logits_indices=None)
 
     def _pack(self, b: int, num_block_ids: int,
               device_tokens: Optional[torch.Tensor] = None) -> None:

@@ -32,9 +32,10 @@ DECODE_GEMM_ROWS = int(os.environ.get("LV_DECODE_GEMM_ROWS", "256"))
 # 6144x1024 15.7 (12.5).
 SMALL_LAYER = 1 << 23
 # fp32 products of up to SMALL_F32 multiply-adds (k up to 1024) run on
-# lv_linear_f32, under the same condition and outside graph capture: 4 us of
-# host time, and 4-13 us on the GPU where the library takes 4-8 us on its good
-# shapes and up to 133 on others (200 rows of 256x688).
+# lv_linear_f32, under the same condition: 4 us of host time, and 4-13 us on the
+# GPU where the library takes 4-8 us on its good shapes and up to 133 on others
+# (200 rows of 256x688).  The decode graphs, whose host time does not count,
+# take neither route.
 SMALL_F32 = 1 << 27
 
 

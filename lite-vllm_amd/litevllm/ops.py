@@ -14,6 +14,7 @@ makes the buffer.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 from typing import NamedTuple, Optional
@@ -790,14 +791,26 @@ def linear_f32(x: torch.Tensor, weight: torch.Tensor,
     return out
 
 
+@contextlib.contextmanager
+def library_products():
+    """Inside, this thread's linear_if_plain answers None: for work whose host
+    time does not count (a graph's forward, its warm-up included)."""
+    native = _native_module or _native()
+    was = native.library_products(True)
+    try:
+        yield
+    finally:
+        native.library_products(was)
+
+
 def linear_if_plain(x: torch.Tensor, weight: torch.Tensor,
                     activation: Optional[str] = None) -> Optional[torch.Tensor]:
     """linear (bf16 / fp16) or linear_f32 (fp32, no activation), or None,
     having done nothing, where nn.Linear has to make the product: operands the
     kernels do not take (rows that overlap or lie off 16-byte boundaries, other
     sizes), bf16 / fp16 sizes at which the library GEMM is clearly faster on the
-    GPU (lv_linear_one_round), graph capture, grad mode, autocast, forward-mode
-    tangents, traces, transforms and Python modes."""
+    GPU (lv_linear_one_round), library_products, grad mode, autocast,
+    forward-mode tangents, traces, transforms and Python modes."""
     if torch.compiler.is_dynamo_compiling():
         return None
     return (_native_module or _native()).layer_linear(x, weight, activation)

@@ -267,16 +267,25 @@ def test_gated_mlp_runs_the_hooks_of_its_projection():
 
 @torch.inference_mode()
 def test_layer_products_leave_graphs_and_slow_sizes_to_the_library():
-    """Under capture the library's product is recorded (host time, all the own
-    kernels save there, is not spent on replays), equal on every replay to the
-    library's eager one; so are sizes whose workgroups do not run at once."""
+    """Inside library_products nn.Linear makes the layer's product, in the
+    warm-up and in the capture, equal on every replay to its eager one; a
+    program's own capture takes the route of its own warm-up; sizes whose
+    workgroups do not run at once are the library's."""
     lin, ref = _layer_and_reference(torch.float32)
     x = torch.randn(9, 512, device="cuda")
-    assert ops.linear_if_plain(x, lin.weight) is not None
-    ref(x)
+    own = ops.linear_if_plain(x, lin.weight)
+    with ops.library_products():
+        assert ops.linear_if_plain(x, lin.weight) is None
+        assert torch.equal(lin(x), ref(x))
+    assert torch.equal(lin(x), own)
     graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
     with torch.cuda.graph(graph, stream=stream):
-        assert ops.linear_if_plain(x, lin.weight) is None
+        y = lin(x)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(y, own)
+    graph = torch.cuda.CUDAGraph()
+    with ops.library_products(), torch.cuda.graph(graph, stream=stream):
         y = lin(x)
     for _ in range(3):
         x.normal_()

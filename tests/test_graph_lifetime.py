@@ -189,3 +189,32 @@ def test_a_capture_that_fails_leaves_the_collector_on(monkeypatch, plain_gc):
     with pytest.raises(ZeroDivisionError):
         gpu.runner().capture_decode_graphs()
     assert gc.isenabled()
+
+
+def test_warm_up_and_capture_take_one_route(monkeypatch, plain_gc):
+    """A library first used by a thread inside a capture makes its handle
+    there, which the runtime does not survive: the forward that is captured and
+    the one that warms up for it leave the same products to the library, on the
+    capturing thread only."""
+    native, seen = mr.ops._native(), []
+
+    def state():
+        was = native.library_products(True)
+        native.library_products(was)
+        return was
+
+    def forward():
+        other = []
+        t = threading.Thread(target=lambda: other.append(state()))
+        t.start()
+        t.join(10)
+        seen.append((bool(gpu.capturing), state(), other[0]))
+        return torch.zeros(1)
+    gpu = Gpu(monkeypatch, forward)
+    gpu.runner().capture_decode_graphs()
+    assert {c for c, _, _ in seen} == {False, True}
+    assert all(on and not elsewhere for _, on, elsewhere in seen) and not state()
+    gpu.forward = lambda: 1 // 0
+    with pytest.raises(ZeroDivisionError):
+        gpu.runner().capture_decode_graphs()
+    assert not state()
