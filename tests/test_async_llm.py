@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import asyncio
 import threading
+import time
 
 import pytest
 
@@ -56,6 +57,7 @@ class FakeEngine:
 
     def step(self):
         self.check_thread()
+        time.sleep(1e-4)      # as a real step, off the interpreter: the reader gets its turn
         self.steps += 1
         if self.fail_at is not None and self.steps == self.fail_at:
             raise RuntimeError("device lost")
